@@ -346,9 +346,8 @@ def plan_blocks_arrays(n, op_nq, op_qubits, op_mats, k=5, effort=1):
     return refs, bqs[:nb], bm[:nb]
 
 
-def _plan_segment(ops, n, k, effort=1):
-    if not ops:
-        return []
+def _op_arrays(ops):
+    """The planners' flat arrays of an op list: (op_nq, op_qubits, op_mats)."""
     m = len(ops)
     nq = np.zeros(m, dtype=np.int32)
     qb = np.full((m, 8), -1, dtype=np.int32)
@@ -358,7 +357,13 @@ def _plan_segment(ops, n, k, effort=1):
         nq[i] = len(qs)
         qb[i, :len(qs)] = qs
         mats.append(np.asarray(op.full_matrix(), dtype=np.complex128).reshape(-1))
-    refs, bqs, bm = plan_blocks_arrays(n, nq, qb, np.concatenate(mats), k, effort)
+    return nq, qb, np.concatenate(mats)
+
+
+def _plan_segment(ops, n, k, effort=1):
+    if not ops:
+        return []
+    refs, bqs, bm = plan_blocks_arrays(n, *_op_arrays(ops), k, effort)
     res = []
     for e in refs:
         if e >= 0:
@@ -367,6 +372,79 @@ def _plan_segment(ops, n, k, effort=1):
         else:
             res.append(ops[-1 - int(e)])
     return res
+
+
+PASS_MIN_QUBITS = 10     # smallest state (and tile) of the block passes
+
+
+class PassRun:
+    """Consecutive block passes: PASS_DTYPE passes, PASS_BLOCK_DTYPE records
+    and float32 [blocks, 1024] matrix fragments, as the library takes them."""
+    __slots__ = ("passes", "blocks", "mats")
+
+    def __init__(self, passes, blocks, mats):
+        self.passes = passes
+        self.blocks = blocks
+        self.mats = mats
+
+
+def plan_passes_arrays(n, op_nq, op_qubits, op_mats, tile_bits, low_bits):
+    """The native pass planner (qsim_plan_passes) on flat arrays: (refs,
+    passes, blocks, mats); refs[e] >= 0 is pass refs[e], refs[e] < 0 is op
+    -1 - refs[e] passed through (more than 4 qubits).  Host code that
+    releases the GIL, as plan_blocks_arrays."""
+    import ctypes
+    from blackwell_kernels import _lib
+    m = len(op_nq)
+    nq = np.ascontiguousarray(op_nq, dtype=np.int32)
+    qb = np.ascontiguousarray(op_qubits, dtype=np.int32).reshape(m, 8)
+    mv = np.ascontiguousarray(op_mats, dtype=np.complex128).reshape(-1)
+    refs = np.zeros(m, dtype=np.int32)
+    passes = np.zeros(m, dtype=_lib.PASS_DTYPE)
+    blocks = np.zeros(m, dtype=_lib.PASS_BLOCK_DTYPE)
+    mats = np.empty((m, _lib.PASS_BLOCK_FLOATS), dtype=np.float32)
+    n_out, n_blk = ctypes.c_int(0), ctypes.c_int(0)
+    vp = lambda a: ctypes.c_void_p(a.ctypes.data)
+    _lib.call("qsim_plan_passes", n, tile_bits, low_bits, m, vp(nq), vp(qb), vp(mv.view(np.float64)),
+              vp(refs), vp(passes), vp(blocks), vp(mats), ctypes.byref(n_out), ctypes.byref(n_blk))
+    refs = refs[:n_out.value]
+    return refs, passes[:int((refs >= 0).sum())], blocks[:n_blk.value], mats[:n_blk.value]
+
+
+def plan_passes(ops, n, tile_bits, low_bits):
+    """Pack unitary ops into block passes (n >= PASS_MIN_QUBITS).  Returns a
+    list of PassRun | Op (measure/reset, and ops of more than 4 qubits)."""
+    out, seg = [], []
+
+    def flush():
+        if not seg:
+            return
+        refs, passes, blocks, mats = plan_passes_arrays(n, *_op_arrays(seg), tile_bits, low_bits)
+        e = 0
+        while e < len(refs):
+            if refs[e] < 0:
+                out.append(seg[-1 - int(refs[e])])
+                e += 1
+                continue
+            a = int(refs[e])                     # passes are numbered in execution order
+            while e < len(refs) and refs[e] >= 0:
+                e += 1
+            b = int(refs[e - 1]) + 1
+            p = passes[a:b].copy()
+            first = int(p["first_block"][0])
+            last = int(p["first_block"][-1] + p["n_blocks"][-1])
+            p["first_block"] -= first
+            out.append(PassRun(p, blocks[first:last], mats[first:last]))
+        seg.clear()
+
+    for op in ops:
+        if op.kind in ("measure", "reset"):
+            flush()
+            out.append(op)
+        else:
+            seg.append(op)
+    flush()
+    return out
 
 
 def apply_to_block(mat, u, qubits, block_qubits):

@@ -12,8 +12,12 @@ Modes:
   blocks - 5-qubit dense blocks on FP32 MFMA (n >= 10), other entries plain;
   blocks/<k> - the same with k-qubit blocks, k = 4, 5, 6 (k = 4 needs
            n >= 11 and k = 6 n >= 13 for their MFMA kernels);
+  passes - 4-qubit dense blocks on FP32 MFMA, many per trip through HBM
+           (n >= 10): tiles of 10..13 qubits stay in LDS for all the blocks
+           of a pass;
   tiles  - LDS tile programs, many ops per HBM pass;
-  auto   - tiles with the whole state in one tile when n <= 13, else blocks;
+  auto   - tiles (the whole state in one tile when n <= 13) for circuits with
+           few ops per qubit on at most 20 qubits, else passes;
   tune   - every applicable mode timed once on the device, fastest kept
            (the fusion width is one of the choices).
 """
@@ -36,7 +40,7 @@ WHOLE_OP_US_12Q = 2.0
 BLOCK_US = 5.0
 # plan steps a HIP graph can hold: library launches on the current stream with
 # device-resident arguments only (no host uploads, no host-side decisions)
-GRAPH_SAFE_STEPS = ("blocks", "mfma", "tile", "mcgate")
+GRAPH_SAFE_STEPS = ("passes", "blocks", "mfma", "tile", "mcgate")
 # fusion widths of the MFMA block kernels and the smallest state each runs on
 BLOCK_WIDTHS = {4: 11, 5: BLOCK_MIN_QUBITS, 6: 13}
 TUNE_REPS = 3
@@ -72,6 +76,18 @@ def default_tile_shape(n):
         return n, min(4, n)
     m = 10 if n <= 20 else (11 if n <= 22 else (12 if n <= 24 else 13))
     return m, 4
+
+
+def pass_shape(n):
+    """(tile qubits, always-included low qubits) of the block passes.  Small
+    tiles spread a small state over more CUs, large ones take fewer passes;
+    times in us on MI355X for tiles of 10 / 11 / 12 / 13 qubits: 12-qubit
+    ladder 44 / 45 / 55, 16-qubit QFT 58 / 60 / 70 / 123, 20-qubit volume 256 /
+    235 / 226 / 283, 24-qubit 3213 / 2572 / 2544 / 2441, 28-qubit 73.3 / 58.0 /
+    54.9 / 52.0 ms.  Four low qubits make 128 B runs, whole cache lines; five
+    or six take more passes (28 qubits: 52.5 and 56.3 ms)."""
+    m = 10 if n <= 15 else (11 if n <= 18 else (12 if n <= 21 else 13))
+    return (n if n <= 11 else m), 4
 
 
 def tune_tile_shapes(n):
@@ -145,10 +161,11 @@ def tile_ops(ops, mask):
 class _Dev:
     """Device copies of a plan's matrices/op tables (one upload per plan)."""
 
-    def __init__(self, device, mats=None, ops=None, coefs=None):
+    def __init__(self, device, mats=None, ops=None, coefs=None, blob=None):
         self.mats = None if mats is None else torch.from_numpy(mats).to(device)
         self.ops = None if ops is None else torch.from_numpy(ops.view(np.uint8).copy()).to(device)
         self.coefs = None if coefs is None else torch.from_numpy(coefs).to(device)
+        self.blob = None if blob is None else torch.from_numpy(blob).to(device)
 
 
 class CompiledCircuit:
@@ -279,10 +296,13 @@ class CompiledCircuit:
 
     def resolve_mode(self, mode, device=None):
         """auto: the whole state as one LDS program below 10 qubits; between
-        10 and 13 qubits that or MFMA blocks, and between 14 and 20 qubits
-        tile programs or MFMA blocks, whichever the cost model says is cheaper
-        (deep circuits favour blocks: one block absorbs many ops); MFMA blocks
-        above.  tune: the mode tuned_mode measured fastest on `device`."""
+        10 and 13 qubits that or MFMA block passes, and between 14 and 20
+        qubits tile programs or block passes, where the cost model prices the
+        MFMA side as one launch per 5-qubit block (deep circuits favour it:
+        one block absorbs many ops); block passes above.  The tile programs'
+        compensated arithmetic is the more exact, so the line between the two
+        stays where one launch per block puts it although a pass is cheaper.
+        tune: the mode tuned_mode measured fastest on `device`."""
         if mode == "tune":
             if device is None:
                 raise ValueError("mode 'tune' needs the device to measure on")
@@ -298,7 +318,7 @@ class CompiledCircuit:
         if n < BLOCK_MIN_QUBITS:
             return "whole"
         if n > AUTO_TILES_MAX_QUBITS:
-            return "blocks"
+            return "passes"
         if n > WHOLE_TILE_MAX:
             passes = sum(1 for e in self.tile_entries() if isinstance(e, C.TilePass))
             others = len(self.tile_entries()) - passes
@@ -306,10 +326,10 @@ class CompiledCircuit:
             t_tiles = (passes * TILE_PASS_US + w_ops * TILE_OP_US_16Q * 1.13 ** (n - 16)
                        + others * BLOCK_US_16Q)
             t_blocks = len(self.block_entries()) * BLOCK_US_16Q * 1.07 ** (n - 16)
-            return "tiles" if t_tiles < t_blocks else "blocks"
+            return "tiles" if t_tiles < t_blocks else "passes"
         t_whole = len(self.ops) * WHOLE_OP_US_12Q * 2.0 ** (n - 12)
         t_blocks = len(self.block_entries()) * BLOCK_US
-        return "blocks" if t_blocks < t_whole else "whole"
+        return "passes" if t_blocks < t_whole else "whole"
 
     def _build(self, mode, device):
         n = self.n_qubits
@@ -331,6 +351,10 @@ class CompiledCircuit:
             if not (1 <= low <= m <= WHOLE_TILE_MAX):
                 raise ValueError(f"tile shape needs 1 <= low <= m <= {WHOLE_TILE_MAX} (got {mode!r})")
             return self._build_tiles(C.plan_tiles(self.ops, n, m=min(m, n), low=low), device)
+        if mode == "passes":
+            if n < C.PASS_MIN_QUBITS:
+                raise ValueError(f"block passes need n >= {C.PASS_MIN_QUBITS} (n = {n})")
+            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n)), device)
         if mode == "blocks":
             if n < 10:
                 return self._build_tiles(C.plan_tiles(self.ops, n, m=n), device)
@@ -417,6 +441,20 @@ class CompiledCircuit:
         flush()
         return _Plan(self, steps, mats, None, None, device)
 
+    def _build_passes(self, entries, device):
+        steps, parts, off = [], [], 0
+        for e in entries:
+            if isinstance(e, C.PassRun):
+                # one device blob per plan: records then fragments of each run
+                steps.append(("passes", (e.passes, e.blocks, off, off + e.blocks.nbytes)))
+                parts += [e.blocks.view(np.uint8).reshape(-1), e.mats.view(np.uint8).reshape(-1)]
+                off += e.blocks.nbytes + e.mats.nbytes
+            elif e.kind not in ("measure", "reset") and len(e.all_qubits) == 5:
+                steps.append(("sub", self._build_blocks(C.plan_blocks([e], self.n_qubits), device)))
+            else:
+                steps.append(("sub", self._build_plain([e], device)))
+        return _Plan(self, steps, [], None, None, device, np.concatenate(parts) if parts else None)
+
     def _build_tiles(self, entries, device):
         all_ops, all_cf, steps = [], [], []
         op_off, cf_off = 0, 0
@@ -439,7 +477,7 @@ class CompiledCircuit:
 
 
 class _Plan:
-    def __init__(self, cc, steps, mats, ops, coefs, device):
+    def __init__(self, cc, steps, mats, ops, coefs, device, blob=None):
         self.cc = cc
         self.steps = steps
         self.n_launches = 0
@@ -451,12 +489,14 @@ class _Plan:
                 self.mat_offsets.append(off)
                 off += m.size
             mats_arr = np.concatenate(mats).astype(np.complex64)
-        self.dev = _Dev(device, mats_arr, ops, coefs)
+        self.dev = _Dev(device, mats_arr, ops, coefs, blob)
         for kind, p in steps:
             if kind == "sub":
                 self.n_launches += p.n_launches
             elif kind == "blocks":
                 self.n_launches += p[1]
+            elif kind == "passes":
+                self.n_launches += len(p[0])
             else:
                 self.n_launches += 1
 
@@ -501,6 +541,12 @@ class _Plan:
             first, count, qs = a
             call("qsim_apply_blocks", s, sp, n, self._mat_ptr(first),
                  ctypes.c_void_p(qs.ctypes.data), count)
+        elif kind == "passes":
+            passes, blocks, boff, moff = a
+            base = self.dev.blob.data_ptr()
+            call("qsim_apply_passes", s, sp, n, ctypes.c_void_p(passes.ctypes.data), len(passes),
+                 ctypes.c_void_p(blocks.ctypes.data), ctypes.c_void_p(base + boff),
+                 ctypes.c_void_p(base + moff), len(blocks))
         elif kind == "tile":
             mask, off, cnt = a
             call("qsim_tile_program", s, sp, n, mask,

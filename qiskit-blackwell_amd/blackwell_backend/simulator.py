@@ -9,8 +9,9 @@ before execution (simulator.py:555-604), the complex64 statevector
 Differences by design:
   * circuits are compiled by blackwell_backend.compiler (FP64 host fusion)
     into plans of prepared launches (blackwell_backend.executor);
-  * the default execution mode is "auto": the whole circuit in one LDS tile
-    program when the state fits (n <= 13), 5-qubit FP32-MFMA blocks above;
+  * the default execution mode is "auto": LDS tile programs for small or
+    shallow circuits, passes of 4-qubit FP32-MFMA blocks for the others;
+    mode="blocks" runs one launch per 5-qubit block,
     mode="plain" runs one kernel per gate, mode="blocks/<k>" fuses into
     k-qubit MFMA blocks (k = 4, 5, 6) and mode="tune" times the modes and
     fusion widths once per circuit and keeps the fastest;
@@ -99,7 +100,7 @@ class BlackwellSimulator:
         result = sim.run(circuit, shots=1024)
     """
 
-    MODES = ("auto", "plain", "blocks", "tiles", "whole", "tune")
+    MODES = ("auto", "plain", "blocks", "passes", "tiles", "whole", "tune")
     # largest circuit run() replays as a HIP graph (the graph owns a state
     # buffer of 8 * 2^n bytes per cached circuit)
     GRAPH_MAX_QUBITS = 20

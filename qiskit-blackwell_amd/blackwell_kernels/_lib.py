@@ -53,6 +53,8 @@ PROTOTYPES = {
     "qsim_plan_blocks": (_i, [_i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _pint]),
     "qsim_plan_blocks_search": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _pint]),
     "qsim_apply_blocks": (_i, [_vp, _vp, _i, _vp, _vp, _i]),
+    "qsim_plan_passes": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _pint, _pint]),
+    "qsim_apply_passes": (_i, [_vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _i]),
     "qsim_apply_block_batch": (_i, [_vp, _vp, _vp, _i64]),
     "qsim_reduce_workspace_bytes": (_i64, [_i]),
     "qsim_norm2": (_i, [_vp, _vp, _i, _vp, _vp]),
@@ -106,6 +108,11 @@ BLOCK_REC_DTYPE = np.dtype([("state", "<u8"), ("mat", "<u8"), ("set_begin", "<u8
                             ("n_qubits", "<i4"), ("q", "i1", (5,)), ("pad", "i1", (7,))])
 SAMPLE_REC_DTYPE = np.dtype([("state", "<u8"), ("out", "<u8"), ("seed", "<u8"), ("leaf_off", "<u8"),
                              ("shot_off", "<u8"), ("n_qubits", "<i4"), ("shots", "<u4")])
+# qsim_pass, qsim_pass_block and the floats of a block's matrix fragments
+PASS_DTYPE = np.dtype([("tile_mask", "<u8"), ("first_block", "<i4"), ("n_blocks", "<i4")])
+PASS_BLOCK_DTYPE = np.dtype([("bit", "<u2", (16,))])
+PASS_BLOCK_FLOATS = 1024
+assert PASS_DTYPE.itemsize == 16 and PASS_BLOCK_DTYPE.itemsize == 32
 assert SAMPLE_REC_DTYPE.itemsize == 48
 assert OP_DTYPE.itemsize == 16 and INSTANCE_DTYPE.itemsize == 40 and BLOCK_REC_DTYPE.itemsize == 40
 

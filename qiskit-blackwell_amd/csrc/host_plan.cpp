@@ -30,6 +30,7 @@
 #include <stdint.h>
 #include <algorithm>
 #include <string.h>
+#include <new>
 #include <vector>
 
 namespace qsim {
@@ -170,6 +171,108 @@ static void apply_rows(double* re, double* im, int D, const double* u, const int
       }
     }
   }
+}
+
+// ------------------------------------------------------------------ passes
+// Pass planner.  A pass is a tile (a set T of at most tile_bits qubits that
+// holds the low_bits lowest ones) and the ops it absorbs, by the rule of
+// absorb_set.  From each start (the low qubits alone, and with the qubits of
+// each op that no earlier remaining op touches) T grows by the op on its
+// frontier that adds the most absorbed ops per added qubit; the T that
+// absorbs the most ops is kept and filled up with the lowest unused qubits.
+// Ops wider than a block are never absorbed.
+constexpr int kPassK = 4;             // qubits per block
+constexpr int kPassD = 1 << kPassK;
+
+struct PassPlan {
+  int n, m;
+  uint64_t low;
+  std::vector<uint64_t> mask;       // per op; wide ops carry kWide as well
+  std::vector<int> rem;
+};
+constexpr uint64_t kWide = 1ull << 63;   // in no tile, so the op is never absorbed
+
+static uint64_t grow_tile(const PassPlan& p, uint64_t S, int* absorbed) {
+  const uint64_t all = (1ull << p.n) - 1;
+  int base = absorb_set(p.rem, p.mask, S, nullptr);
+  while (__builtin_popcountll(S) < p.m) {
+    uint64_t blocked = 0, best = 0;
+    int best_gain = -1, best_add = 1;
+    for (int i : p.rem) {
+      const uint64_t mk = p.mask[i];
+      if ((mk & blocked) == 0 && (mk & ~S) == 0) continue;      // absorbed already
+      if ((mk & blocked) == 0 && !(mk & kWide)) {
+        const uint64_t un = S | mk;
+        const int add = __builtin_popcountll(mk & ~S);
+        if (__builtin_popcountll(un) <= p.m) {
+          const int gain = absorb_set(p.rem, p.mask, un, nullptr) - base;
+          if (best_gain < 0 || (long long)gain * best_add > (long long)best_gain * add) {
+            best_gain = gain;
+            best_add = add;
+            best = un;
+          }
+        }
+      }
+      blocked |= mk;
+      if ((blocked & all) == all) break;
+    }
+    if (best_gain < 0) break;
+    S = best;
+    base += best_gain;
+  }
+  *absorbed = base;
+  return S;
+}
+
+// Swizzled LDS index of tile bit p: bits 5..9 and 10..13 fold onto bits 0..4.
+static uint16_t pass_index(int p) {
+  const uint32_t j = 1u << p;
+  return (uint16_t)(j ^ ((j >> 5) & 31u) ^ ((j >> 10) & 31u));
+}
+
+// Record of a block on tile bits row[0..4): the lane bits take one bit of each
+// residue mod 5 (the LDS bank bits they fold onto) where one is free, then the
+// rest in ascending order.
+static void pass_record(qsim_pass_block* rec, int m, const int* row) {
+  memset(rec, 0, sizeof *rec);
+  uint32_t used = 0;
+  int at = 0;
+  for (int j = 0; j < kPassK; ++j) {
+    used |= 1u << row[j];
+    rec->bit[at++] = pass_index(row[j]);
+  }
+  int lane[5];
+  for (int j = 0; j < 5; ++j) {
+    lane[j] = -1;
+    for (int p = j; p < m && lane[j] < 0; p += 5)
+      if (!(used >> p & 1)) {
+        lane[j] = p;
+        used |= 1u << p;
+      }
+  }
+  for (int j = 0; j < 5; ++j) {
+    for (int p = 0; p < m && lane[j] < 0; ++p)
+      if (!(used >> p & 1)) {
+        lane[j] = p;
+        used |= 1u << p;
+      }
+    rec->bit[at++] = pass_index(lane[j]);
+  }
+  for (int p = 0; p < m; ++p)
+    if (!(used >> p & 1)) rec->bit[at++] = pass_index(p);
+}
+
+// MFMA A fragments of the 16 x 16 complex matrix u: row i = 2 r + part of the
+// real 32 x 32 form, slice s, half h -> out[s / 4][lane = 32 h + i][s % 4].
+static void pass_fragments(float* out, const double* u) {
+  for (int s = 0; s < kPassD; ++s)
+    for (int h = 0; h < 2; ++h)
+      for (int i = 0; i < 2 * kPassD; ++i) {
+        const double* e = u + 2 * ((i >> 1) * kPassD + s);
+        const int part = i & 1;
+        const double v = part == h ? e[0] : (part ? e[1] : -e[1]);
+        out[((s >> 2) * 64 + 32 * h + i) * 4 + (s & 3)] = (float)v;
+      }
 }
 
 }  // namespace qsim
@@ -348,6 +451,129 @@ int qsim_plan_blocks(int n_qubits, int k, int n_ops, const int32_t* op_nq, const
                      double* block_mats, int* n_out) {
   return qsim_plan_blocks_search(n_qubits, k, 0, n_ops, op_nq, op_qubits, op_mats, out_ref,
                                  block_qubits, block_mats, n_out);
+}
+
+int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const int32_t* op_nq,
+                     const int32_t* op_qubits, const double* op_mats, int32_t* out_ref,
+                     qsim_pass* passes, qsim_pass_block* blocks, float* mats, int* n_out,
+                     int* n_blocks) {
+  if (n_qubits < QSIM_PASS_MIN_TILE || n_qubits > QSIM_MAX_QUBITS)
+    return fail(QSIM_ERANGE, "n_qubits=%d outside %d..%d", n_qubits, QSIM_PASS_MIN_TILE, QSIM_MAX_QUBITS);
+  if (tile_bits < QSIM_PASS_MIN_TILE || tile_bits > QSIM_PASS_MAX_TILE)
+    return fail(QSIM_ERANGE, "tile of %d qubits outside %d..%d", tile_bits, QSIM_PASS_MIN_TILE, QSIM_PASS_MAX_TILE);
+  const int m = std::min(tile_bits, n_qubits);
+  if (low_bits < 1 || low_bits > m - kPassK)
+    return fail(QSIM_EINVAL, "low_bits %d outside 1..%d", low_bits, m - kPassK);
+  if (n_ops < 0) return fail(QSIM_EINVAL, "n_ops < 0");
+  if (!n_out || !n_blocks || (n_ops > 0 && (!op_nq || !op_qubits || !op_mats || !out_ref || !passes || !blocks ||
+                                            !mats)))
+    return fail(QSIM_EINVAL, "NULL pointer argument");
+  try {
+    PassPlan p;
+    p.n = n_qubits;
+    p.m = m;
+    p.low = (1ull << low_bits) - 1;
+    p.mask.resize(n_ops);
+    std::vector<size_t> moff(n_ops);
+    size_t off = 0;
+    for (int i = 0; i < n_ops; ++i) {
+      const int nq = op_nq[i];
+      if (nq < 1 || nq > 8) return fail(QSIM_EINVAL, "op %d has %d qubits (1..8)", i, nq);
+      uint64_t mk = 0;
+      for (int j = 0; j < nq; ++j) {
+        const int q = op_qubits[i * 8 + j];
+        if (q < 0 || q >= n_qubits) return fail(QSIM_EINVAL, "op %d: qubit %d out of range", i, q);
+        if (mk >> q & 1) return fail(QSIM_EINVAL, "op %d: repeated qubit %d", i, q);
+        mk |= 1ull << q;
+      }
+      p.mask[i] = mk | (nq > kPassK ? kWide : 0);
+      moff[i] = off;
+      off += (size_t)1 << (2 * nq);
+    }
+    p.rem.resize(n_ops);
+    for (int i = 0; i < n_ops; ++i) p.rem[i] = i;
+    const uint64_t all = (1ull << n_qubits) - 1;
+    std::vector<int> chosen, keep, sub_nq, sub_q, ref, bq;
+    std::vector<double> sub_m, bm;
+    std::vector<uint64_t> starts;
+    int np = 0, nb = 0, ne = 0;
+    while (!p.rem.empty()) {
+      // candidate tiles
+      uint64_t best_S = 0;
+      int best_cnt = 0;
+      starts.assign(1, p.low);
+      uint64_t blocked = 0;
+      for (int i : p.rem) {
+        const uint64_t mk = p.mask[i];
+        if (!(mk & blocked) && !(mk & kWide)) {
+          const uint64_t un = p.low | mk;
+          if (std::find(starts.begin(), starts.end(), un) == starts.end()) starts.push_back(un);
+        }
+        blocked |= mk;
+        if ((blocked & all) == all) break;
+      }
+      for (uint64_t s0 : starts) {
+        int cnt = 0;
+        const uint64_t S = m == n_qubits ? all : grow_tile(p, s0, &cnt);
+        if (m == n_qubits) cnt = absorb_set(p.rem, p.mask, S, nullptr);
+        if (cnt > best_cnt) {
+          best_cnt = cnt;
+          best_S = S;
+        }
+        if (m == n_qubits) break;
+      }
+      if (best_cnt == 0) {               // the first op is wider than a block
+        out_ref[ne++] = -1 - p.rem[0];
+        p.rem.erase(p.rem.begin());
+        continue;
+      }
+      for (int q = 0; q < n_qubits && __builtin_popcountll(best_S) < m; ++q) best_S |= 1ull << q;
+      chosen.clear();
+      absorb_set(p.rem, p.mask, best_S, &chosen);
+      keep.clear();
+      {
+        size_t c = 0;
+        for (int i : p.rem) {
+          if (c < chosen.size() && chosen[c] == i) ++c;
+          else keep.push_back(i);
+        }
+      }
+      p.rem.swap(keep);
+      // the pass's ops on tile-local qubits, packed into blocks
+      const int ns = (int)chosen.size();
+      sub_nq.resize(ns);
+      sub_q.assign((size_t)ns * 8, -1);
+      sub_m.clear();
+      for (int c = 0; c < ns; ++c) {
+        const int i = chosen[c], nq = op_nq[i];
+        sub_nq[c] = nq;
+        for (int j = 0; j < nq; ++j)
+          sub_q[c * 8 + j] = __builtin_popcountll(best_S & ((1ull << op_qubits[i * 8 + j]) - 1));
+        const double* u = op_mats + 2 * moff[i];
+        sub_m.insert(sub_m.end(), u, u + ((size_t)2 << (2 * nq)));
+      }
+      ref.resize(ns);
+      bq.resize((size_t)ns * 8);
+      bm.resize((size_t)ns * kPassD * kPassD * 2);
+      int n_ent = 0;
+      if (int rc = qsim_plan_blocks_search(m, kPassK, 1, ns, sub_nq.data(), sub_q.data(), sub_m.data(), ref.data(),
+                                           bq.data(), bm.data(), &n_ent))
+        return rc;
+      passes[np].tile_mask = best_S;
+      passes[np].first_block = nb;
+      passes[np].n_blocks = n_ent;        // every entry is a block: no op here is wider than one
+      for (int b = 0; b < n_ent; ++b, ++nb) {
+        pass_record(blocks + nb, m, &bq[(size_t)b * 8]);
+        pass_fragments(mats + (size_t)nb * QSIM_PASS_BLOCK_FLOATS, &bm[(size_t)b * kPassD * kPassD * 2]);
+      }
+      out_ref[ne++] = np++;
+    }
+    *n_out = ne;
+    *n_blocks = nb;
+    return QSIM_OK;
+  } catch (const std::bad_alloc&) {
+    return fail(QSIM_ENOMEM, "pass planner: out of host memory");
+  }
 }
 
 }  // extern "C"
