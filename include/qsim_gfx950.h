@@ -202,11 +202,12 @@ int qsim_apply_blocks(void* stream, void* state, int n_qubits, const void* block
  * tile qubits, 10..13 of them, qubit 0 among them).  A block record holds
  * the LDS index of each single tile bit (pass order: 4 row bits, 5 lane
  * bits, then the rest; index j sits at j with bits 5..9 and 10..12 XORed onto
- * bits 0..4), and QSIM_PASS_BLOCK_FLOATS floats hold its matrix in MFMA
- * fragment order.  qsim_plan_passes writes all three.                     */
+ * bits 0..4), and QSIM_PASS_BLOCK_BF16 bf16 values hold its matrix, each
+ * coefficient as the sum of three bf16 parts, in MFMA fragment order.
+ * qsim_plan_passes writes all three.                                      */
 #define QSIM_PASS_MIN_TILE 10
 #define QSIM_PASS_MAX_TILE 13
-#define QSIM_PASS_BLOCK_FLOATS 1024
+#define QSIM_PASS_BLOCK_BF16 3072
 typedef struct qsim_pass {
   uint64_t tile_mask;
   int32_t  first_block;
@@ -220,19 +221,19 @@ typedef struct qsim_pass_block {
  * qubits that hold qubits 0..low_bits-1, and each pass's ops into 4-qubit
  * blocks (qsim_plan_blocks_search, effort 1, on the tile).  Outputs, in
  * execution order, *n_out entries out_ref[e]: p >= 0 names passes[p], and
- * -1-i passes op i through (more than 4 qubits).  blocks and mats
- * (QSIM_PASS_BLOCK_FLOATS floats each) hold *n_blocks blocks in pass order.
+ * -1-i passes op i through (more than 4 qubits).  blocks and frags
+ * (QSIM_PASS_BLOCK_BF16 bf16 bit patterns each) hold *n_blocks blocks in pass order.
  * Capacity: n_ops entries, passes and blocks.                             */
 int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const int32_t* op_nq,
                      const int32_t* op_qubits, const double* op_mats, int32_t* out_ref,
-                     qsim_pass* passes, qsim_pass_block* blocks, float* mats, int* n_out,
+                     qsim_pass* passes, qsim_pass_block* blocks, uint16_t* frags, int* n_out,
                      int* n_blocks);
 /* Applies passes[0..n_passes) in order, one launch each.  blocks_host is
- * validated and must hold the bytes of the device copy blocks_dev; mats_dev
- * is the device copy of the planner's mats.                               */
+ * validated and must hold the bytes of the device copy blocks_dev; frags_dev
+ * is the device copy of the planner's frags.                              */
 int qsim_apply_passes(void* stream, void* state, int n_qubits, const qsim_pass* passes, int n_passes,
                       const qsim_pass_block* blocks_host, const void* blocks_dev,
-                      const void* mats_dev, int n_blocks);
+                      const void* frags_dev, int n_blocks);
 
 /* ---- reductions, measurement, sampling ---------------------------------- */
 /* Size in bytes of the workspace the reduction entry points need for a

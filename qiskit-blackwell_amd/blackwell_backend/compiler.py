@@ -379,18 +379,19 @@ PASS_MIN_QUBITS = 10     # smallest state (and tile) of the block passes
 
 class PassRun:
     """Consecutive block passes: PASS_DTYPE passes, PASS_BLOCK_DTYPE records
-    and float32 [blocks, 1024] matrix fragments, as the library takes them."""
-    __slots__ = ("passes", "blocks", "mats")
+    and uint16 [blocks, 3072] matrix fragments (bf16 bits), as the library
+    takes them."""
+    __slots__ = ("passes", "blocks", "frags")
 
-    def __init__(self, passes, blocks, mats):
+    def __init__(self, passes, blocks, frags):
         self.passes = passes
         self.blocks = blocks
-        self.mats = mats
+        self.frags = frags
 
 
 def plan_passes_arrays(n, op_nq, op_qubits, op_mats, tile_bits, low_bits):
     """The native pass planner (qsim_plan_passes) on flat arrays: (refs,
-    passes, blocks, mats); refs[e] >= 0 is pass refs[e], refs[e] < 0 is op
+    passes, blocks, frags); refs[e] >= 0 is pass refs[e], refs[e] < 0 is op
     -1 - refs[e] passed through (more than 4 qubits).  Host code that
     releases the GIL, as plan_blocks_arrays."""
     import ctypes
@@ -402,13 +403,13 @@ def plan_passes_arrays(n, op_nq, op_qubits, op_mats, tile_bits, low_bits):
     refs = np.zeros(m, dtype=np.int32)
     passes = np.zeros(m, dtype=_lib.PASS_DTYPE)
     blocks = np.zeros(m, dtype=_lib.PASS_BLOCK_DTYPE)
-    mats = np.empty((m, _lib.PASS_BLOCK_FLOATS), dtype=np.float32)
+    frags = np.empty((m, _lib.PASS_BLOCK_BF16), dtype=np.uint16)
     n_out, n_blk = ctypes.c_int(0), ctypes.c_int(0)
     vp = lambda a: ctypes.c_void_p(a.ctypes.data)
     _lib.call("qsim_plan_passes", n, tile_bits, low_bits, m, vp(nq), vp(qb), vp(mv.view(np.float64)),
-              vp(refs), vp(passes), vp(blocks), vp(mats), ctypes.byref(n_out), ctypes.byref(n_blk))
+              vp(refs), vp(passes), vp(blocks), vp(frags), ctypes.byref(n_out), ctypes.byref(n_blk))
     refs = refs[:n_out.value]
-    return refs, passes[:int((refs >= 0).sum())], blocks[:n_blk.value], mats[:n_blk.value]
+    return refs, passes[:int((refs >= 0).sum())], blocks[:n_blk.value], frags[:n_blk.value]
 
 
 def plan_passes(ops, n, tile_bits, low_bits):
@@ -419,7 +420,7 @@ def plan_passes(ops, n, tile_bits, low_bits):
     def flush():
         if not seg:
             return
-        refs, passes, blocks, mats = plan_passes_arrays(n, *_op_arrays(seg), tile_bits, low_bits)
+        refs, passes, blocks, frags = plan_passes_arrays(n, *_op_arrays(seg), tile_bits, low_bits)
         e = 0
         while e < len(refs):
             if refs[e] < 0:
@@ -434,7 +435,7 @@ def plan_passes(ops, n, tile_bits, low_bits):
             first = int(p["first_block"][0])
             last = int(p["first_block"][-1] + p["n_blocks"][-1])
             p["first_block"] -= first
-            out.append(PassRun(p, blocks[first:last], mats[first:last]))
+            out.append(PassRun(p, blocks[first:last], frags[first:last]))
         seg.clear()
 
     for op in ops:

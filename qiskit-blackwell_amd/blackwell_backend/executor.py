@@ -12,9 +12,9 @@ Modes:
   blocks - 5-qubit dense blocks on FP32 MFMA (n >= 10), other entries plain;
   blocks/<k> - the same with k-qubit blocks, k = 4, 5, 6 (k = 4 needs
            n >= 11 and k = 6 n >= 13 for their MFMA kernels);
-  passes - 4-qubit dense blocks on FP32 MFMA, many per trip through HBM
-           (n >= 10): tiles of 10..13 qubits stay in LDS for all the blocks
-           of a pass;
+  passes - 4-qubit dense blocks, FP32 values as exact bf16 triples on the
+           bf16 MFMA, many per trip through HBM (n >= 10): tiles of 10..13
+           qubits stay in LDS for all the blocks of a pass;
   tiles  - LDS tile programs, many ops per HBM pass;
   auto   - tiles (the whole state in one tile when n <= 13) for circuits with
            few ops per qubit on at most 20 qubits, else passes;
@@ -80,14 +80,17 @@ def default_tile_shape(n):
 
 def pass_shape(n):
     """(tile qubits, always-included low qubits) of the block passes.  Small
-    tiles spread a small state over more CUs, large ones take fewer passes;
-    times in us on MI355X for tiles of 10 / 11 / 12 / 13 qubits: 12-qubit
-    ladder 44 / 45 / 55, 16-qubit QFT 58 / 60 / 70 / 123, 20-qubit volume 256 /
-    235 / 226 / 283, 24-qubit 3213 / 2572 / 2544 / 2441, 28-qubit 73.3 / 58.0 /
-    54.9 / 52.0 ms.  Four low qubits make 128 B runs, whole cache lines; five
-    or six take more passes (28 qubits: 52.5 and 56.3 ms)."""
-    m = 10 if n <= 15 else (11 if n <= 18 else (12 if n <= 21 else 13))
-    return (n if n <= 11 else m), 4
+    tiles spread a small state over more CUs, large ones take fewer passes.
+    Times on MI355X for tiles of 10 / 11 / 12 / 13 qubits, us: 12-qubit ladder
+    36 / 32 / 32 / -, 14-qubit volume 48 / 47 / 51 / 76, 16-qubit QFT
+    48 / 44 / 44 / 82, 18-qubit volume 98 / 90 / 93 / 130, 20 qubits
+    222 / 188 / 175 / 209, 21 qubits 389 / 305 / 269 / 277, 22 qubits
+    641 / 515 / 444 / 431, 24 qubits 2650 / 2119 / 1986 / 1853; 28 qubits, ms:
+    64.5 / 50.8 / 43.1 / 41.8.  Four low qubits make 128 B runs, whole cache
+    lines; with five a plan takes more passes and is never faster."""
+    if n <= 12:
+        return n, 4
+    return (11 if n <= 15 else (12 if n <= 21 else 13)), 4
 
 
 def tune_tile_shapes(n):
@@ -447,8 +450,8 @@ class CompiledCircuit:
             if isinstance(e, C.PassRun):
                 # one device blob per plan: records then fragments of each run
                 steps.append(("passes", (e.passes, e.blocks, off, off + e.blocks.nbytes)))
-                parts += [e.blocks.view(np.uint8).reshape(-1), e.mats.view(np.uint8).reshape(-1)]
-                off += e.blocks.nbytes + e.mats.nbytes
+                parts += [e.blocks.view(np.uint8).reshape(-1), e.frags.view(np.uint8).reshape(-1)]
+                off += e.blocks.nbytes + e.frags.nbytes
             elif e.kind not in ("measure", "reset") and len(e.all_qubits) == 5:
                 steps.append(("sub", self._build_blocks(C.plan_blocks([e], self.n_qubits), device)))
             else:

@@ -10,7 +10,7 @@ Differences by design:
   * circuits are compiled by blackwell_backend.compiler (FP64 host fusion)
     into plans of prepared launches (blackwell_backend.executor);
   * the default execution mode is "auto": LDS tile programs for small or
-    shallow circuits, passes of 4-qubit FP32-MFMA blocks for the others;
+    shallow circuits, passes of 4-qubit MFMA blocks for the others;
     mode="blocks" runs one launch per 5-qubit block,
     mode="plain" runs one kernel per gate, mode="blocks/<k>" fuses into
     k-qubit MFMA blocks (k = 4, 5, 6) and mode="tune" times the modes and

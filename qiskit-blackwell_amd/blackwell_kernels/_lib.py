@@ -108,10 +108,10 @@ BLOCK_REC_DTYPE = np.dtype([("state", "<u8"), ("mat", "<u8"), ("set_begin", "<u8
                             ("n_qubits", "<i4"), ("q", "i1", (5,)), ("pad", "i1", (7,))])
 SAMPLE_REC_DTYPE = np.dtype([("state", "<u8"), ("out", "<u8"), ("seed", "<u8"), ("leaf_off", "<u8"),
                              ("shot_off", "<u8"), ("n_qubits", "<i4"), ("shots", "<u4")])
-# qsim_pass, qsim_pass_block and the floats of a block's matrix fragments
+# qsim_pass, qsim_pass_block and the bf16 values of a block's matrix fragments
 PASS_DTYPE = np.dtype([("tile_mask", "<u8"), ("first_block", "<i4"), ("n_blocks", "<i4")])
 PASS_BLOCK_DTYPE = np.dtype([("bit", "<u2", (16,))])
-PASS_BLOCK_FLOATS = 1024
+PASS_BLOCK_BF16 = 3072
 assert PASS_DTYPE.itemsize == 16 and PASS_BLOCK_DTYPE.itemsize == 32
 assert SAMPLE_REC_DTYPE.itemsize == 48
 assert OP_DTYPE.itemsize == 16 and INSTANCE_DTYPE.itemsize == 40 and BLOCK_REC_DTYPE.itemsize == 40

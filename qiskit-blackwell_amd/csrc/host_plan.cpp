@@ -262,17 +262,39 @@ static void pass_record(qsim_pass_block* rec, int m, const int* row) {
     if (!(used >> p & 1)) rec->bit[at++] = pass_index(p);
 }
 
-// MFMA A fragments of the 16 x 16 complex matrix u: row i = 2 r + part of the
-// real 32 x 32 form, slice s, half h -> out[s / 4][lane = 32 h + i][s % 4].
-static void pass_fragments(float* out, const double* u) {
-  for (int s = 0; s < kPassD; ++s)
+// x rounded to the nearest bf16 (ties to even); coefficients are finite.
+static uint16_t bf16_bits(float x) {
+  uint32_t u;
+  memcpy(&u, &x, 4);
+  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+static float bf16_value(uint16_t b) {
+  const uint32_t u = (uint32_t)b << 16;
+  float x;
+  memcpy(&x, &u, 4);
+  return x;
+}
+
+// A fragments of the 16 x 16 complex matrix u: row i = 2 r + part of its real
+// 32 x 32 form, split into hi + mid + lo, each the bf16 nearest to what the
+// parts before it leave (so the sum is within 2^-26 of the FP64 coefficient,
+// closer than its FP32 rounding).  Part k, half t of the K range: out[k][t][lane = 32 h + i][j], j the component (amplitude
+// 4 q + 2 h + e, part c) with j = 4 (q - 2 t) + 2 e + c.
+static void pass_fragments(uint16_t* out, const double* u) {
+  for (int t = 0; t < 2; ++t)
     for (int h = 0; h < 2; ++h)
-      for (int i = 0; i < 2 * kPassD; ++i) {
-        const double* e = u + 2 * ((i >> 1) * kPassD + s);
-        const int part = i & 1;
-        const double v = part == h ? e[0] : (part ? e[1] : -e[1]);
-        out[((s >> 2) * 64 + 32 * h + i) * 4 + (s & 3)] = (float)v;
-      }
+      for (int i = 0; i < 2 * kPassD; ++i)
+        for (int j = 0; j < 8; ++j) {
+          const int amp = 4 * (2 * t + (j >> 2)) + 2 * h + ((j >> 1) & 1), c = j & 1;
+          const double* e = u + 2 * ((i >> 1) * kPassD + amp);
+          const int part = i & 1;
+          double v = part == c ? e[0] : (part ? e[1] : -e[1]);
+          for (int k = 0; k < 3; ++k) {
+            const uint16_t b = bf16_bits((float)v);
+            out[((2 * k + t) * 64 + 32 * h + i) * 8 + j] = b;
+            v -= (double)bf16_value(b);
+          }
+        }
 }
 
 }  // namespace qsim
@@ -455,7 +477,7 @@ int qsim_plan_blocks(int n_qubits, int k, int n_ops, const int32_t* op_nq, const
 
 int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const int32_t* op_nq,
                      const int32_t* op_qubits, const double* op_mats, int32_t* out_ref,
-                     qsim_pass* passes, qsim_pass_block* blocks, float* mats, int* n_out,
+                     qsim_pass* passes, qsim_pass_block* blocks, uint16_t* frags, int* n_out,
                      int* n_blocks) {
   if (n_qubits < QSIM_PASS_MIN_TILE || n_qubits > QSIM_MAX_QUBITS)
     return fail(QSIM_ERANGE, "n_qubits=%d outside %d..%d", n_qubits, QSIM_PASS_MIN_TILE, QSIM_MAX_QUBITS);
@@ -466,7 +488,7 @@ int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const
     return fail(QSIM_EINVAL, "low_bits %d outside 1..%d", low_bits, m - kPassK);
   if (n_ops < 0) return fail(QSIM_EINVAL, "n_ops < 0");
   if (!n_out || !n_blocks || (n_ops > 0 && (!op_nq || !op_qubits || !op_mats || !out_ref || !passes || !blocks ||
-                                            !mats)))
+                                            !frags)))
     return fail(QSIM_EINVAL, "NULL pointer argument");
   try {
     PassPlan p;
@@ -564,7 +586,7 @@ int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const
       passes[np].n_blocks = n_ent;        // every entry is a block: no op here is wider than one
       for (int b = 0; b < n_ent; ++b, ++nb) {
         pass_record(blocks + nb, m, &bq[(size_t)b * 8]);
-        pass_fragments(mats + (size_t)nb * QSIM_PASS_BLOCK_FLOATS, &bm[(size_t)b * kPassD * kPassD * 2]);
+        pass_fragments(frags + (size_t)nb * QSIM_PASS_BLOCK_BF16, &bm[(size_t)b * kPassD * kPassD * 2]);
       }
       out_ref[ne++] = np++;
     }

@@ -9,16 +9,26 @@
 // A block is the real 32 x 32 matrix [[Re, -Im], [Im, Re]] of its 16 x 16
 // complex matrix, with rows and columns interleaved (index 2 r + part), acting
 // on the 32 real components of each group of 16 amplitudes.  One wave takes a
-// set of 32 groups: D (32 x 32) = A (32 x 32) B (32 x 32) in 16
-// v_mfma_f32_32x32x2_f32 with FP32 accumulation.
-//   A[i][2 s + h]: lane (h = l / 32, i = l % 32), packed by the planner in
-//     fragment order [s / 4][l][s % 4], so a wave reads it as four
-//     contiguous 1 KiB loads.
-//   B[2 s + h][c]: part h (0 = re, 1 = im) of amplitude s of group c: one
-//     ds_read_b32 per slice s, 64 lanes on 64 banks.
-//   D[i][c]: register q * 4 + 2 e + part of lane (h, c) is part `part` of
-//     amplitude 4 q + 2 h + e, so results leave as whole amplitudes
-//     (ds_write_b64).
+// set of 32 groups: D (32 x 32) = A (32 x 32) B (32 x 32).  Lane (h = l / 32,
+// c = l % 32) holds amplitudes 4 q + 2 h + e (q < 4, e < 2) of group c, both
+// as B operand and as D result (register 4 q + 2 e + part), so a set is read
+// and written as whole amplitudes at the same eight LDS addresses.
+//
+// Arithmetic: FP32 amplitudes as exact sums of three bf16 (hi + mid + lo, each
+// rounded to nearest, 3 x 8 bits), coefficients as three bf16 within 2^-26 of
+// their FP64 value (closer than FP32), multiplied on v_mfma_f32_32x32x16_bf16
+// with FP32 accumulation.  Products of two bf16 are exact.  The hi*hi sums have
+// an accumulator of their own, where they are all but exact; the five smaller
+// products (lo with hi, mid with mid, mid with hi; the three left out are below
+// 2^-26 of a term) are summed from the smallest up in a second one, and one
+// FP32 addition joins the two.  Error of the norm against FP64: 1.9e-7 after
+// 24 random blocks on 13 qubits, 5.0e-7 on the FP32 matrix instructions; SU(4)
+// volume 28 qubits 5.4e-7 against 1.2e-6.  Accumulating everything in one chain
+// doubles the error of structured blocks (27-qubit QFT 5.7e-7 against 3.5e-7).
+// A permutation block moves its amplitudes bit for bit (hi + (mid + lo) has no
+// rounding).  The FP32 instructions run at 1/16 of the bf16 rate and, measured
+// here, not beside VALU work: 277 us per block at 28 qubits (218 at their peak)
+// against 190 us.
 //
 // LDS addresses are linear over GF(2): amplitude j of the tile sits at
 // sw(j) = j with bits 5..9 and 10..13 folded onto bits 0..4.  The planner
@@ -27,14 +37,19 @@
 // banks whatever the block's qubits are.  The block record holds the swizzled
 // index of each single bit, so an address is an XOR of record entries.
 //
-// What bounds it: 128 flop per amplitude and block at the FP32 MFMA rate
-// (256 for a 5-qubit block, while a 4-qubit block absorbs about 3/4 of the ops
-// of a 5-qubit one) once a pass has three or more blocks; the trip through
-// memory below that.  At 28 qubits a block takes 277 us on top of the others
-// (218 at the matrix peak; tiles of 11, 12 or 13 qubits and 4, 8 or 16 waves
-// all measure 267-299) and a pass of one block 0.9 ms (0.68 for its bytes).
-// The depth-28 SU(4) circuit: 92 launches of 5-qubit blocks 76.7 ms, 32 passes
-// of 147 blocks 52.4 ms; depth 24 at 24 qubits 3.85 -> 2.44 ms.
+// What bounds it: the CU's issue of the phases of a block.  At 28 qubits a
+// block takes 190 us on top of the others; copies without one phase show
+// 74 us for the products, 57-74 for the splits (11 VALU instructions per
+// amplitude), 36-68 for the LDS writes and 29 for addresses and LDS reads,
+// nearly additive whatever the waves per SIMD, and a pass 0.42 ms (0.68 for
+// its bytes alone, partly hidden).  Two workgroups of 8 waves per CU (13-qubit
+// tiles) are the best of 4, 8 and 16 waves for states that fill the chip; a
+// 12-qubit tile takes 8 waves for the sake of states of at most 21 qubits, which
+// leave a CU one or two tiles (20 qubits: 175 us against 192 with 4 waves).
+// Loading a set's amplitudes beside the products of the set before it costs
+// registers and measured 208 against 190 us.  The depth-28 SU(4) circuit: 92
+// launches of 5-qubit blocks 76.7 ms, 32 passes of 147 blocks 40.4 ms; depth 24
+// at 24 qubits 3.85 -> 1.75 ms.
 #include "qsim_internal.hpp"
 #include <string.h>
 #include <algorithm>
@@ -42,17 +57,56 @@
 namespace qsim {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 struct PassGeom {
-  uint8_t tq[16];        // tile qubits, ascending; tq[0] = 0
+  uint32_t w[4];         // tile qubits, ascending, one byte each; the first is 0
+  __host__ __device__ int tq(int j) const { return (int)((w[j >> 2] >> (8 * (j & 3))) & 255u); }
 };
 
 constexpr uint32_t pass_sw(uint32_t j) { return j ^ ((j >> 5) & 31u) ^ ((j >> 10) & 31u); }
 
+constexpr int kFrags = 6;     // bf16 fragments of a block: parts hi, mid, lo x halves of the K range
+
+__device__ __forceinline__ bf16x8 as_frag(float4 v) { return __builtin_bit_cast(bf16x8, v); }
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+  const f32x2v v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+// x = hi + mid + lo exactly, each a pair of bf16 rounded to nearest.
+__device__ __forceinline__ void split3(float2 x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = pk_bf16(x.x, x.y);
+  const float rx = x.x - __uint_as_float(hi << 16), ry = x.y - __uint_as_float(hi & 0xffff0000u);
+  mid = pk_bf16(rx, ry);
+  lo = pk_bf16(rx - __uint_as_float(mid << 16), ry - __uint_as_float(mid & 0xffff0000u));
+}
+// The B fragments of a set: amplitudes 4 t .. 4 t + 3 of a lane are half t of
+// its K range.
+__device__ __forceinline__ void split_set(const float2 x[8], bf16x8 b[kFrags]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) split3(x[4 * t + p], w[0][p], w[1][p], w[2][p]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint4 v = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+      b[2 * k + t] = __builtin_bit_cast(bf16x8, v);
+    }
+  }
+}
+template <int KA, int KB>
+__device__ __forceinline__ f32x16 mul_parts(const bf16x8 a[kFrags], const bf16x8 b[kFrags], f32x16 acc) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2 * KA], b[2 * KB], acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2 * KA + 1], b[2 * KB + 1], acc, 0, 0, 0);
+}
+
 template <int M, int W, bool NT>
-__global__ __launch_bounds__(64 * W) void k_pass(float4* __restrict__ st, uint64_t n_tiles, PassGeom g,
-                                                 const uint4* __restrict__ blocks,
-                                                 const float4* __restrict__ mats, int n_blocks) {
+__global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uint64_t n_tiles, PassGeom g,
+                                                    const uint4* __restrict__ blocks,
+                                                    const float4* __restrict__ frags, int n_blocks) {
   constexpr int T = 64 * W;
   constexpr int SLOTS = (1 << (M - 1)) / T;           // float4 slots per thread
   constexpr int TB = __builtin_ctz(T);                // slot bits that run over the threads
@@ -61,23 +115,23 @@ __global__ __launch_bounds__(64 * W) void k_pass(float4* __restrict__ st, uint64
   extern __shared__ float4 X4[];
   char* Xb = reinterpret_cast<char*>(X4);
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint64_t base = gblock<uint64_t>();
   if (base >= n_tiles) return;                        // whole workgroup: past the last tile
 #pragma unroll
-  for (int j = 0; j < M; ++j) base = ins0(base, g.tq[j]);
-  base >>= 1;                                         // in slots; tq[0] = 0
+  for (int j = 0; j < M; ++j) base = ins0(base, g.tq(j));
+  base >>= 1;                                         // in slots; the first tile qubit is 0
   uint64_t toff = 0;
 #pragma unroll
-  for (int j = 0; j < TB; ++j) toff |= (uint64_t)((tid >> j) & 1) << (g.tq[j + 1] - 1);
+  for (int j = 0; j < TB; ++j) toff |= (uint64_t)((tid >> j) & 1) << (g.tq(j + 1) - 1);
   const uint32_t tsw = pass_sw(2u * tid);
   uint64_t koff[SLOTS];
 #pragma unroll
   for (int k = 0; k < SLOTS; ++k) {
     koff[k] = base;
 #pragma unroll
-    for (int j = TB; j < M - 1; ++j) koff[k] |= (uint64_t)((k >> (j - TB)) & 1) << (g.tq[j + 1] - 1);
+    for (int j = TB; j < M - 1; ++j) koff[k] |= (uint64_t)((k >> (j - TB)) & 1) << (g.tq(j + 1) - 1);
   }
   {
     float4 v[SLOTS];
@@ -92,66 +146,62 @@ __global__ __launch_bounds__(64 * W) void k_pass(float4* __restrict__ st, uint64
                                odd ? v[k].y : v[k].w);
     }
   }
-  const int h = lane >> 5;
-  float4 a[4];
+  bf16x8 a[kFrags];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) a[q] = mats[q * 64 + lane];
+  for (int q = 0; q < kFrags; ++q) a[q] = as_frag(frags[q * 64 + lane]);
   uint4 d0 = blocks[0], d1 = blocks[1];
   __syncthreads();
   for (int b = 0; b < n_blocks; ++b) {
     // record: row[4], lane[5], set[5] (16-bit swizzled single-bit indices)
     const uint32_t r0 = (d0.x & 0xffffu) * 8u, r1 = (d0.x >> 16) * 8u, r2 = (d0.y & 0xffffu) * 8u,
                    r3 = (d0.y >> 16) * 8u;
-    uint32_t lb = 4u * h;
+    uint32_t lb = h ? r1 : 0u;            // row bit 1 is the lane half
     lb ^= (lane & 1) ? (d0.z & 0xffffu) * 8u : 0u;
     lb ^= (lane & 2) ? (d0.z >> 16) * 8u : 0u;
     lb ^= (lane & 4) ? (d0.w & 0xffffu) * 8u : 0u;
     lb ^= (lane & 8) ? (d0.w >> 16) * 8u : 0u;
     lb ^= (lane & 16) ? (d1.x & 0xffffu) * 8u : 0u;
-    const uint32_t sb[5] = {(d1.x >> 16) * 8u, (d1.y & 0xffffu) * 8u, (d1.y >> 16) * 8u, (d1.z & 0xffffu) * 8u,
-                            (d1.z >> 16) * 8u};
-    uint32_t ro[16];
+    const uint32_t sb[4] = {(d1.x >> 16) * 8u, (d1.y & 0xffffu) * 8u, (d1.y >> 16) * 8u, (d1.z & 0xffffu) * 8u};
+    uint32_t ro[8];                       // amplitude 4 q + e of a lane at index 2 q + e
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
-      ro[s] = ((s & 1) ? r0 : 0u) ^ ((s & 2) ? r1 : 0u) ^ ((s & 4) ? r2 : 0u) ^ ((s & 8) ? r3 : 0u);
-    // the next block's fragments and record arrive while this one runs
+    for (int s = 0; s < 8; ++s) ro[s] = ((s & 1) ? r0 : 0u) ^ ((s & 2) ? r2 : 0u) ^ ((s & 4) ? r3 : 0u);
     const int nb = b + 1 < n_blocks ? b + 1 : b;
-    float4 an[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) an[q] = mats[(size_t)nb * 256 + q * 64 + lane];
     const uint4 e0 = blocks[2 * nb], e1 = blocks[2 * nb + 1];
-    const float* af = reinterpret_cast<const float*>(a);
     if (SETS >= W || wave < SETS) {
-      float x[SPW][16];
       uint32_t sbase[SPW];
 #pragma unroll
       for (int i = 0; i < SPW; ++i) {
         const int set = wave + W * i;
-        uint32_t so = 0;
+        sbase[i] = lb;
 #pragma unroll
-        for (int j = 0; j < M - 9; ++j) so ^= ((set >> j) & 1) ? sb[j] : 0u;
-        sbase[i] = lb ^ so;
-#pragma unroll
-        for (int s = 0; s < 16; ++s) x[i][s] = *reinterpret_cast<const float*>(Xb + (sbase[i] ^ ro[s]));
+        for (int j = 0; j < M - 9; ++j) sbase[i] ^= ((set >> j) & 1) ? sb[j] : 0u;
       }
 #pragma unroll
       for (int i = 0; i < SPW; ++i) {
-        f32x16 acc = {0.f};
+        float2 x[8];
 #pragma unroll
-        for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[s], x[i][s], acc, 0, 0, 0);
-        // rows 4 q + 2 h + e: row bit 1 is the lane half
-        const uint32_t wb = sbase[i] ^ (h ? (r1 ^ 4u) : 0u);
+        for (int s = 0; s < 8; ++s) x[s] = *reinterpret_cast<const float2*>(Xb + (sbase[i] ^ ro[s]));
+        bf16x8 bp[kFrags];
+        split_set(x, bp);
+        f32x16 big = {0.f}, small = {0.f};
+        big = mul_parts<0, 0>(a, bp, big);
+        small = mul_parts<0, 2>(a, bp, small);
+        small = mul_parts<2, 0>(a, bp, small);
+        small = mul_parts<1, 1>(a, bp, small);
+        small = mul_parts<0, 1>(a, bp, small);
+        small = mul_parts<1, 0>(a, bp, small);
+        if (i + 1 == SPW) {
+          // the next block's fragments travel while the results are written
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+          for (int q = 0; q < kFrags; ++q) a[q] = as_frag(frags[(size_t)nb * (64 * kFrags) + q * 64 + lane]);
+        }
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            *reinterpret_cast<float2*>(Xb + (wb ^ ro[4 * q + e])) =
-                make_float2(acc[4 * q + 2 * e], acc[4 * q + 2 * e + 1]);
+        for (int s = 0; s < 8; ++s)
+          *reinterpret_cast<float2*>(Xb + (sbase[i] ^ ro[s])) =
+              make_float2(big[2 * s] + small[2 * s], big[2 * s + 1] + small[2 * s + 1]);
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = an[q];
     d0 = e0;
     d1 = e1;
   }
@@ -166,15 +216,15 @@ __global__ __launch_bounds__(64 * W) void k_pass(float4* __restrict__ st, uint64
 
 template <int M, int W>
 static void launch_pass(hipStream_t s, void* state, int n, const PassGeom& g, const qsim_pass_block* blocks,
-                        const float* mats, int n_blocks) {
+                        const void* frags, int n_blocks) {
   const uint64_t tiles = 1ull << (n - M);
   const size_t lds = sizeof(float2) << M;
   if (nt_for_qubits(n))
     hipLaunchKernelGGL((k_pass<M, W, true>), grid1d(tiles), dim3(64 * W), lds, s, (float4*)state, tiles, g,
-                       (const uint4*)blocks, (const float4*)mats, n_blocks);
+                       (const uint4*)blocks, (const float4*)frags, n_blocks);
   else
     hipLaunchKernelGGL((k_pass<M, W, false>), grid1d(tiles), dim3(64 * W), lds, s, (float4*)state, tiles, g,
-                       (const uint4*)blocks, (const float4*)mats, n_blocks);
+                       (const uint4*)blocks, (const float4*)frags, n_blocks);
 }
 
 // Host check of one record: the swizzled indices of m distinct tile bits.
@@ -197,13 +247,13 @@ using namespace qsim;
 extern "C" {
 
 int qsim_apply_passes(void* stream, void* state, int n_qubits, const qsim_pass* passes, int n_passes,
-                      const qsim_pass_block* blocks_host, const void* blocks_dev, const void* mats_dev,
+                      const qsim_pass_block* blocks_host, const void* blocks_dev, const void* frags_dev,
                       int n_blocks) {
   clear_error();
   if (int rc = check_n(n_qubits)) return rc;
   if (n_passes < 0 || n_blocks < 0) return fail(QSIM_EINVAL, "negative count");
   if (n_passes == 0) return QSIM_OK;
-  if (!state || !passes || !blocks_host || !blocks_dev || !mats_dev)
+  if (!state || !passes || !blocks_host || !blocks_dev || !frags_dev)
     return fail(QSIM_EINVAL, "NULL pointer argument");
   for (int i = 0; i < n_passes; ++i) {
     const qsim_pass& p = passes[i];
@@ -228,14 +278,17 @@ int qsim_apply_passes(void* stream, void* state, int n_qubits, const qsim_pass* 
     memset(&g, 0, sizeof g);
     int m = 0;
     for (int q = 0; q < n_qubits; ++q)
-      if (p.tile_mask >> q & 1) g.tq[m++] = (uint8_t)q;
+      if (p.tile_mask >> q & 1) {
+        g.w[m >> 2] |= (uint32_t)q << (8 * (m & 3));
+        ++m;
+      }
     const qsim_pass_block* bd = (const qsim_pass_block*)blocks_dev + p.first_block;
-    const float* md = (const float*)mats_dev + (size_t)p.first_block * QSIM_PASS_BLOCK_FLOATS;
+    const uint16_t* fd = (const uint16_t*)frags_dev + (size_t)p.first_block * QSIM_PASS_BLOCK_BF16;
     switch (m) {
-      case 10: launch_pass<10, 4>(s, state, n_qubits, g, bd, md, p.n_blocks); break;
-      case 11: launch_pass<11, 4>(s, state, n_qubits, g, bd, md, p.n_blocks); break;
-      case 12: launch_pass<12, 8>(s, state, n_qubits, g, bd, md, p.n_blocks); break;
-      default: launch_pass<13, 8>(s, state, n_qubits, g, bd, md, p.n_blocks); break;
+      case 10: launch_pass<10, 4>(s, state, n_qubits, g, bd, fd, p.n_blocks); break;
+      case 11: launch_pass<11, 4>(s, state, n_qubits, g, bd, fd, p.n_blocks); break;
+      case 12: launch_pass<12, 8>(s, state, n_qubits, g, bd, fd, p.n_blocks); break;
+      default: launch_pass<13, 8>(s, state, n_qubits, g, bd, fd, p.n_blocks); break;
     }
     if (int rc = launch_status("apply_passes")) return rc;
   }

@@ -17,12 +17,14 @@ def _sw(p):
 
 
 def _matrix(frag):
-    """16 x 16 complex matrix of a block's fragments [4][64][4]."""
+    """16 x 16 complex matrix of a block's fragments bf16 [3][2][64][8]."""
+    f = (np.asarray(frag).astype(np.uint32) << 16).view(np.float32).astype(np.float64).reshape(3, 2, 64, 8).sum(axis=0)
     a = np.zeros((32, 32))
-    f = np.asarray(frag, dtype=np.float64).reshape(4, 64, 4)
-    for s in range(16):
+    for t in range(2):
         for h in range(2):
-            a[:, 2 * s + h] = f[s >> 2, 32 * h:32 * h + 32, s & 3]
+            for j in range(8):
+                amp = 4 * (2 * t + (j >> 2)) + 2 * h + ((j >> 1) & 1)
+                a[:, 2 * amp + (j & 1)] = f[t, 32 * h:32 * h + 32, j]
     assert np.array_equal(a[1::2, 1::2], a[0::2, 0::2]) and np.array_equal(a[0::2, 1::2], -a[1::2, 0::2])
     return a[0::2, 0::2] + 1j * a[1::2, 0::2]
 
@@ -35,7 +37,7 @@ def _replay(psi, n, run):
             assert sorted(bits) == list(range(len(tile)))
             assert [int(v) for v in run.blocks["bit"][b][:len(tile)]] == [_sw(x) for x in bits]
             assert not run.blocks["bit"][b][len(tile):].any()
-            psi = O.apply_matrix(psi, _matrix(run.mats[b]), [tile[x] for x in bits[:4]])
+            psi = O.apply_matrix(psi, _matrix(run.frags[b]), [tile[x] for x in bits[:4]])
     return psi
 
 
@@ -57,8 +59,8 @@ def test_planned_passes_equal_the_circuit(n, m, low):
             wide += 1
             psi = O.apply_matrix(psi, e.full_matrix(), list(e.all_qubits))
     assert wide == sum(len(o.all_qubits) > 4 for o in ops)
-    # fragments are rounded to FP32 once: at most 2^-24 per coefficient, 16 per row, over the blocks
-    assert np.max(np.abs(psi - _sim_ops(n, ops))) < 150 * 16 * 2.0 ** -24
+    # coefficients are within 2^-26, two parts of 16 to a row, over at most 150 blocks
+    assert np.max(np.abs(psi - _sim_ops(n, ops))) < 150 * 32 * 2.0 ** -26
 
 
 def test_pass_arguments_are_checked():
@@ -84,7 +86,7 @@ def test_pass_arguments_are_checked():
         assert call(blk=bad) == 1, (at, v)
     nq, qs, mat = np.array([2], np.int32), np.full((1, 8), -1, np.int32), np.eye(4, dtype=np.complex128)
     qs[0, :2] = 0, 9
-    out = [np.zeros(1, np.int32), passes, blocks, np.zeros(1024, np.float32)]
+    out = [np.zeros(1, np.int32), passes, blocks, np.zeros(3072, np.uint16)]
     a, b = ctypes.c_int(), ctypes.c_int()
 
     def plan(n=12, m=10, low=4, w=2, q=9):
@@ -102,7 +104,7 @@ def test_pass_arguments_are_checked():
 def test_pass_kernel_matches_fp64(bk, dev, n, m):
     """Random 1-, 2- and 4-qubit unitaries on spread-out qubits (every tile
     bit takes part) on a random state.  One block costs at most 8e-6 max|a|
-    (32-term FP32 dot products on groups of 16 amplitudes)."""
+    (32-term dot products accumulated in FP32 on groups of 16 amplitudes)."""
     import torch
     from blackwell_backend import compiler as C
     from blackwell_backend.executor import CompiledCircuit
