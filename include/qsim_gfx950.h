@@ -516,6 +516,33 @@ int qsim_cheb_pauli_step(void* stream, int n_qubits, int n_groups, const void* x
                          const void* sm, const void* coef, const void* gconst, double scale,
                          const void* t_cur, void* t_prev_next, void* acc, void* comp, double c_re,
                          double c_im, int first);
+/* One X-mask group of a Pauli sum with real entries, for
+ * qsim_cheb_pauli_batch_step: X mask, its nt terms at [t0, t0 + nt) of sm and
+ * coef, and by kind
+ *   CONST  same = the entry, the same in every row;
+ *   PAIR   one or two terms: masks m0, m1 and coefficients c0, c1 (a missing
+ *          second term has mask and coefficient 0), same = c0 + c1 and
+ *          diff = c0 - c1 rounded to FP32;
+ *   TERMS  any number of terms, read from sm and coef (real parts).        */
+#define QSIM_PAULI_GROUP_CONST 0
+#define QSIM_PAULI_GROUP_PAIR  1
+#define QSIM_PAULI_GROUP_TERMS 2
+#define QSIM_PAULI_BATCH_MIN_QUBITS 9
+typedef struct qsim_pauli_group {
+  uint64_t xm;
+  uint32_t t0;
+  uint16_t nt, kind;
+  double   same, diff, c0, c1;
+  uint64_t m0, m1;
+} qsim_pauli_group;
+/* qsim_cheb_pauli_step for n_rhs vectors (vector j at j * 2^n_qubits elements
+ * of t_cur, t_prev_next, acc and comp) and a Hamiltonian whose entries are all
+ * real: groups (device, ascending X masks), sm and coef as in its tables.
+ * Same sums in the same order.  t_cur: 16-byte aligned.  (new)            */
+int qsim_cheb_pauli_batch_step(void* stream, int n_qubits, int n_groups, const void* groups,
+                               const void* sm, const void* coef, int n_rhs, double scale,
+                               const void* t_cur, void* t_prev_next, void* acc, void* comp,
+                               double c_re, double c_im, int first);
 /* acc = c * t, comp = 0 (first Chebyshev term), n elements. (new)        */
 int qsim_cheb_init_acc(void* stream, void* acc, void* comp, const void* t, int64_t n,
                        double c_re, double c_im);

@@ -13,7 +13,7 @@ Device work per term is ONE launch (qsim_cheb_spmm_step): SpMM of the
 scaled Hamiltonian against the current term, the recurrence
 T_{k+1} = 2 H~ T_k - T_{k-1} written over T_{k-1}, and the Kahan/Neumaier
 accumulation acc += c_k T_{k+1} with its compensation vector.  Any number
-of right-hand sides runs in the same launch, stored RHS-contiguous.
+of right-hand sides runs in the same launch (RHS-contiguous on the CSR).
 
 split=True runs each term as two launches over the CSR split at bit n/2
 (HamiltonianCSR.split, qsim_cheb_spmm_step_split; 32 right-hand sides,
@@ -28,8 +28,12 @@ the default.
 A Hamiltonian built from a Pauli sum keeps its grouped Pauli tables, and a
 single state with FP64 row sums runs each term matrix-free by default
 (qsim_cheb_pauli_step): every entry is recomputed from the tables as the
-CSR builder computes it, so no index or value stream is read, and the CSR
-stays for batches, fp32c row sums and the split term.
+CSR builder computes it, so no index or value stream is read.  Batches of
+16 qubits and more do the same when all entries are real
+(qsim_cheb_pauli_batch_step, state-major, so without the two transposes):
+the states share the entry evaluation and a tile of T_k in LDS, and the
+sums are those of the CSR term bit for bit.  The CSR stays for small
+batches, complex entries, fp32c row sums and the split term.
 
 Row sums of the SpMM (accumulate=):
   "fp64"   every FP32 x FP32 product is exact in FP64 and is summed with
@@ -79,6 +83,21 @@ def chebyshev_coefficients(t, spectral_bound, precision=1e-10):
 ACCUMULATE = {"fp64": 0, "fp32c": 1}
 
 
+def tiled_term(pauli, n, R):
+    """Whether the tiled matrix-free term (qsim_cheb_pauli_batch_step) runs R
+    states of n qubits: real entries, and a size where it measured faster
+    than what it replaces.  Batches against the CSR term, us per term of a
+    Heisenberg chain: 17 qubits with 2 / 32 states 23 -> 16 and 81 -> 67,
+    16 qubits with 16 states 33 -> 30 but with 8 states 20 -> 24, 14 qubits
+    with 32 states 12 -> 16 (the CSR and T_k fit the L2s there).  One state
+    against the untiled term: 18 qubits 17.1 -> 14.3, 19 qubits 25 -> 26."""
+    if pauli.groups is None or n < _lib.PAULI_BATCH_MIN_QUBITS:
+        return False
+    if R == 1:
+        return n <= 18
+    return R > 1 and (n >= 17 or (n == 16 and R >= 16))
+
+
 def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumulate="fp64", split=False,
                            matrix_free=None):
     """Evolve R states at once.  states: complex64 [R, 2^n] (or [2^n]) on the
@@ -87,7 +106,8 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     matrix_free: run each term from the Pauli tables the Hamiltonian was
     built from (qsim_cheb_pauli_step) instead of the CSR; None (default)
     does so for one state with accumulate="fp64" when the Hamiltonian
-    carries its Pauli tables."""
+    carries its Pauli tables, and, when its entries are real, for batches of
+    the sizes tiled_term names (qsim_cheb_pauli_batch_step)."""
     if accumulate not in ACCUMULATE:
         raise ValueError(f"accumulate must be one of {sorted(ACCUMULATE)}, got {accumulate!r}")
     mode = ACCUMULATE[accumulate]
@@ -102,12 +122,22 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     t_start = time.perf_counter()
     coeffs, K, tail = chebyshev_coefficients(t, h.spectral_bound, precision)
     scale = 1.0 / h.spectral_bound
-    # RHS-contiguous buffers [N, R]; A is always a copy (for one state the
-    # transpose is already contiguous and would alias the caller's tensor,
-    # which the recurrence overwrites)
-    A = X.transpose(0, 1).contiguous()
-    if A.data_ptr() == X.data_ptr():
-        A = A.clone()
+    pauli = getattr(h, "pauli", None)
+    use_split = bool(split)
+    if use_split and not (mode == ACCUMULATE["fp64"] and R == 32 and 4 <= N <= (1 << 24)):
+        raise ValueError("split=True needs accumulate='fp64', 32 states and 4..2^24 rows "
+                         f"(got {accumulate!r}, {R} states, {N} rows)")
+    mf_ok = pauli is not None and R == 1 and mode == ACCUMULATE["fp64"] and not use_split
+    use_mf = mf_ok if matrix_free is None else bool(matrix_free)
+    if use_mf and not mf_ok:
+        raise ValueError("matrix_free=True needs a Hamiltonian built from a Pauli sum, one state, "
+                         f"accumulate='fp64' and split=False (got {R} states, {accumulate!r})")
+    use_tiled = (pauli is not None and mode == ACCUMULATE["fp64"] and not use_split
+                 and (use_mf or matrix_free is None) and tiled_term(pauli, h.n_qubits, R))
+    # A is always a copy, the recurrence overwrites it: [R, N] as given for
+    # the tiled term, else RHS-contiguous [N, R]
+    A = torch.empty(X.shape if use_tiled else (N, R), dtype=X.dtype, device=dev)
+    A.copy_(X if use_tiled else X.transpose(0, 1))
     B = torch.empty_like(A)
     acc = torch.empty_like(A)
     comp = torch.empty_like(A)
@@ -115,17 +145,13 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     n_el = N * R
     c0 = complex(coeffs[0])
     call("qsim_cheb_init_acc", s, ptr(acc), ptr(comp), ptr(A), n_el, c0.real, c0.imag)
-    use_split = bool(split)
-    if use_split and not (mode == ACCUMULATE["fp64"] and R == 32 and 4 <= N <= (1 << 24)):
-        raise ValueError("split=True needs accumulate='fp64', 32 states and 4..2^24 rows "
-                         f"(got {accumulate!r}, {R} states, {N} rows)")
-    pauli = getattr(h, "pauli", None)
-    mf_ok = pauli is not None and R == 1 and mode == ACCUMULATE["fp64"] and not use_split
-    use_mf = mf_ok if matrix_free is None else bool(matrix_free)
-    if use_mf and not mf_ok:
-        raise ValueError("matrix_free=True needs a Hamiltonian built from a Pauli sum, one state, "
-                         f"accumulate='fp64' and split=False (got {R} states, {accumulate!r})")
-    if use_mf:
+    if use_tiled:
+        targs = (h.n_qubits,) + pauli.batch_args() + (R, scale)
+
+        def term(cur_, prv_, ck, first):
+            call("qsim_cheb_pauli_batch_step", s, *targs, ptr(cur_), ptr(prv_), ptr(acc), ptr(comp),
+                 ck.real, ck.imag, first)
+    elif use_mf:
         pargs = (h.n_qubits,) + pauli.step_args() + (scale,)
 
         def term(cur_, prv_, ck, first):
@@ -151,7 +177,7 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
         term(cur, prv, complex(coeffs[k]), 0)
         cur, prv = prv, cur
     call("qsim_cheb_finish", s, ptr(prv), ptr(acc), ptr(comp), n_el)
-    out = prv.transpose(0, 1).contiguous()
+    out = prv if use_tiled else prv.transpose(0, 1).contiguous()
     torch.cuda.synchronize(dev)
     elapsed = time.perf_counter() - t_start
     info = {
@@ -167,7 +193,7 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
         "n_rhs": R,
         "accumulate": accumulate,
         "split_term": bool(use_split),
-        "matrix_free": bool(use_mf),
+        "matrix_free": bool(use_mf or use_tiled),
     }
     return (out[0] if single else out), info
 

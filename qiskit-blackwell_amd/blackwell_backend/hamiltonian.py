@@ -91,9 +91,10 @@ def constant_group_entries(toff, sm, coef):
     coefficients in term order, as the device evaluates it; NaN where the
     entry depends on the row."""
     out = np.full((len(toff) - 1, 2), np.nan)
+    masked = (sm != 0).tolist()
     for g in range(len(toff) - 1):
         t0, t1 = int(toff[g]), int(toff[g + 1])
-        if np.any(sm[t0:t1] != 0):
+        if any(masked[t0:t1]):
             continue
         re = im = 0.0
         for t in range(t0, t1):
@@ -103,11 +104,38 @@ def constant_group_entries(toff, sm, coef):
     return out
 
 
+def real_group_records(xm, toff, sm, coef, gconst):
+    """PAULI_GROUP_DTYPE records of pauli_groups() tables and their
+    constant_group_entries (see qsim_pauli_group), or None when a coefficient has an imaginary part or a
+    group more terms than a record counts."""
+    from blackwell_kernels import _lib
+    counts = np.diff(toff)
+    if np.any(coef.imag != 0) or np.any(counts > 0xffff):
+        return None
+    recs = np.zeros(len(xm), dtype=_lib.PAULI_GROUP_DTYPE)
+    if not len(xm):
+        return recs
+    t0 = toff[:-1]
+    t1 = np.minimum(t0 + 1, len(sm) - 1)
+    two = counts > 1
+    c = np.stack([coef.real[t0], np.where(two, coef.real[t1], 0.0)], axis=1)
+    const = ~np.isnan(gconst[:, 0])
+    pair = ~const & (counts <= 2)
+    recs["xm"], recs["t0"], recs["nt"] = xm, t0, counts
+    recs["kind"] = np.where(const, _lib.PAULI_CONST, np.where(pair, _lib.PAULI_PAIR, _lib.PAULI_TERMS))
+    recs["c"][pair] = c[pair]
+    recs["m"][pair] = np.stack([sm[t0], np.where(two, sm[t1], 0)], axis=1)[pair]
+    recs["same"] = np.where(const, gconst[:, 0], (c[:, 0] + c[:, 1]).astype(np.float32))
+    recs["diff"][pair] = (c[:, 0] - c[:, 1]).astype(np.float32)[pair]
+    return recs
+
+
 class PauliTables:
     """pauli_groups() on a device: n_groups and the tensors xm (uint64 as
     int64), toff (int32), sm (uint64 as int64), coef (FP64 pairs), the
     layout qsim_pauli_csr_count and qsim_cheb_pauli_step take, plus gconst
-    (constant_group_entries) for the matrix-free Chebyshev term."""
+    (constant_group_entries) for the matrix-free Chebyshev term and, when
+    every coefficient is real, groups (real_group_records, else None)."""
 
     def __init__(self, labels, coeffs, device):
         xm, toff, sm, coef = pauli_groups(labels, coeffs)
@@ -119,6 +147,8 @@ class PauliTables:
         self.coef = torch.from_numpy(coef.view(np.float64) if coef.size else np.zeros(2)).to(dev)
         gc = constant_group_entries(toff, sm, coef)
         self.gconst = torch.from_numpy(gc.reshape(-1) if gc.size else np.zeros(2)).to(dev)
+        recs = real_group_records(xm, toff, sm, coef, gc)
+        self.groups = None if recs is None or not recs.size else torch.from_numpy(recs.view(np.uint8)).to(dev)
 
     def args(self):
         """(n_groups, xm, toff, sm, coef) pointers for qsim_pauli_csr_count / _fill."""
@@ -129,6 +159,11 @@ class PauliTables:
         """args() plus gconst, for qsim_cheb_pauli_step."""
         from blackwell_kernels import _lib
         return self.args() + (_lib.ptr(self.gconst),)
+
+    def batch_args(self):
+        """(n_groups, groups, sm, coef) pointers for qsim_cheb_pauli_batch_step."""
+        from blackwell_kernels import _lib
+        return (self.n_groups, _lib.ptr(self.groups), _lib.ptr(self.sm), _lib.ptr(self.coef))
 
 
 def pauli_to_csr_device(labels, coeffs, n, device, tables=None):

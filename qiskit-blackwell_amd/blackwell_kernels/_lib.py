@@ -94,6 +94,7 @@ PROTOTYPES = {
     "qsim_cheb_spmm_step_split": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _d, _vp, _vp, _vp,
                                        _vp, _vp, _d, _d, _i]),
     "qsim_cheb_pauli_step": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _d, _vp, _vp, _vp, _vp, _d, _d, _i]),
+    "qsim_cheb_pauli_batch_step": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _d, _vp, _vp, _vp, _vp, _d, _d, _i]),
     "qsim_cheb_init_acc": (_i, [_vp, _vp, _vp, _vp, _i64, _d, _d]),
     "qsim_cheb_finish": (_i, [_vp, _vp, _vp, _vp, _i64]),
 }
@@ -112,6 +113,12 @@ SAMPLE_REC_DTYPE = np.dtype([("state", "<u8"), ("out", "<u8"), ("seed", "<u8"), 
 PASS_DTYPE = np.dtype([("tile_mask", "<u8"), ("first_block", "<i4"), ("n_blocks", "<i4")])
 PASS_BLOCK_DTYPE = np.dtype([("bit", "<u2", (16,))])
 PASS_BLOCK_BF16 = 3072
+# qsim_pauli_group and its kinds
+PAULI_GROUP_DTYPE = np.dtype([("xm", "<u8"), ("t0", "<u4"), ("nt", "<u2"), ("kind", "<u2"), ("same", "<f8"),
+                              ("diff", "<f8"), ("c", "<f8", (2,)), ("m", "<u8", (2,))])
+PAULI_CONST, PAULI_PAIR, PAULI_TERMS = range(3)
+PAULI_BATCH_MIN_QUBITS = 9
+assert PAULI_GROUP_DTYPE.itemsize == 64
 assert PASS_DTYPE.itemsize == 16 and PASS_BLOCK_DTYPE.itemsize == 32
 assert SAMPLE_REC_DTYPE.itemsize == 48
 assert OP_DTYPE.itemsize == 16 and INSTANCE_DTYPE.itemsize == 40 and BLOCK_REC_DTYPE.itemsize == 40

@@ -205,6 +205,10 @@ struct RowSum<kAccF64> {
     i = __builtin_fma(vr, xi, i);
     i = __builtin_fma(vi, xr, i);
   }
+  __device__ __forceinline__ void add_r(double vr, float2 x) {
+    r = __builtin_fma(vr, (double)x.x, r);
+    i = __builtin_fma(vr, (double)x.y, i);
+  }
   // scale * sum, rounded once to FP32 after the recurrence update
   __device__ __forceinline__ float2 next(double scale, float2 tp, bool first) const {
     const double wr = r * scale, wi = i * scale;
@@ -717,6 +721,197 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli1(int n_groups, const ui
   }
 }
 
+// Matrix-free term over a Pauli sum with real entries, C right-hand sides per
+// workgroup (RHS-major: vector j at j * 2^n).  A workgroup owns a tile of 256
+// consecutive rows, lane = row: it copies the tile's T_k (C vectors) into LDS,
+// serves the groups whose X mask stays inside the tile from there, and loads
+// the others as the contiguous partner tile (lanes permuted by the mask's low
+// bits).  Entries, their rounding and the FP64 sum in group order are those of
+// k_cheb_pauli1, so the results have its bits; a row whose entry is zero adds
+// nothing, and a group whose entry is zero in the whole wave loads nothing.
+//  * Tables: one 64-byte record per group (qsim_pauli_group) holds everything
+//    of a group of one or two terms, so a group costs one scalar load instead
+//    of a chain of four.
+//  * C = 4: the entry of one or two terms is picked, not summed: the wave's
+//    part of the parities on the scalar unit, the lane's part by popcounts
+//    only where a mask reaches the lane bits.  C = 1 sums the signed terms
+//    (the scalar work would not be shared).
+//  * A branch merges before the FMAs: every kind of group yields one value per
+//    row, and one sequence of FMAs adds it (FMAs in each branch made the
+//    compiler copy the FP64 sums at every merge: 48 VALU instructions per
+//    group at C = 4 against 36; 12.5 against 11.2 us at C = 1, 17 qubits).
+// What bounds it: at C = 4 the T_k loads that miss L2 (3.2 GB per 20-qubit term
+// of 32 right-hand sides, about 5.5 TB/s), then the entry evaluation; at C = 1
+// the evaluation.  Times per term of a Heisenberg chain against the kernels
+// before, us: 20 qubits with 2 / 4 / 8 / 32 right-hand sides 273 / 278 / 385 /
+// 838 (CSR) -> 72 / 88 / 153 / 617, 22 qubits with 32 3660 -> 2672; one
+// right-hand side of 10 / 15 / 18 qubits 9.5 / 14.1 / 17.1 (k_cheb_pauli1) ->
+// 7.5 / 10.0 / 14.3.  C = 2 and 8 and tiles of 512 and 1024 rows measured the
+// same to 15 % slower.
+struct PauliGroup {       // qsim_pauli_group
+  uint64_t xm;
+  uint32_t t0;
+  uint16_t nt, kind;
+  double same, diff, c0, c1;
+  uint64_t m0, m1;
+};
+static_assert(sizeof(PauliGroup) == 64 && sizeof(qsim_pauli_group) == 64, "group record");
+__device__ __forceinline__ bool nonzero(double v) { return (__double_as_longlong(v) << 1) != 0; }
+__device__ __forceinline__ double flip_sign(double v, uint32_t bit31) {
+  return __hiloint2double((int)((uint32_t)__double2hiint(v) ^ bit31), __double2loint(v));
+}
+
+template <typename R, int C, int U, bool NT>
+__global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const PauliGroup* __restrict__ tab,
+                                                         const uint64_t* __restrict__ sm,
+                                                         const double2* __restrict__ coef, int n_bits,
+                                                         int n_rhs, int by_rhs, double scale,
+                                                         const float2* __restrict__ tc,
+                                                         float2* __restrict__ tpn, float2* __restrict__ acc,
+                                                         float2* __restrict__ comp, float2 c, int first) {
+  constexpr uint32_t rows = kThreads;
+  constexpr int b = __builtin_ctz(rows);
+  __shared__ float4 X4[C * rows / 2];
+  const float2* X = reinterpret_cast<const float2*>(X4);
+  const uint64_t n_rows = 1ull << n_bits;
+  const uint64_t n_tiles = n_rows >> b;
+  const uint64_t bid = gblock<uint64_t>();
+  const uint32_t ng = (uint32_t)((n_rhs + C - 1) / C);
+  if (bid >= n_tiles * ng) return;              // whole workgroup: past the last tile
+  uint64_t tile;
+  uint32_t grp;
+  if (by_rhs) {                                 // ng a multiple of 8: a group of vectors per XCD
+    const uint64_t i = bid >> 3;
+    grp = (uint32_t)((bid & 7u) + 8u * (i >> (n_bits - b)));
+    tile = i & (n_tiles - 1);
+  } else {                                      // each XCD walks its own eighth of the tiles
+    grp = (uint32_t)(bid >> (n_bits - b));
+    tile = bid & (n_tiles - 1);
+    if (n_tiles >= 8) tile = (tile & 7u) * (n_tiles >> 3) + (tile >> 3);
+  }
+  uint64_t voff[C];                             // past the last vector: the last one again, not stored
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const uint32_t q = grp * C + j;
+    voff[j] = (uint64_t)(q < (uint32_t)n_rhs ? q : (uint32_t)n_rhs - 1) << n_bits;
+  }
+  const uint64_t base = tile << b;
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const float4* src = reinterpret_cast<const float4*>(tc + voff[j] + base);
+    for (uint32_t i = threadIdx.x; i < rows / 2; i += kThreads) X4[j * (rows / 2) + i] = src[i];
+  }
+  const uint32_t l = threadIdx.x;
+  const R r = (R)base | (R)l;
+  RowSum<kAccF64> sum[C];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t wbase = base | (uint64_t)(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6);
+  // parity of the wave's part of the row under mask m
+  auto wpar = [&](uint64_t m) -> uint32_t { return (uint32_t)__builtin_popcountll(wbase & m) & 1u; };
+  // entry of a one- or two-term group from its parities: +-(c0 + c1) where
+  // they agree, +-(c0 - c1) where they differ, the sign that of c0
+  auto uniform_entry = [&](const PauliGroup d) -> double {
+    const uint32_t p0 = wpar(d.m0), p1 = wpar(d.m1);
+    return flip_sign(p0 == p1 ? d.same : d.diff, p0 << 31);
+  };
+  auto needed = [&](const PauliGroup d) -> bool {
+    if (C == 1 || d.kind != QSIM_PAULI_GROUP_PAIR || ((d.m0 | d.m1) & 63u)) return true;
+    return nonzero(uniform_entry(d));
+  };
+  auto row_parity = [&](uint64_t m) -> uint32_t {
+    return (sizeof(R) == 4 ? (uint32_t)__popc((uint32_t)r & (uint32_t)m) : (uint32_t)__popcll((uint64_t)r & m)) << 31;
+  };
+  auto add_group = [&](const PauliGroup d, const float2 (&x)[C]) {
+    double v;
+    if (d.kind == QSIM_PAULI_GROUP_PAIR && C == 1) {
+      v = (double)(float)(flip_sign(d.c0, row_parity(d.m0)) + flip_sign(d.c1, row_parity(d.m1)));
+    } else if (d.kind == QSIM_PAULI_GROUP_PAIR && ((d.m0 | d.m1) & 63u)) {
+      const uint32_t p0 = (uint32_t)__popc(lane & (uint32_t)d.m0) + wpar(d.m0);
+      const uint32_t p1 = (uint32_t)__popc(lane & (uint32_t)d.m1) + wpar(d.m1);
+      v = flip_sign(((p0 ^ p1) & 1u) == 0 ? d.same : d.diff, p0 << 31);
+    } else if (d.kind == QSIM_PAULI_GROUP_TERMS) {
+      v = 0.0;
+#pragma unroll 4
+      for (uint32_t t = d.t0; t < d.t0 + d.nt; ++t) {
+        const uint64_t m = sm[t];
+        v += flip_sign(coef[t].x, (wpar(m) << 31) ^ ((uint32_t)__popc(lane & (uint32_t)m) << 31));
+      }
+      v = (double)(float)v;
+    } else {
+      v = d.kind == QSIM_PAULI_GROUP_PAIR ? uniform_entry(d) : d.same;
+    }
+    asm volatile("" : "+v"(v));                 // one vector value from here on, whatever the kind
+    if (v != 0.0) {
+#pragma unroll
+      for (int j = 0; j < C; ++j) sum[j].add_r(v, x[j]);
+    }
+  };
+  __syncthreads();
+  int g = 0;
+  for (; g < n_groups && tab[g].xm < rows; ++g) {
+    const PauliGroup d = tab[g];
+    if (!needed(d)) continue;
+    const uint32_t m = (uint32_t)d.xm;
+    float2 x[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) x[j] = X[j * rows + (l ^ m)];
+    add_group(d, x);
+  }
+  for (; g < n_groups; g += U) {
+    float2 x[U][C];
+    PauliGroup d[U];
+    bool need[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) d[u] = tab[g + u < n_groups ? g + u : n_groups - 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) need[u] = g + u < n_groups && needed(d[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (!need[u]) continue;
+      const R m = (R)d[u].xm & (R)(n_rows - 1);
+#pragma unroll
+      for (int j = 0; j < C; ++j) x[u][j] = (tc + voff[j])[r ^ m];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (need[u]) add_group(d[u], x[u]);
+  }
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    if (grp * C + j >= (uint32_t)n_rhs) continue;
+    const uint64_t at = voff[j] + r;
+    const float2 tp = first ? make_float2(0.f, 0.f) : ld2<NT>(tpn + at);
+    const float2 tn = sum[j].next(scale, tp, first != 0);
+    st2<NT>(tpn + at, tn);
+    const float2 v = cmulc(c, tn);
+    float2 a = ld2<NT>(acc + at), k2 = ld2<NT>(comp + at);
+    neu_add(a.x, k2.x, v.x);
+    neu_add(a.y, k2.y, v.y);
+    st2<NT>(acc + at, a);
+    st2<NT>(comp + at, k2);
+  }
+}
+
+template <typename R, int C, int U>
+static void launch_pauli(hipStream_t s, int n_groups, const void* groups, const void* sm, const void* coef, int n,
+                         int n_rhs, double scale, const void* tc, void* tpn, void* acc, void* comp, float2 c,
+                         int first) {
+  const uint64_t ng = ceil_div((uint64_t)n_rhs, C);
+  const uint64_t blocks = ng * ((1ull << n) / kThreads);
+  // T_k, T_{k-1} and the accumulator pair stream together: nontemporal once
+  // the four exceed the MALL (20 qubits, 32 right-hand sides: 622 against
+  // 659 us; 8, which fit: 171 against 155 us)
+  const bool nt = nt_for_bytes((32ull * n_rhs) << n);
+  // a group of vectors per XCD while its T_k (32 B a row) is a few L2s large:
+  // 16 qubits, 32 right-hand sides 38 against 44 us, 20 qubits 609 against
+  // 622; 22 qubits 2890 against 2733 us
+  const int by_rhs = ng % 8 == 0 && n <= 20;
+  auto* kern = nt ? k_cheb_pauli<R, C, U, true> : k_cheb_pauli<R, C, U, false>;
+  hipLaunchKernelGGL(kern, grid1d(blocks), dim3(kThreads), 0, s, n_groups, (const PauliGroup*)groups,
+                     (const uint64_t*)sm, (const double2*)coef, n, n_rhs, by_rhs, scale, (const float2*)tc,
+                     (float2*)tpn, (float2*)acc, (float2*)comp, c, first);
+}
+
 __global__ __launch_bounds__(kThreads) void k_cheb_init(float2* __restrict__ acc,
                                                         float2* __restrict__ comp,
                                                         const float2* __restrict__ t, int64_t n,
@@ -868,6 +1063,25 @@ int qsim_cheb_pauli_step(void* stream, int n_qubits, int n_groups, const void* x
                      (const float2*)t_cur,
                      (float2*)t_prev_next, (float2*)acc, (float2*)comp, f2(c_re, c_im), first);
   return launch_status("cheb_pauli_step");
+}
+
+int qsim_cheb_pauli_batch_step(void* stream, int n_qubits, int n_groups, const void* groups, const void* sm,
+                               const void* coef, int n_rhs, double scale, const void* t_cur, void* t_prev_next,
+                               void* acc, void* comp, double c_re, double c_im, int first) {
+  if (n_qubits < QSIM_PAULI_BATCH_MIN_QUBITS || n_qubits > QSIM_MAX_QUBITS)
+    return fail(QSIM_ERANGE, "n_qubits=%d outside %d..%d", n_qubits, QSIM_PAULI_BATCH_MIN_QUBITS, QSIM_MAX_QUBITS);
+  if (n_groups < 0 || n_rhs < 1 || n_rhs > (1 << 20))
+    return fail(QSIM_EINVAL, "bad sizes (n_groups=%d, n_rhs=%d)", n_groups, n_rhs);
+  if ((n_groups > 0 && (!groups || !sm || !coef)) || !t_cur || !t_prev_next || !acc || !comp)
+    return fail(QSIM_EINVAL, "NULL pointer argument");
+  if (((uintptr_t)t_cur & 15u) != 0) return fail(QSIM_EINVAL, "t_cur must be 16-byte aligned");
+  hipStream_t s = as_stream(stream);
+  const float2 c = f2(c_re, c_im);
+  const bool wide = n_qubits > 32, one = n_rhs == 1;
+  auto* launch = one ? (wide ? launch_pauli<uint64_t, 1, 2> : launch_pauli<uint32_t, 1, 2>)
+                     : (wide ? launch_pauli<uint64_t, 4, 1> : launch_pauli<uint32_t, 4, 1>);
+  launch(s, n_groups, groups, sm, coef, n_qubits, n_rhs, scale, t_cur, t_prev_next, acc, comp, c, first);
+  return launch_status("cheb_pauli_batch_step");
 }
 
 int qsim_cheb_init_acc(void* stream, void* acc, void* comp, const void* t, int64_t n, double c_re,

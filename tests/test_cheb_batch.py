@@ -1,0 +1,139 @@
+"""The tiled matrix-free Chebyshev term (qsim_cheb_pauli_batch_step) and its
+group records."""
+import os
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+for _p in (ROOT, os.path.join(ROOT, "qiskit-blackwell_amd")):
+    if _p not in sys.path:
+        sys.path.insert(0, _p)
+
+from blackwell_backend.hamiltonian import (HamiltonianCSR, PauliTables, SparsePauliOp, constant_group_entries,
+                                            pauli_groups, real_group_records)
+from blackwell_backend.chebyshev import chebyshev_evolve_batch
+from blackwell_kernels import _lib
+from blackwell_kernels._lib import ptr
+
+
+def mixed_terms(n, seed, real=True):
+    """Every kind of group: constant entries (X only), one and two terms on
+    near and far masks, a pair that cancels in half of the rows, three and
+    nine terms, a label given twice, and pairs whose masks stay above the
+    wave's bits."""
+    rng = np.random.default_rng(seed)
+
+    def lab(**ops):
+        s = ["I"] * n
+        for q, ch in ops.items():
+            s[n - 1 - int(q[1:])] = ch
+        return "".join(s)
+
+    q = lambda i: f"q{i}"
+    out = [(lab(**{q(i): "X"}), rng.uniform(-1, 1)) for i in range(n)]
+    out += [(lab(**{q(n - 1): "Z"}), 0.75), (lab(**{q(0): "Z", q(1): "Z"}), -0.3)]
+    for i in range(n - 1):
+        c = rng.uniform(-1, 1)
+        out += [(lab(**{q(i): "X", q(i + 1): "X"}), c), (lab(**{q(i): "Y", q(i + 1): "Y"}), c)]
+    for z in range(3, 6):                                   # three terms on a far mask
+        out.append((lab(**{q(0): "X", q(n - 1): "X", q(z): "Z"}), rng.uniform(-1, 1)))
+    for z in (0, 1, 3, 4, 5, 6, 7, 8, 0):                   # nine, one of them twice
+        out.append((lab(**{q(2): "X", q(z): "Z"}), rng.uniform(-1, 1)))
+    out.append((lab(**{q(3): "X", q(n - 2): "Z"}), 0.5))
+    out.append((lab(**{q(5): "X", q(6): "X", q(n - 1): "Z", q(n - 2): "Z"}), 0.25))
+    out.append(out[-1])
+    if not real:
+        out.append((lab(**{q(4): "Y"}), 0.5))
+    return out
+
+
+def test_group_records_give_the_entries():
+    """Per row of a 9-qubit Hamiltonian, the entry from the records is the
+    FP64 sum over the tables rounded to FP32; imaginary entries have none."""
+    n = 9
+    terms = mixed_terms(n, 1)
+    tables = lambda ts: pauli_groups([t[0] for t in ts], [t[1] for t in ts])
+    records = lambda xm, *tab: real_group_records(xm, *tab, constant_group_entries(*tab))
+    xm, toff, sm, coef = tables(terms)
+    recs = records(xm, toff, sm, coef)
+    rows = np.arange(1 << n, dtype=np.uint64)
+    par = lambda m: np.array([bin(int(r) & int(m)).count("1") & 1 for r in rows])
+    assert set(recs["kind"]) == {_lib.PAULI_CONST, _lib.PAULI_PAIR, _lib.PAULI_TERMS}
+    for g, rec in enumerate(recs):
+        want = np.zeros(1 << n)
+        for t in range(toff[g], toff[g + 1]):
+            want += np.where(par(sm[t]), -coef[t].real, coef[t].real)
+        want = want.astype(np.float32)
+        if rec["kind"] == _lib.PAULI_CONST:
+            got = np.full(1 << n, rec["same"])
+        elif rec["kind"] == _lib.PAULI_PAIR:
+            p0, p1 = par(rec["m"][0]), par(rec["m"][1])
+            got = np.where(p0, -1.0, 1.0) * np.where(p0 == p1, rec["same"], rec["diff"])
+            assert np.array_equal(np.where(p0, -rec["c"][0], rec["c"][0]) +
+                                  np.where(p1, -rec["c"][1], rec["c"][1]),
+                                  np.where(p0, -1.0, 1.0) * np.where(p0 == p1, rec["c"][0] + rec["c"][1],
+                                                                     rec["c"][0] - rec["c"][1]))
+        else:
+            assert (rec["t0"], rec["nt"]) == (toff[g], toff[g + 1] - toff[g])
+            continue
+        assert np.array_equal(got.astype(np.float32), want), g
+    bad = mixed_terms(n, 1, real=False)
+    assert records(*tables(bad)) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,R", [(9, 1), (9, 3), (10, 2), (11, 33), (14, 5), (17, 4), (18, 1), (16, 32)])
+def test_tiled_term_has_the_bits_of_the_untiled_one(n, R):
+    """One term, first and later, on R vectors: T_{k+1}, accumulator and
+    compensation are those of qsim_cheb_pauli_step on each vector alone."""
+    dev = torch.device("cuda", 0)
+    terms = mixed_terms(n, n)
+    pt = PauliTables([t[0] for t in terms], [t[1] for t in terms], dev)
+    assert pt.groups is not None
+    g = torch.Generator(device=dev).manual_seed(n * 100 + R)
+    new = lambda: torch.view_as_complex(torch.randn(R, 1 << n, 2, device=dev, generator=g))
+    T, prev, acc, comp = new(), new(), new(), new() * 1e-8
+    s = _lib.stream_handle(dev)
+    for first in (1, 0):
+        want, got = [[x.clone() for x in (prev, acc, comp)] for _ in range(2)]
+        for j in range(R):
+            _lib.call("qsim_cheb_pauli_step", s, n, *pt.step_args(), 0.21, ptr(T[j]), *(ptr(x[j]) for x in want),
+                      0.3, -0.2, first)
+        _lib.call("qsim_cheb_pauli_batch_step", s, n, *pt.batch_args(), R, 0.21, ptr(T), *(ptr(x) for x in got),
+                  0.3, -0.2, first)
+        for a, b in zip(want, got):
+            assert np.array_equal(torch.view_as_real(a).cpu().numpy(), torch.view_as_real(b).cpu().numpy()), first
+
+
+@pytest.mark.gpu
+def test_batch_evolution_by_tiles_equals_the_csr_terms():
+    """17 qubits, three states in a strided view: the default route reports
+    matrix-free terms and gives the CSR route's bits; the states are left as
+    they were; a Hamiltonian with imaginary entries stays on the CSR."""
+    dev = torch.device("cuda", 0)
+    n = 17
+    g = torch.Generator(device=dev).manual_seed(5)
+    X = torch.view_as_complex(torch.randn(6, 1 << n, 2, device=dev, generator=g))
+    X = (X / torch.linalg.vector_norm(X, dim=1, keepdim=True))[::2]
+    keep = X.clone()
+    h = HamiltonianCSR.from_sparse_pauli_op(SparsePauliOp.from_list(mixed_terms(n, 3)), device=dev)
+    a, ia = chebyshev_evolve_batch(X, h, 0.4, 1e-8)
+    b, ib = chebyshev_evolve_batch(X, h, 0.4, 1e-8, matrix_free=False)
+    assert ia["matrix_free"] and not ib["matrix_free"] and ia["chebyshev_degree"] == ib["chebyshev_degree"]
+    assert a.shape == b.shape and a.is_contiguous() and torch.equal(keep, X)
+    assert np.array_equal(a.cpu().numpy(), b.cpu().numpy())
+    h = HamiltonianCSR.from_sparse_pauli_op(SparsePauliOp.from_list(mixed_terms(n, 3, real=False)), device=dev)
+    _, ic = chebyshev_evolve_batch(X, h, 0.1, 1e-6)
+    assert not ic["matrix_free"]
+
+
+def test_tiled_term_checks_its_arguments():
+    lib = _lib.load()
+    z = (1.0, 16, 16, 16, 16, 0.0, 0.0, 0)
+    assert lib.qsim_cheb_pauli_batch_step(None, 8, 1, 16, 16, 16, 1, *z) == 2
+    assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, None, 16, 16, 1, *z) == 1
+    assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, 16, 16, 16, 0, *z) == 1
+    assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, 16, 16, 16, 1, 1.0, 24, 16, 16, 16, 0.0, 0.0, 0) == 1
