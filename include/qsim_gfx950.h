@@ -308,8 +308,9 @@ int qsim_sample_batch(void* stream, const qsim_sample_rec* recs_host, const void
  * a fixed order (deterministic), written as doubles to out_dev.            */
 int64_t qsim_expectation_workspace_bytes(int n_qubits);
 /* out_dev[k] = <psi|P_k|psi> for n_terms strings.  Terms with the same
- * x mask share one pass over the state (up to 8 per pass).  (new; the
- * reference evaluates one Z string or one X/Y qubit per call)            */
+ * x mask share their pair products (up to 8 at a time), and x masks that lie
+ * together in 13 qubits share one pass over the state.  (new; the
+ * reference evaluates one Z string or one X/Y qubit per call)              */
 int qsim_expectation_paulis(void* stream, const void* state, int n_qubits, int64_t n_terms,
                             const uint64_t* x_masks, const uint64_t* z_masks, void* workspace,
                             void* out_dev);

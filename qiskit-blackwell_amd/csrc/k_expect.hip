@@ -188,8 +188,243 @@ static void launch_expect_kind(hipStream_t s, const void* state, int n, uint64_t
   else launch_expect<NT, 2>(s, state, n, x, a, part, out);
 }
 
-// Workspace (doubles): pass-1 partials [kRedBlocks][kExpMaxTerms].
-constexpr int64_t kExpWsDoubles = (int64_t)kRedBlocks * kExpMaxTerms;
+// Tiled pass: many term groups per read of the state.  A workgroup copies a
+// tile of 2^M amplitudes (M qubits, among them the lowest 4, so that loads are
+// whole 128-byte lines) into LDS and evaluates there every group whose x mask
+// lies inside the tile's qubits.  x and the part of z inside the tile arrive
+// as tile-local masks; the rest of z gives one sign per tile.
+//
+// A unit of work is a group (up to 8 terms of one x mask and one Y parity)
+// and one of 2^seg equal parts of its index pairs.  A wave takes them 64 slots
+// (two amplitudes each) at a time: with i0 = the slots whose highest x bit is
+// clear, a slot index splits into a lane part and a wave part, so both LDS
+// addresses are a lane constant plus a wave constant, and the sign of a term
+// is a lane constant (applied once, to the unit's sum) times a wave sign,
+// taken from a bit mask over the unit's steps that one ballot computes.  Every
+// unit belongs to one wave, which adds its reduced sum to the unit's LDS slot
+// tile after tile; slots are added in order at the end, so sums are
+// deterministic as before.
+//
+// What bounds it: FP64 issue (14 of the 20 vector instructions per 64 slots of
+// a group of one term are FP64, at about 4.4 cycles each), then the tile loads,
+// which do not overlap it.  The 93 terms of a Heisenberg chain, plain passes
+// (two launches and a read of the state per group) -> tiled passes: 12 / 16 /
+// 20 / 24 / 28 qubits 151 / 245 / 302 / 1208 / 18600 -> 27 / 44 / 43 / 256 /
+// 4000 us.  Measured and not taken: the next tile loaded into registers during
+// the evaluation 4290 us, tiles of 2^12 at 256 threads 4556, 1024 threads 4675
+// (two parts a group; 512 threads there 4713).
+struct ExpGroup {
+  uint16_t x;                     // tile-local x mask
+  uint8_t h, im;                  // its highest bit; Im(zc) instead of Re(zc)
+  uint16_t t0, nt;                // terms [t0, t0 + nt), nt <= kExpMaxTerms
+  uint16_t zl[4];                 // tile-local z masks of the first four
+};
+struct ExpTerm {
+  uint64_t z;                     // z mask outside the tile
+  uint16_t zl;                    // tile-local z mask
+  int16_t fac;                    // +-1 (x = 0) or +-2
+  int32_t out;
+};
+constexpr int kPassGroups = 64, kPassTerms = 144, kPassBlocks = 512, kPassThreads = 512;
+constexpr int kPassWaves = kPassThreads / 64, kExpTileMax = 13, kExpTileMin = 10;
+// A pass of two groups already beats two plain passes: 24 qubits 30 against
+// 49 us, 28 qubits 340 against 635; a single group stays on the plain pass.
+constexpr int kPassMinGroups = 2;
+constexpr size_t kPassWindow = 2048;   // groups looked at per pass: planning stays linear in their number
+struct ExpPass {
+  uint32_t tq[4];                 // tile qubits, ascending, one byte each; the first four are 0..3
+  int n_groups, n_terms, seg;
+  ExpGroup g[kPassGroups];
+  ExpTerm t[kPassTerms];
+};
+static_assert(sizeof(ExpPass) <= 3584, "kernel arguments");
+__host__ __device__ inline int exp_tq(const ExpPass& a, int j) { return (int)((a.tq[j >> 2] >> (8 * (j & 3))) & 255u); }
+
+// Sums of a unit kept per term: the lanes are added over the lane bits whose
+// exchange is a DPP or permlane move (0, 1, 3, 5); bits 2 and 4, whose exchange
+// goes through the LDS unit, stay apart until the end.
+constexpr int kSlotLanes = 4;
+
+// Kinds of a group: x = 0; x = 1 (pairs inside a slot); x > 1 even; x > 1 odd.
+enum { kDiag, kInSlot, kPair, kPairSwap };
+
+// A unit's sums for its NT terms: steps of 64 slots from slot step p0 on.
+template <int NT, bool IM, int KIND>
+__device__ __forceinline__ void exp_unit(const char* Xb, const ExpPass& a, const ExpGroup g, uint32_t p0,
+                                         uint32_t steps, uint64_t base, uint32_t lane, double* slot) {
+  constexpr int U = 4;
+  constexpr bool pair = KIND >= kPair;
+  const int hs = (int)g.h - 1;
+  const uint32_t xs = g.x >> 1, lm = pair && hs < 6 ? 127u : 63u;
+  auto clear_h = [&](uint32_t p) -> uint32_t { return pair ? ins0(p, hs) : p; };
+  const uint32_t il = clear_h(lane);
+  const uint32_t la = il * 16, lb = (il ^ (xs & lm)) * 16, xw = xs & ~lm;
+  double acc[NT], c1[NT];
+  uint64_t neg[NT];                       // bit k: the wave sign of step k is -1
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const uint32_t z = j < 4 ? g.zl[j] : a.t[g.t0 + (j < g.nt ? j : 0)].zl;
+    acc[j] = 0.0;
+    c1[j] = (z & 1) ? -1.0 : 1.0;
+    neg[j] = __ballot(__popc(clear_h((p0 + lane) * 64) & (z >> 1)) & 1);
+  }
+  for (uint32_t k0 = 0; k0 < steps; k0 += U) {
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const uint32_t iw = clear_h((p0 + k0 + q) * 64);
+      const float4 u = *reinterpret_cast<const float4*>(Xb + (la + iw * 16));
+      double v0, v1 = 0.0;
+      auto prod = [](float2 x, float2 y) -> double {
+        return IM ? (double)x.x * y.y - (double)x.y * y.x : (double)x.x * y.x + (double)x.y * y.y;
+      };
+      if (KIND == kDiag) {
+        v0 = prod(lo2(u), lo2(u));
+        v1 = prod(hi2(u), hi2(u));
+      } else if (KIND == kInSlot) {
+        v0 = prod(lo2(u), hi2(u));
+      } else {
+        const float4 w = *reinterpret_cast<const float4*>(Xb + (lb + (iw ^ xw) * 16));
+        v0 = prod(lo2(u), KIND == kPairSwap ? hi2(w) : lo2(w));
+        v1 = prod(hi2(u), KIND == kPairSwap ? lo2(w) : hi2(w));
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const uint32_t m = (uint32_t)(neg[j] >> k0);
+        const double t = KIND == kInSlot ? v0 : __builtin_fma(c1[j], v1, v0);
+        acc[j] = __builtin_fma(__hiloint2double((m >> q & 1u) ? (int)0xbff00000 : 0x3ff00000, 0), t, acc[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    if (j >= g.nt) continue;
+    const ExpTerm t = a.t[g.t0 + j];
+    const int minus = (__popc(il & (uint32_t)(t.zl >> 1)) + __popcll(base & t.z)) & 1;
+    double r = acc[j] * (double)(minus ? -t.fac : t.fac);
+    r += lane_xor(r, 1);
+    r += lane_xor(r, 2);
+    r += lane_xor(r, 8);
+    r += lane_xor(r, 32);
+    if ((lane & 0x2b) == 0) slot[(j << a.seg) * kSlotLanes + (lane >> 4) * 2 + (lane >> 2 & 1)] += r;
+  }
+}
+
+template <int M, bool NTL>
+__global__ __launch_bounds__(kPassThreads) void k_expect_tile(ExpPass args, const float4* __restrict__ st,
+                                                              uint64_t n_tiles, double* __restrict__ part) {
+  // read in place by scalar loads: indexed through `args` itself, the compiler
+  // copied all of it to scratch (93 terms, 24 qubits: 783 against 272 us)
+  const ExpPass& a = *(const ExpPass*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ float4 X4[];
+  const char* Xb = reinterpret_cast<const char*>(X4);
+  double* slots = reinterpret_cast<double*>(X4 + (1 << (M - 1)));
+  constexpr int TB = __builtin_ctz(kPassThreads);
+  constexpr int SLOTS = (1 << (M - 1)) / kPassThreads;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int per_term = kSlotLanes << a.seg;
+  const uint32_t units = (uint32_t)a.n_groups << a.seg;
+  auto group = [&](uint32_t u) -> ExpGroup { return a.g[(u < units ? u : units - 1) >> a.seg]; };
+  for (int i = tid; i < a.n_terms * per_term; i += kPassThreads) slots[i] = 0.0;
+  uint64_t toff = 0;
+#pragma unroll
+  for (int j = 0; j < TB; ++j) toff |= (uint64_t)((tid >> j) & 1) << (exp_tq(a, j + 1) - 1);
+  for (uint64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    uint64_t base = tile;
+#pragma unroll
+    for (int j = 0; j < M; ++j) base = ins0(base, exp_tq(a, j));
+    float4 v[SLOTS];
+#pragma unroll
+    for (int k = 0; k < SLOTS; ++k) {
+      uint64_t off = base >> 1;
+#pragma unroll
+      for (int j = TB; j < M - 1; ++j) off |= (uint64_t)((k >> (j - TB)) & 1) << (exp_tq(a, j + 1) - 1);
+      v[k] = ld4<NTL>(st + (off + toff));
+    }
+    __syncthreads();              // the tile before has been read
+#pragma unroll
+    for (int k = 0; k < SLOTS; ++k) X4[k * kPassThreads + tid] = v[k];
+    __syncthreads();
+    ExpGroup next = group(wave);
+    for (uint32_t u = wave; u < units; u += kPassWaves) {
+      const ExpGroup g = next;
+      next = group(u + kPassWaves);
+      const uint32_t part_no = u & ((1u << a.seg) - 1u);
+      const uint32_t steps = (1u << (g.x > 1 ? M - 8 : M - 7)) >> a.seg;
+      double* slot = slots + (((uint32_t)g.t0 << a.seg) + part_no) * kSlotLanes;
+#define QSIM_UNIT(NT, IM, KIND) exp_unit<NT, IM, KIND>(Xb, a, g, part_no * steps, steps, base, lane, slot)
+#define QSIM_UNIT_NT(IM, KIND)                 \
+  do {                                         \
+    if (g.nt == 1) QSIM_UNIT(1, IM, KIND);     \
+    else if (g.nt == 2) QSIM_UNIT(2, IM, KIND); \
+    else QSIM_UNIT(8, IM, KIND);               \
+  } while (0)
+      if (g.x == 0) {
+        if (g.nt <= 4) QSIM_UNIT(4, false, kDiag);
+        else QSIM_UNIT(8, false, kDiag);
+      } else if (g.x == 1) {
+        if (g.im) QSIM_UNIT(8, true, kInSlot);
+        else QSIM_UNIT(8, false, kInSlot);
+      } else if (g.im) {
+        if (g.x & 1) QSIM_UNIT_NT(true, kPairSwap);
+        else QSIM_UNIT_NT(true, kPair);
+      } else {
+        if (g.x & 1) QSIM_UNIT_NT(false, kPairSwap);
+        else QSIM_UNIT_NT(false, kPair);
+      }
+#undef QSIM_UNIT_NT
+#undef QSIM_UNIT
+    }
+  }
+  __syncthreads();
+  for (int t = tid; t < a.n_terms; t += kPassThreads) {
+    double r = 0.0;
+    for (int i = 0; i < per_term; ++i) r += slots[t * per_term + i];
+    part[(uint64_t)t * gridDim.x + blockIdx.x] = r;
+  }
+}
+
+// One wave per term adds its nb partials in index order per lane, then the lanes.
+__global__ __launch_bounds__(64) void k_expect_tile_final(const double* __restrict__ part, int nb, ExpPass a,
+                                                          double* __restrict__ out) {
+  double r = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 64) r += part[(uint64_t)blockIdx.x * nb + b];
+  r = wsum64(r);
+  if (threadIdx.x == 0) out[a.t[blockIdx.x].out] = r;
+}
+
+template <int M>
+static void launch_expect_tile(hipStream_t s, const void* state, int n, const ExpPass& a, double* part, double* out) {
+  const uint64_t tiles = 1ull << (n - M);
+  const int blocks = (int)std::min<uint64_t>(tiles, kPassBlocks);
+  const size_t lds = (sizeof(float2) << M) + ((size_t)a.n_terms * kSlotLanes * sizeof(double) << a.seg);
+  auto* kern = nt_for_qubits(n) ? k_expect_tile<M, true> : k_expect_tile<M, false>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPassThreads), lds, s, a, (const float4*)state, tiles, part);
+  hipLaunchKernelGGL(k_expect_tile_final, dim3(a.n_terms), dim3(64), 0, s, part, blocks, a, out);
+}
+
+// Workspace (doubles): a plain pass's partials [kRedBlocks][kExpMaxTerms] or a
+// tiled pass's [kPassTerms][kPassBlocks].
+constexpr int64_t kExpWsDoubles =
+    std::max((int64_t)kRedBlocks * kExpMaxTerms, (int64_t)kPassTerms * kPassBlocks);
+
+// One group: terms order[beg, beg + cnt) with one x mask and Y parity.
+struct TermGroup {
+  uint64_t x;
+  int im, beg, cnt;
+  bool done;
+};
+
+static int pair_factor(uint64_t x, uint64_t z) {
+  return x == 0 ? 1 : ((__builtin_popcountll(x & z) >> 1) & 1) ? -2 : 2;
+}
+// The bits of v at the positions set in m, packed (v within m).
+static uint32_t pack_bits(uint64_t v, uint64_t m) {
+  uint32_t r = 0;
+  for (int j = 0; m; ++j, m &= m - 1)
+    if (v & m & (0 - m)) r |= 1u << j;
+  return r;
+}
 
 static int expectation_impl(hipStream_t s, const void* state, int n, int64_t n_terms,
                             const uint64_t* xm, const uint64_t* zm, double* ws, double* out) {
@@ -202,7 +437,7 @@ static int expectation_impl(hipStream_t s, const void* state, int n, int64_t n_t
     if (xm[k] >= lim || zm[k] >= lim)
       return fail(QSIM_EINVAL, "Pauli term %lld: mask has a qubit >= n_qubits (%d)", (long long)k, n);
   // terms sharing an x mask and the parity of their Y count (Re or Im of
-  // the pair products) share a state pass: visit them grouped, in input
+  // the pair products) share the pair products: visit them grouped, in input
   // order within a group
   std::vector<int64_t> order(n_terms);
   for (int64_t k = 0; k < n_terms; ++k) order[k] = k;
@@ -211,30 +446,81 @@ static int expectation_impl(hipStream_t s, const void* state, int n, int64_t n_t
   };
   std::stable_sort(order.begin(), order.end(),
                    [&key](int64_t a, int64_t b) { return key(a) < key(b); });
-  int rc = QSIM_OK;
-  for (int64_t g = 0; g < n_terms && rc == QSIM_OK;) {
+  std::vector<TermGroup> groups;
+  for (int64_t g = 0; g < n_terms;) {
     const auto k0 = key(order[g]);
-    const uint64_t x = k0.first;
-    int cnt = 0;
+    int cnt = 1;
+    while (g + cnt < n_terms && cnt < kExpMaxTerms && key(order[g + cnt]) == k0) ++cnt;
+    groups.push_back({k0.first, k0.second, (int)g, cnt, false});
+    g += cnt;
+  }
+  // Tiled passes: the first group not done opens a tile, and every later one
+  // whose x mask still fits joins.
+  const int m = n < kExpTileMin ? 0 : n < kExpTileMax ? n : kExpTileMax;
+  for (size_t first = 0; m && first < groups.size(); ++first) {
+    if (groups[first].done || __builtin_popcountll(groups[first].x | 15) > m) continue;
+    uint64_t tile = 15;
+    std::vector<size_t> in;
+    int terms = 0;
+    const size_t last = std::min(groups.size(), first + kPassWindow);
+    for (size_t i = first; i < last && in.size() < (size_t)kPassGroups; ++i) {
+      const TermGroup& g = groups[i];
+      if (g.done || __builtin_popcountll(tile | g.x) > m || terms + g.cnt > kPassTerms) continue;
+      tile |= g.x;
+      terms += g.cnt;
+      in.push_back(i);
+    }
+    if (in.size() < (size_t)kPassMinGroups) continue;
+    for (int q = 0; __builtin_popcountll(tile) < m; ++q) tile |= 1ull << q;
+    ExpPass a = {};
+    uint64_t rest = tile;
+    for (int j = 0; j < m; ++j, rest &= rest - 1) a.tq[j >> 2] |= (uint32_t)__builtin_ctzll(rest) << (8 * (j & 3));
+    a.n_groups = (int)in.size();
+    a.n_terms = terms;
+    // the fewest parts that give each wave a unit (28 qubits, 93 terms: 3.99 ms
+    // with one part, 4.59 with two, 4.90 with four; 2 groups: 355 us with two
+    // parts, 340 with four), and at least 4 steps a unit
+    a.seg = std::min(a.n_groups >= kPassWaves ? 0 : a.n_groups >= kPassWaves / 2 ? 1 : 2, m - 10);
+    int t = 0;
+    for (size_t i = 0; i < in.size(); ++i) {
+      TermGroup& g = groups[in[i]];
+      const uint32_t x = pack_bits(g.x, tile);
+      a.g[i] = {(uint16_t)x, (uint8_t)(x ? 31 - __builtin_clz(x) : 0), (uint8_t)g.im, (uint16_t)t, (uint16_t)g.cnt, {}};
+      for (int j = 0; j < g.cnt; ++j, ++t) {
+        const int64_t k = order[g.beg + j];
+        a.t[t] = {zm[k] & ~tile, (uint16_t)pack_bits(zm[k] & tile, tile), (int16_t)pair_factor(g.x, zm[k]), (int32_t)k};
+        if (j < 4) a.g[i].zl[j] = a.t[t].zl;
+      }
+      g.done = true;
+    }
+    switch (m) {
+      case 10: launch_expect_tile<10>(s, state, n, a, ws, out); break;
+      case 11: launch_expect_tile<11>(s, state, n, a, ws, out); break;
+      case 12: launch_expect_tile<12>(s, state, n, a, ws, out); break;
+      default: launch_expect_tile<13>(s, state, n, a, ws, out); break;
+    }
+    if (int rc = launch_status("expectation")) return rc;
+  }
+  for (const TermGroup& g : groups) {
+    if (g.done) continue;
+    const uint64_t x = g.x;
+    const int cnt = g.cnt;
     ExpTerms a = {};
-    a.im = k0.second;
-    while (g + cnt < n_terms && cnt < kExpMaxTerms && key(order[g + cnt]) == k0) {
-      const int64_t k = order[g + cnt];
-      const int y = __builtin_popcountll(x & zm[k]);
-      a.z[cnt] = zm[k];
-      a.out[cnt] = (int)k;
-      a.fac[cnt] = x == 0 ? 1.0 : (((y >> 1) & 1) ? -2.0 : 2.0);
-      ++cnt;
+    a.im = g.im;
+    for (int j = 0; j < cnt; ++j) {
+      const int64_t k = order[g.beg + j];
+      a.z[j] = zm[k];
+      a.out[j] = (int)k;
+      a.fac[j] = pair_factor(x, zm[k]);
     }
     for (int j = cnt; j < kExpMaxTerms; ++j) { a.out[j] = -1; a.fac[j] = 0.0; }
     if (cnt == 1) launch_expect_kind<1>(s, state, n, x, a, ws, out);
     else if (cnt == 2) launch_expect_kind<2>(s, state, n, x, a, ws, out);
     else if (cnt <= 4) launch_expect_kind<4>(s, state, n, x, a, ws, out);
     else launch_expect_kind<8>(s, state, n, x, a, ws, out);
-    rc = launch_status("expectation");
-    g += cnt;
+    if (int rc = launch_status("expectation")) return rc;
   }
-  return rc;
+  return QSIM_OK;
 }
 
 // ------------------------------------------------------------ apply P
