@@ -187,6 +187,7 @@ class CompiledCircuit:
         self._blocks = None
         self._tiles = None
         self._auto = None
+        self._arrays = None
         self._graphs = {}
         self._tuned = {}
         self.has_stochastic = any(o.kind in ("measure", "reset") for o in ops)
@@ -272,13 +273,13 @@ class CompiledCircuit:
                 best, best_ms = mode, ms
         return best
 
-    def block_entries(self, k=5):
+    def block_entries(self, k=5, arrays=None):
         """plan_blocks of the ops with k-qubit blocks (computed once per
         compiled circuit and width)."""
         if self._blocks is None:
             self._blocks = {}
         if k not in self._blocks:
-            self._blocks[k] = C.plan_blocks(self.ops, self.n_qubits, k=k)
+            self._blocks[k] = C.plan_blocks(self.ops, self.n_qubits, k=k, arrays=arrays)
         return self._blocks[k]
 
     # ---------------------------------------------------------------- plans
@@ -313,10 +314,13 @@ class CompiledCircuit:
         if mode != "auto":
             return mode
         if self._auto is None:
-            self._auto = self._auto_mode()
+            arrays = []
+            self._auto = self._auto_mode(arrays)
+            # the plan that follows takes the decision's arrays over
+            self._arrays = arrays if self._auto == "passes" else None
         return self._auto
 
-    def _auto_mode(self):
+    def _auto_mode(self, arrays):
         n = self.n_qubits
         if n < BLOCK_MIN_QUBITS:
             return "whole"
@@ -328,10 +332,10 @@ class CompiledCircuit:
             w_ops = sum(TILE_OP_WEIGHT.get(o.kind, 1.0) for o in self.ops)
             t_tiles = (passes * TILE_PASS_US + w_ops * TILE_OP_US_16Q * 1.13 ** (n - 16)
                        + others * BLOCK_US_16Q)
-            t_blocks = len(self.block_entries()) * BLOCK_US_16Q * 1.07 ** (n - 16)
+            t_blocks = len(self.block_entries(arrays=arrays)) * BLOCK_US_16Q * 1.07 ** (n - 16)
             return "tiles" if t_tiles < t_blocks else "passes"
         t_whole = len(self.ops) * WHOLE_OP_US_12Q * 2.0 ** (n - 12)
-        t_blocks = len(self.block_entries()) * BLOCK_US
+        t_blocks = len(self.block_entries(arrays=arrays)) * BLOCK_US
         return "passes" if t_blocks < t_whole else "whole"
 
     def _build(self, mode, device):
@@ -357,7 +361,8 @@ class CompiledCircuit:
         if mode == "passes":
             if n < C.PASS_MIN_QUBITS:
                 raise ValueError(f"block passes need n >= {C.PASS_MIN_QUBITS} (n = {n})")
-            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n)), device)
+            arrays, self._arrays = self._arrays, None
+            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n), arrays=arrays), device)
         if mode == "blocks":
             if n < 10:
                 return self._build_tiles(C.plan_tiles(self.ops, n, m=n), device)
