@@ -234,6 +234,27 @@ int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const
 int qsim_apply_passes(void* stream, void* state, int n_qubits, const qsim_pass* passes, int n_passes,
                       const qsim_pass_block* blocks_host, const void* blocks_dev,
                       const void* frags_dev, int n_blocks);
+/* One state's pass in a batched step: device address of a complex64 state of
+ * n_qubits, its tile of tile_bits qubits (ascending in tile_qubits, the first
+ * 0), its n_blocks block records from first_block on, and the prefix sum of
+ * 2^(n_qubits - tile_bits) over the records before it.                     */
+typedef struct qsim_pass_rec {
+  uint64_t state;
+  uint64_t tile_begin;
+  int32_t  n_qubits;
+  int32_t  tile_bits;
+  int32_t  first_block;
+  int32_t  n_blocks;
+  uint8_t  tile_qubits[16];
+} qsim_pass_rec;
+/* One pass of each of n_recs states in one launch, with the bits of
+ * qsim_apply_passes on each state alone.  recs_host and blocks_host are
+ * validated and must hold the bytes of recs_dev and blocks_dev; blocks and
+ * frags are the states' planner outputs one after another.  The states of one
+ * call must not overlap.  (new; the serving HBM lane)                      */
+int qsim_apply_pass_batch(void* stream, const qsim_pass_rec* recs_host, const void* recs_dev,
+                          int64_t n_recs, const qsim_pass_block* blocks_host, const void* blocks_dev,
+                          const void* frags_dev, int64_t n_blocks);
 
 /* ---- reductions, measurement, sampling ---------------------------------- */
 /* Size in bytes of the workspace the reduction entry points need for a

@@ -8,11 +8,15 @@ concurrently on separate HIP streams:
   * LDS lane (n <= 14): many circuits per launch of qsim_run_instances, one
     workgroup per circuit with its whole state in LDS, its own gate table,
     and in-kernel sampling.  Nothing but the samples touches HBM.
-  * HBM lane (n > 14): each circuit in its own slab of HBM, run as fused
-    5-qubit blocks on FP32 MFMA (one qsim_apply_blocks call per circuit),
-    then sampled with qsim_sample.  Block plans are built ahead of time on a
-    pool of host threads (the native planner releases the GIL), so planning
-    overlaps the device work of the circuits before it.
+  * HBM lane (n > 14): each circuit in its own slab of HBM, run as block
+    passes (qsim_apply_passes; circuits admitted together take their passes
+    step by step in one qsim_apply_pass_batch launch each), then sampled.
+    Pass plans are built ahead of time on a pool of host threads (the native
+    planner releases the GIL), so planning overlaps the device work of the
+    circuits before it.  Against 5-qubit block steps, one launch per block:
+    48 circuits of 10 to 18 qubits 4.18 -> 3.03 ms, the lane's part on the
+    device 2.0 -> 0.65 ms (81 launches of 7.5 us, 5 us apart -> 21 of 11 us),
+    and a plan takes a quarter of the host time.
 
 Admission is by statevector bytes against an HBM budget (default 80 % of
 the free device memory; tests inject a small one).  A request that arrives
@@ -24,10 +28,10 @@ running batches and the HBM lane.
 Repeated circuits on the HBM lane replay as HIP graphs: a request that
 carries a circuit (no gate payload) and whose compiled circuit the server
 has already run once is executed by replaying a captured graph of state
-init + its block plan (one host call instead of one launch per block), into
+init + its pass plan (one host call instead of one launch per pass), into
 the graph's own buffer, which is sampled before the next replay on the
 same stream.  Gate-payload requests are unique by construction and run as
-batched block steps instead.
+batched pass steps instead.
 
 Sampling in both lanes uses the same rule and the same uniforms for a given
 seed: u_k = SplitMix64(seed + (k+1) * golden) >> 11 scaled by 2^-53 and
@@ -48,18 +52,19 @@ import numpy as np
 import torch
 
 from blackwell_kernels import _lib
-from blackwell_kernels._lib import call, BLOCK_REC_DTYPE, OP_DTYPE, INSTANCE_DTYPE, SAMPLE_REC_DTYPE
+from blackwell_kernels._lib import call, PASS_REC_DTYPE, OP_DTYPE, INSTANCE_DTYPE, SAMPLE_REC_DTYPE
 from . import compiler as C
 from .circuit import instructions
-from .executor import CompiledCircuit, tile_ops
+from .executor import CompiledCircuit, pass_shape, tile_ops
 from . import workloads as W
 
 LDS_MAX_QUBITS = 14
 # HBM-lane states up to this size are sampled together (qsim_sample_batch)
 SAMPLE_BATCH_MAX_QUBITS = 20
 # state bytes per HBM-lane batch: the 256 MB MALL (Infinity Cache) of MI355X,
-# which keeps a batch's states resident between its block steps
+# which keeps a batch's states resident between its steps
 HBM_BATCH_BYTES = 1 << 28
+FRAG_BYTES = 2 * _lib.PASS_BLOCK_BF16
 GOLDEN = 0x9E3779B97F4A7C15
 
 
@@ -276,7 +281,7 @@ class _LdsBatch:
 
 # ---------------------------------------------------------------- HBM lane
 class _PinnedPool:
-    """Reusable pinned host buffers for the block-matrix uploads: a buffer
+    """Reusable pinned host buffers for the plan uploads: a buffer
     goes back to the pool when the job that used it has finished on the
     device, so no page-locking happens on the launch path."""
 
@@ -306,10 +311,10 @@ class _HbmJob:
         self.staging = None
         self.event = None
         self.prepared = None      # future of prepare() when planned ahead
-        self.blocks = None        # (block qubits int32 [B, 8], matrices complex64 [B, 32, 32])
+        self.plan = None          # PassRun of a gate payload
 
     def prepare(self):
-        """Host-only block planning for gate-payload requests (thread safe,
+        """Host-only pass planning for gate-payload requests (thread safe,
         touches no device state)."""
         r = self.req
         if r.gates is not None:
@@ -317,9 +322,9 @@ class _HbmJob:
             g = len(pairs)
             qb = np.full((g, 8), -1, dtype=np.int32)
             qb[:, :2] = pairs
-            refs, bqs, bm = C.plan_blocks_arrays(r.n_qubits, np.full(g, 2, np.int32), qb, us, k=5)
-            assert (refs >= 0).all()          # two-qubit gates always fit a 5-qubit block
-            self.blocks = (np.ascontiguousarray(bqs), np.ascontiguousarray(bm, dtype=np.complex64))
+            refs, *plan = C.plan_passes_arrays(r.n_qubits, np.full(g, 2, np.int32), qb, us, *pass_shape(r.n_qubits))
+            assert (refs >= 0).all()          # two-qubit gates always fit a block
+            self.plan = C.PassRun(*plan)
         return self
 
     def launch(self):
@@ -331,18 +336,21 @@ class _HbmJob:
             self.prepare()
         sh = ctypes.c_void_p(self.stream.cuda_stream)
         with torch.cuda.stream(self.stream):
-            if self.blocks is not None:
+            if self.plan is not None:
                 self.state = torch.empty(1 << r.n_qubits, dtype=torch.complex64, device=dev)
                 call("qsim_state_init", sh, ctypes.c_void_p(self.state.data_ptr()), r.n_qubits)
-                bqs, bm = self.blocks
-                raw = bm.view(np.uint8).reshape(-1)
-                self.staging = self.pool.acquire(raw.size)
-                self.staging[:raw.size].numpy()[:] = raw
-                self.d_mats = torch.empty(raw.size, dtype=torch.uint8, device=dev)
-                self.d_mats.copy_(self.staging[:raw.size], non_blocking=True)
-                call("qsim_apply_blocks", sh, ctypes.c_void_p(self.state.data_ptr()), r.n_qubits,
-                     ctypes.c_void_p(self.d_mats.data_ptr()), ctypes.c_void_p(bqs.ctypes.data),
-                     len(bqs))
+                p = self.plan
+                total = p.blocks.nbytes + p.frags.nbytes
+                self.staging = self.pool.acquire(total)
+                host = self.staging.numpy()
+                host[:p.blocks.nbytes] = p.blocks.view(np.uint8).reshape(-1)
+                host[p.blocks.nbytes:total] = p.frags.view(np.uint8).reshape(-1)
+                self.d_buf = torch.empty(max(total, 1), dtype=torch.uint8, device=dev)
+                self.d_buf[:total].copy_(self.staging[:total], non_blocking=True)
+                at = self.d_buf.data_ptr()
+                call("qsim_apply_passes", sh, ctypes.c_void_p(self.state.data_ptr()), r.n_qubits,
+                     ctypes.c_void_p(p.passes.ctypes.data), len(p.passes), ctypes.c_void_p(p.blocks.ctypes.data),
+                     ctypes.c_void_p(at), ctypes.c_void_p(at + p.blocks.nbytes), len(p.blocks))
             else:
                 cc = self.sim.compile(_circuit_of(r))
                 g = self.graphs.get(cc, dev) if self.graphs is not None else None
@@ -352,7 +360,7 @@ class _HbmJob:
                 else:
                     self.state = torch.empty(1 << r.n_qubits, dtype=torch.complex64, device=dev)
                     cc.init_state(self.state)
-                    cc.plan(cc.resolve_mode("blocks"), dev).run(self.state)
+                    cc.plan(cc.resolve_mode("passes"), dev).run(self.state)
             from blackwell_kernels import sample_with_uniforms, uniforms_splitmix
             u = uniforms_splitmix(r.seed, r.shots, dev)
             self.d_out = sample_with_uniforms(self.state, u)
@@ -375,18 +383,18 @@ class _HbmJob:
             self.req.state = self.h_state.numpy().copy()
             self.h_state = None
         self.req.t_done = now
-        self.state = self.d_mats = None
+        self.state = self.d_buf = None
         self.pool.release(self.staging)
         self.staging = None
 
 
 class _HbmBatch:
-    """HBM-lane requests with gate payloads, run together: their block plans
-    execute as batched block steps (one qsim_apply_block_batch launch per
-    step applies block s of every request that has one), then each state is
-    sampled with its own seeded device uniforms.  Block matrices and step
-    records go to the device in one pinned copy.  Each request's arithmetic
-    is that of qsim_apply_blocks, so its samples do not depend on the batch."""
+    """HBM-lane requests with gate payloads, run together: their block passes
+    execute as batched steps (one qsim_apply_pass_batch launch per step applies
+    pass s of every request that has one), then each state is sampled with its
+    own seeded device uniforms.  Block records, fragments and step records go
+    to the device in one pinned copy.  Each request's arithmetic is that of
+    qsim_apply_passes, so its samples do not depend on the batch."""
 
     def __init__(self, jobs, stream, pool):
         self.jobs = jobs
@@ -398,7 +406,7 @@ class _HbmBatch:
 
     def launch(self):
         from blackwell_kernels import sample_with_uniforms, uniforms_splitmix
-        from blackwell_kernels.cuquantum import (block_step_records, run_block_steps, run_sample_batch,
+        from blackwell_kernels.cuquantum import (pass_step_records, run_pass_steps, run_sample_batch,
                                                  sample_records)
         for j in self.jobs:
             if j.prepared is not None:
@@ -408,12 +416,13 @@ class _HbmBatch:
         dev = self.jobs[0].sim.device
         sh = ctypes.c_void_p(self.stream.cuda_stream)
         ns = [r.n_qubits for r in self.reqs]
-        mats = [j.blocks[1] for j in self.jobs]
-        moff = np.concatenate([[0], np.cumsum([m.nbytes for m in mats])]).astype(np.int64)
-        n_rec = sum(len(m) for m in mats)
+        plans = [j.plan for j in self.jobs]
+        blocks = np.concatenate([p.blocks for p in plans])
+        first = np.cumsum([0] + [len(p.blocks) for p in plans])
+        rec_at = blocks.nbytes + len(blocks) * FRAG_BYTES
+        n_rec = sum(len(p.passes) for p in plans)
         small = [i for i, n in enumerate(ns) if n <= SAMPLE_BATCH_MAX_QUBITS]
-        rec_at = int(moff[-1])
-        srec_at = rec_at + n_rec * BLOCK_REC_DTYPE.itemsize
+        srec_at = rec_at + n_rec * PASS_REC_DTYPE.itemsize
         total = srec_at + len(small) * SAMPLE_REC_DTYPE.itemsize
         with torch.cuda.stream(self.stream):
             soff = np.concatenate([[0], np.cumsum([1 << n for n in ns])]).astype(np.int64)
@@ -422,24 +431,32 @@ class _HbmBatch:
             self.d_buf = torch.empty(max(total, 1), dtype=torch.uint8, device=dev)
             self.d_out = torch.empty(max(int(shot_off[-1]), 1), dtype=torch.int64, device=dev)
             base, obase = self.slab.data_ptr(), self.d_out.data_ptr()
-            recs, off = block_step_records([base + 8 * int(o) for o in soff[:-1]], ns,
-                                           [self.d_buf.data_ptr() + int(o) for o in moff[:-1]],
-                                           [j.blocks[0] for j in self.jobs])
+            recs, off = pass_step_records([base + 8 * int(o) for o in soff[:-1]], ns, [p.passes for p in plans],
+                                          first[:-1])
             srecs, leaves = sample_records([base + 8 * int(soff[i]) for i in small], [ns[i] for i in small],
                                            [obase + 8 * int(shot_off[i]) for i in small],
                                            [self.reqs[i].seed for i in small],
                                            [self.reqs[i].shots for i in small])
             self.staging = self.pool.acquire(total)
             host = self.staging.numpy()
-            for m, o in zip(mats, moff[:-1]):
-                host[int(o):int(o) + m.nbytes] = m.view(np.uint8).reshape(-1)
+            host[:blocks.nbytes] = blocks.view(np.uint8).reshape(-1)
+            for p, f in zip(plans, first):
+                at = blocks.nbytes + int(f) * FRAG_BYTES
+                host[at:at + p.frags.nbytes] = p.frags.view(np.uint8).reshape(-1)
             host[rec_at:srec_at] = recs.view(np.uint8)
             host[srec_at:total] = srecs.view(np.uint8)
             self.d_buf[:total].copy_(self.staging[:total], non_blocking=True)
-            self.recs, self.srecs = recs, srecs     # validated host copies of the records
+            self.recs, self.srecs, self.blocks = recs, srecs, blocks     # validated host copies
             for n, o in zip(ns, soff[:-1]):
                 call("qsim_state_init", sh, ctypes.c_void_p(base + 8 * int(o)), n)
-            run_block_steps(sh, recs, self.d_buf[rec_at:], off)
+            dbuf = self.d_buf.data_ptr()
+            if len(self.jobs) == 1:       # kernels chosen for the one size, and nontemporal access for large states
+                p = plans[0]
+                call("qsim_apply_passes", sh, ctypes.c_void_p(base), ns[0], ctypes.c_void_p(p.passes.ctypes.data),
+                     len(p.passes), ctypes.c_void_p(blocks.ctypes.data), ctypes.c_void_p(dbuf),
+                     ctypes.c_void_p(dbuf + blocks.nbytes), len(blocks))
+            else:
+                run_pass_steps(sh, recs, dbuf + rec_at, off, blocks, dbuf, dbuf + blocks.nbytes)
             if small:
                 run_sample_batch(sh, srecs, self.d_buf[srec_at:], leaves, dev)
             for i, r in enumerate(self.reqs):
@@ -505,7 +522,7 @@ class _GraphCache:
         if g is None:
             if self.seen[cc] < 2:
                 return None
-            mode = cc.resolve_mode("blocks")
+            mode = cc.resolve_mode("passes")
             g = cc.graphed(mode, device)
             if g is None:
                 return None
@@ -535,9 +552,9 @@ class Server:
     max_hbm_batch    most HBM-lane circuits per batch
     max_hbm_batch_bytes  most state bytes per HBM-lane batch (a larger
                      circuit runs alone); the default is the 256 MB MALL of
-                     MI355X, so a batch stays cache-resident across its block
+                     MI355X, so a batch stays cache-resident across its
                      steps
-    planner_threads  host threads that build HBM-lane block plans ahead
+    planner_threads  host threads that build HBM-lane pass plans ahead
     plan_ahead       most queued HBM-lane circuits planned ahead of admission
     graph_repeats    replay repeated HBM-lane circuits as HIP graphs (at most
                      this many graphs kept; 0 turns it off)

@@ -55,6 +55,7 @@ PROTOTYPES = {
     "qsim_apply_blocks": (_i, [_vp, _vp, _i, _vp, _vp, _i]),
     "qsim_plan_passes": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _pint, _pint]),
     "qsim_apply_passes": (_i, [_vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _i]),
+    "qsim_apply_pass_batch": (_i, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64]),
     "qsim_apply_block_batch": (_i, [_vp, _vp, _vp, _i64]),
     "qsim_reduce_workspace_bytes": (_i64, [_i]),
     "qsim_norm2": (_i, [_vp, _vp, _i, _vp, _vp]),
@@ -113,6 +114,9 @@ SAMPLE_REC_DTYPE = np.dtype([("state", "<u8"), ("out", "<u8"), ("seed", "<u8"), 
 PASS_DTYPE = np.dtype([("tile_mask", "<u8"), ("first_block", "<i4"), ("n_blocks", "<i4")])
 PASS_BLOCK_DTYPE = np.dtype([("bit", "<u2", (16,))])
 PASS_BLOCK_BF16 = 3072
+PASS_REC_DTYPE = np.dtype([("state", "<u8"), ("tile_begin", "<u8"), ("n_qubits", "<i4"), ("tile_bits", "<i4"),
+                           ("first_block", "<i4"), ("n_blocks", "<i4"), ("tile_qubits", "u1", (16,))])
+assert PASS_REC_DTYPE.itemsize == 48
 # qsim_pauli_group and its kinds
 PAULI_GROUP_DTYPE = np.dtype([("xm", "<u8"), ("t0", "<u4"), ("nt", "<u2"), ("kind", "<u2"), ("same", "<f8"),
                               ("diff", "<f8"), ("c", "<f8", (2,)), ("m", "<u8", (2,))])

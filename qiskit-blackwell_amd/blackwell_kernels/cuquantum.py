@@ -280,6 +280,48 @@ def apply_blocks_batched(states, mats, qubits):
     return states
 
 
+def pass_step_records(state_ptrs, n_qubits, passes, first_blocks):
+    """Records of batched block passes (numpy PASS_REC_DTYPE) and the offsets
+    of each step in them.  state_ptrs[i] / n_qubits[i]: instance i's state;
+    passes[i]: its PASS_DTYPE passes; first_blocks[i]: where its block records
+    begin in the batch's.  Step s holds pass s of every instance that has one,
+    in instance order."""
+    counts = np.array([len(p) for p in passes], dtype=np.int64)
+    steps = int(counts.max()) if counts.size else 0
+    cat = np.concatenate(passes) if counts.size else np.zeros(0, _lib.PASS_DTYPE)
+    inst = np.repeat(np.arange(counts.size), counts)
+    step = np.arange(cat.size) - np.repeat(np.cumsum(counts) - counts, counts)
+    order = np.lexsort((inst, step))             # by step, then instance
+    cat, inst, step = cat[order], inst[order], step[order]
+    nq = np.asarray(n_qubits, dtype=np.int64)[inst] if inst.size else np.zeros(0, np.int64)
+    row, bit = np.nonzero((cat["tile_mask"][:, None] >> np.arange(64, dtype=np.uint64)) & np.uint64(1))
+    bits = np.bincount(row, minlength=cat.size)
+    recs = np.zeros(cat.size, dtype=_lib.PASS_REC_DTYPE)
+    recs["state"] = np.asarray(state_ptrs, dtype=np.uint64)[inst] if inst.size else 0
+    recs["n_qubits"], recs["tile_bits"] = nq, bits
+    recs["first_block"] = cat["first_block"] + np.asarray(first_blocks, dtype=np.int64)[inst] if inst.size else 0
+    recs["n_blocks"] = cat["n_blocks"]
+    recs["tile_qubits"][row, np.arange(row.size) - np.repeat(np.cumsum(bits) - bits, bits)] = bit
+    off = np.zeros(steps + 1, dtype=np.int64)
+    off[1:] = np.cumsum(np.bincount(step, minlength=steps))
+    tiles = np.left_shift(np.int64(1), nq - bits)
+    csum = np.cumsum(tiles) - tiles              # exclusive prefix over all records
+    recs["tile_begin"] = csum - csum[off[step]] if inst.size else 0
+    return recs, off
+
+
+def run_pass_steps(stream, recs, recs_dev, off, blocks, blocks_dev, frags_dev):
+    """One qsim_apply_pass_batch launch per step.  recs, blocks: host records;
+    recs_dev, blocks_dev, frags_dev: device addresses of the same bytes and of
+    the blocks' fragments."""
+    vp = _lib.ctypes.c_void_p
+    size = _lib.PASS_REC_DTYPE.itemsize
+    for s in range(len(off) - 1):
+        a, b = int(off[s]), int(off[s + 1])
+        call("qsim_apply_pass_batch", stream, vp(recs.ctypes.data + a * size), vp(recs_dev + a * size), b - a,
+             vp(blocks.ctypes.data), vp(blocks_dev), vp(frags_dev), len(blocks))
+
+
 def _tile_mask(n, must, bits=None):
     """Tile mask holding `must` plus the lowest other qubits (qubit 0 always)."""
     bits = min(n, bits or 10)

@@ -56,6 +56,8 @@
 
 namespace qsim {
 
+static_assert(sizeof(qsim_pass_rec) == 48, "batch pass record");
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -103,10 +105,11 @@ __device__ __forceinline__ f32x16 mul_parts(const bf16x8 a[kFrags], const bf16x8
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2 * KA + 1], b[2 * KB + 1], acc, 0, 0, 0);
 }
 
+// One tile of one pass, by a workgroup of W waves.
 template <int M, int W, bool NT>
-__global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uint64_t n_tiles, PassGeom g,
-                                                    const uint4* __restrict__ blocks,
-                                                    const float4* __restrict__ frags, int n_blocks) {
+__device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile, const PassGeom& g,
+                                          const uint4* __restrict__ blocks, const float4* __restrict__ frags,
+                                          int n_blocks) {
   constexpr int T = 64 * W;
   constexpr int SLOTS = (1 << (M - 1)) / T;           // float4 slots per thread
   constexpr int TB = __builtin_ctz(T);                // slot bits that run over the threads
@@ -117,8 +120,7 @@ __global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uin
   const int tid = threadIdx.x;
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint64_t base = gblock<uint64_t>();
-  if (base >= n_tiles) return;                        // whole workgroup: past the last tile
+  uint64_t base = tile;
 #pragma unroll
   for (int j = 0; j < M; ++j) base = ins0(base, g.tq(j));
   base >>= 1;                                         // in slots; the first tile qubit is 0
@@ -214,6 +216,51 @@ __global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uin
   }
 }
 
+template <int M, int W, bool NT>
+__global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uint64_t n_tiles, PassGeom g,
+                                                    const uint4* __restrict__ blocks,
+                                                    const float4* __restrict__ frags, int n_blocks) {
+  const uint64_t tile = gblock<uint64_t>();
+  if (tile >= n_tiles) return;                        // whole workgroup: past the last tile
+  pass_tile<M, W, NT>(st, tile, g, blocks, frags, n_blocks);
+}
+
+// One pass of each of n_recs states in one launch: workgroup b takes the tile
+// b - tile_begin of the record it falls to, found by one load per lane and a
+// ballot (records ascend; more than 64 take further rounds).  pass_tile does
+// not depend on W or on the tile's place in the grid, so a state's bits are
+// those of its passes run alone.  What bounds it is the latency of a pass, a
+// tile or less per CU: a step of 6 states of 15 to 17 qubits takes 13 us, and
+// replaces three to four launches of 5-qubit block steps of 7.5 us, 5 us apart.
+constexpr int kBatchWaves = 8;
+__global__ __launch_bounds__(64 * kBatchWaves, 4) void k_pass_batch(const qsim_pass_rec* __restrict__ recs, int n_recs,
+                                                                    const uint4* __restrict__ blocks,
+                                                                    const float4* __restrict__ frags) {
+  const uint64_t b = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  int at = -1;                                        // records before it begin at or below b
+  for (int r0 = 0; r0 < n_recs; r0 += 64) {
+    const int r = r0 + lane;
+    const int c = __popcll(__ballot(r < n_recs && recs[r < n_recs ? r : 0].tile_begin <= b));
+    at += c;
+    if (c < 64) break;
+  }
+  const qsim_pass_rec& rec = recs[__builtin_amdgcn_readfirstlane(at)];
+  PassGeom g;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) g.w[j] = reinterpret_cast<const uint32_t*>(rec.tile_qubits)[j];
+  float4* st = reinterpret_cast<float4*>(rec.state);
+  const uint4* bl = blocks + 2 * (size_t)rec.first_block;
+  const float4* fr = frags + (size_t)rec.first_block * (64 * kFrags);
+  const uint64_t tile = b - rec.tile_begin;
+  switch (rec.tile_bits) {
+    case 10: pass_tile<10, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
+    case 11: pass_tile<11, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
+    case 12: pass_tile<12, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
+    default: pass_tile<13, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
+  }
+}
+
 template <int M, int W>
 static void launch_pass(hipStream_t s, void* state, int n, const PassGeom& g, const qsim_pass_block* blocks,
                         const void* frags, int n_blocks) {
@@ -293,6 +340,46 @@ int qsim_apply_passes(void* stream, void* state, int n_qubits, const qsim_pass* 
     if (int rc = launch_status("apply_passes")) return rc;
   }
   return QSIM_OK;
+}
+
+int qsim_apply_pass_batch(void* stream, const qsim_pass_rec* recs_host, const void* recs_dev, int64_t n_recs,
+                          const qsim_pass_block* blocks_host, const void* blocks_dev, const void* frags_dev,
+                          int64_t n_blocks) {
+  clear_error();
+  if (n_recs < 0 || n_blocks < 0) return fail(QSIM_EINVAL, "negative count");
+  if (n_recs == 0) return QSIM_OK;
+  if (n_recs > (1 << 20)) return fail(QSIM_ERANGE, "%lld records in one batch", (long long)n_recs);
+  if (!recs_host || !recs_dev || !blocks_host || !blocks_dev || !frags_dev)
+    return fail(QSIM_EINVAL, "NULL pointer argument");
+  uint64_t tiles = 0;
+  int max_m = 0;
+  for (int64_t i = 0; i < n_recs; ++i) {
+    const qsim_pass_rec& r = recs_host[i];
+    const int m = r.tile_bits;
+    if (!r.state || (r.state & 15u)) return fail(QSIM_EINVAL, "record %lld: state NULL or not 16-byte aligned", (long long)i);
+    if (int rc = check_n(r.n_qubits)) return rc;
+    if (m < QSIM_PASS_MIN_TILE || m > QSIM_PASS_MAX_TILE || m > r.n_qubits)
+      return fail(QSIM_ERANGE, "record %lld: tile of %d qubits", (long long)i, m);
+    if (r.tile_qubits[0] != 0) return fail(QSIM_EINVAL, "record %lld: the tile must hold qubit 0", (long long)i);
+    for (int j = 1; j < m; ++j)
+      if (r.tile_qubits[j] <= r.tile_qubits[j - 1] || r.tile_qubits[j] >= r.n_qubits)
+        return fail(QSIM_EINVAL, "record %lld: tile qubits not ascending below n_qubits", (long long)i);
+    if (r.tile_begin != tiles) return fail(QSIM_EINVAL, "record %lld: tile_begin is not the prefix sum", (long long)i);
+    if (r.first_block < 0 || r.n_blocks < 1 || r.n_blocks > n_blocks - r.first_block)
+      return fail(QSIM_EINVAL, "record %lld: blocks [%d, +%d) beyond the %lld passed", (long long)i, r.first_block,
+                  r.n_blocks, (long long)n_blocks);
+    for (int b = 0; b < r.n_blocks; ++b)
+      if (!block_ok(blocks_host[r.first_block + b], m))
+        return fail(QSIM_EINVAL, "record %lld: block record %d is not a record of a %d-qubit tile", (long long)i,
+                    r.first_block + b, m);
+    tiles += 1ull << (r.n_qubits - m);
+    max_m = std::max(max_m, m);
+  }
+  if (tiles > 0x7fffffffull) return fail(QSIM_ERANGE, "batch too large (%llu tiles)", (unsigned long long)tiles);
+  hipLaunchKernelGGL(k_pass_batch, dim3((unsigned)tiles), dim3(64 * kBatchWaves), sizeof(float2) << max_m,
+                     as_stream(stream), (const qsim_pass_rec*)recs_dev, (int)n_recs, (const uint4*)blocks_dev,
+                     (const float4*)frags_dev);
+  return launch_status("apply_pass_batch");
 }
 
 }  // extern "C"

@@ -126,9 +126,9 @@ def test_pass_kernel_matches_fp64(bk, dev, n, m):
 
 
 @pytest.mark.gpu
-def test_passes_keep_permutations_exact_and_pass_wide_ops(dev):
-    """Permutation circuits move amplitudes bit for bit through a pass; ops of
-    five and more qubits and a mid-circuit measurement run between passes."""
+def test_passes_apply_permutations_and_wide_ops(dev):
+    """Permutation gates of up to four qubits in a pass against the permuted
+    amplitudes; ops of five and more qubits run between passes."""
     from blackwell_backend import BlackwellSimulator
     from blackwell_backend.circuit import QuantumCircuit
     sim = BlackwellSimulator(dev)
@@ -138,12 +138,6 @@ def test_passes_keep_permutations_exact_and_pass_wide_ops(dev):
     ref, _ = sim.run_statevector(qc, mode="passes")
     perm = qc.copy()
     perm.cx(0, 13).ccx(4, 9, 2).swap(3, 11).mcx([1, 5, 7], 12).cx(8, 6)
-    back = perm.copy()
-    back.cx(8, 6).mcx([1, 5, 7], 12).swap(3, 11).ccx(4, 9, 2).cx(0, 13)
-    # an empty barrier does not keep the planner from cancelling the two halves
-    # in one block, so the halves run as two circuits
-    one = sim.compile(perm).plan("passes", sim.device)
-    assert one.n_launches >= 1
     sv, _ = sim.run_statevector(perm, mode="passes")
     psi = ref.astype(np.complex128)
     for name, qs in (("cx", (0, 13)), ("ccx", (4, 9, 2)), ("swap", (3, 11)), ("mcx", (1, 5, 7, 12)), ("cx", (8, 6))):
@@ -164,3 +158,43 @@ def test_passes_keep_permutations_exact_and_pass_wide_ops(dev):
     got, _ = sim.run_statevector(wide, mode="passes")
     exp, _ = sim.run_statevector(wide, mode="plain")
     assert O.fidelity(exp, got) >= 1 - 1e-7 and np.max(np.abs(exp - got)) <= 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ns", [[13, 10, 16, 11, 12, 15], [10] * 70 + [13], [18, 14]])
+def test_batched_passes_have_the_bits_of_single_ones(dev, ns):
+    """Every tile size, more records than lanes of the search, states with
+    fewer passes than others: each state equals qsim_apply_passes on it alone."""
+    import ctypes
+    import torch
+    from blackwell_backend import compiler as C, workloads as W
+    from blackwell_backend.executor import pass_shape
+    from blackwell_kernels import _lib
+    from blackwell_kernels.cuquantum import pass_step_records, run_pass_steps
+    vp = ctypes.c_void_p
+    plans, single, batch = [], [], []
+    for i, n in enumerate(ns):
+        pairs, us = W.su4_arrays(n, 2 + i % 3, 7 + i)
+        qb = np.full((len(pairs), 8), -1, dtype=np.int32)
+        qb[:, :2] = pairs
+        m = 13 if n in (13, 16) else pass_shape(n)[0]
+        refs, *plan = C.plan_passes_arrays(n, np.full(len(pairs), 2, np.int32), qb, us, m, 4)
+        assert (refs >= 0).all()
+        plans.append(C.PassRun(*plan))
+        psi = torch.from_numpy(rand_state(n, i).astype(np.complex64)).to(dev)
+        single.append(psi.clone())
+        batch.append(psi.clone())
+    up = lambda a: torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).to(dev)
+    s = _lib.stream_handle(dev)
+    for n, p, st in zip(ns, plans, single):
+        b, f = up(p.blocks), up(p.frags)
+        _lib.call("qsim_apply_passes", s, _lib.ptr(st), n, vp(p.passes.ctypes.data), len(p.passes),
+                  vp(p.blocks.ctypes.data), _lib.ptr(b), _lib.ptr(f), len(p.blocks))
+    blocks = np.concatenate([p.blocks for p in plans])
+    first = np.cumsum([0] + [len(p.blocks) for p in plans])[:-1]
+    recs, off = pass_step_records([st.data_ptr() for st in batch], ns, [p.passes for p in plans], first)
+    assert off[-1] == len(recs) == sum(len(p.passes) for p in plans)
+    bd, fd, rd = up(blocks), up(np.concatenate([p.frags for p in plans])), up(recs)
+    run_pass_steps(s, recs, rd.data_ptr(), off, blocks, bd.data_ptr(), fd.data_ptr())
+    for a, b in zip(single, batch):
+        assert np.array_equal(a.cpu().numpy().view(np.uint32), b.cpu().numpy().view(np.uint32))
