@@ -36,8 +36,8 @@ batched pass steps instead.
 Sampling in both lanes uses the same rule and the same uniforms for a given
 seed: u_k = SplitMix64(seed + (k+1) * golden) >> 11 scaled by 2^-53 and
 index = smallest i with cdf(i) > u_k * ||psi||^2.  Each instance's arithmetic
-is independent of the batch it runs in (one workgroup per instance, fixed
-thread count), so a request's samples are bitwise the same alone and in a
+is independent of the batch it runs in (one workgroup per instance, whose
+thread count changes neither sums nor sampling), so a request's samples are bitwise the same alone and in a
 mix.
 
 The reference has no serving loop; its batched precedent is fixed-n and

@@ -26,7 +26,14 @@
 namespace qsim {
 
 constexpr int kTileMaxBits = 14;
-constexpr int kTileThreads = 256;
+constexpr int kTileThreadsMax = 1024;
+// Threads of an LDS program on m qubits: a step is a quad of amplitudes of a
+// two-qubit op, so 2^10 to 2^12 quads at m = 12..14 feed 8 to 16 waves, and the
+// CU holds about 16 waves whatever LDS leaves (one workgroup at m = 14, two
+// at 13, four at 12).  us with 256 / 512 / 1024 threads: one circuit of 10 / 12 /
+// 13 qubits 44 / 44 / 45, 122 / 108 / 111 and 218 / 182 / 180, 64 circuits of 14
+// qubits 506 / 407 / 387; 512 circuits of 10 qubits 71 / 73 / 107.
+static int tile_threads(int m) { return m <= 10 ? 256 : m <= 13 ? 512 : kTileThreadsMax; }
 
 // ------------------------------------------------------------ op executor
 __device__ __forceinline__ bool ctl_ok(uint32_t i, uint32_t cmask) { return (i & cmask) == cmask; }
@@ -46,6 +53,30 @@ __device__ __forceinline__ float2 crowk(const float2* __restrict__ row, const fl
   }
   return make_float2(sr + er, si + ei);
 }
+
+// Row of a one- or two-qubit matrix: products of FP32 are exact in FP64, sums
+// are FP64, one rounding at the end.  An FP64 FMA issues at about the cost of
+// two FP32 operations here and replaces the four of a compensated product, and
+// the result is the more exact one.  What bounds a program is this FP64 issue
+// from 12 qubits on (about 440 cycles per 64 quads) and the chain of an op
+// below (descriptor, coefficients, quad, sums, barrier: 0.7 us).  us, compensated
+// FP32 with 256 threads -> now: one SU(4) volume circuit of 8 / 10 / 12 / 13 qubits
+// 37 / 58 / 206 / 400 -> 27 / 44 / 108 / 182, 64 circuits of 14 qubits 952 -> 387,
+// 16-qubit programs on 10 / 12-qubit tiles 57 / 114 -> 49 / 66.
+template <int K>
+__device__ __forceinline__ float2 crowd(const double2 (&g)[K * K], int row, const double2 (&a)[K]) {
+  double r = 0.0, i = 0.0;
+#pragma unroll
+  for (int c = 0; c < K; ++c) {
+    const double2 v = g[row * K + c];
+    r = __builtin_fma(v.x, a[c].x, r);
+    r = __builtin_fma(-v.y, a[c].y, r);
+    i = __builtin_fma(v.x, a[c].y, i);
+    i = __builtin_fma(v.y, a[c].x, i);
+  }
+  return make_float2((float)r, (float)i);
+}
+__device__ __forceinline__ double2 wide(float2 v) { return make_double2(v.x, v.y); }
 
 // Dense 2^K block, one group per thread iteration; in-place safe because a
 // thread reads its whole group into registers before writing any of it.
@@ -88,37 +119,39 @@ __device__ void op_mk(float2* sh, int m, const qsim_op& op, const float2* __rest
   }
 }
 
-__device__ void apply_op(float2* sh, int m, const qsim_op& op, const float2* __restrict__ cf) {
+__device__ __forceinline__ void apply_op(float2* sh, int m, const qsim_op& op, const float2* __restrict__ cf) {
   const uint32_t N = 1u << m;
   const int nt = blockDim.x;
   switch (op.kind) {
     case QSIM_OP_M1: {
       const int q = op.q[0];
-      const float2 g0 = cf[op.coef], g1 = cf[op.coef + 1], g2 = cf[op.coef + 2], g3 = cf[op.coef + 3];
+      double2 g[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) g[k] = wide(cf[op.coef + k]);
       for (uint32_t p = threadIdx.x; p < N / 2; p += nt) {
         const uint32_t i0 = ins0(p, q), i1 = i0 | (1u << q);
         if (!ctl_ok(i0, op.cmask)) continue;
-        const float2 a0 = sh[i0], a1 = sh[i1];
-        sh[i0] = crow2(g0, a0, g1, a1);
-        sh[i1] = crow2(g2, a0, g3, a1);
+        const double2 a[2] = {wide(sh[i0]), wide(sh[i1])};
+        sh[i0] = crowd<2>(g, 0, a);
+        sh[i1] = crowd<2>(g, 1, a);
       }
       break;
     }
     case QSIM_OP_M2: {
       const int qa = op.q[0], qb = op.q[1];
       const int lo = qa < qb ? qa : qb, hi = qa < qb ? qb : qa;
-      float2 g[16];
+      double2 g[16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) g[k] = cf[op.coef + k];
+      for (int k = 0; k < 16; ++k) g[k] = wide(cf[op.coef + k]);
       for (uint32_t p = threadIdx.x; p < N / 4; p += nt) {
         const uint32_t b = ins0(ins0(p, lo), hi);
         if (!ctl_ok(b, op.cmask)) continue;
         const uint32_t i1 = b | (1u << qa), i2 = b | (1u << qb), i3 = i1 | (1u << qb);
-        const float2 a0 = sh[b], a1 = sh[i1], a2 = sh[i2], a3 = sh[i3];
-        sh[b] = crow4(g + 0, a0, a1, a2, a3);
-        sh[i1] = crow4(g + 4, a0, a1, a2, a3);
-        sh[i2] = crow4(g + 8, a0, a1, a2, a3);
-        sh[i3] = crow4(g + 12, a0, a1, a2, a3);
+        const double2 a[4] = {wide(sh[b]), wide(sh[i1]), wide(sh[i2]), wide(sh[i3])};
+        sh[b] = crowd<4>(g, 0, a);
+        sh[i1] = crowd<4>(g, 1, a);
+        sh[i2] = crowd<4>(g, 2, a);
+        sh[i3] = crowd<4>(g, 3, a);
       }
       break;
     }
@@ -239,6 +272,58 @@ __device__ __forceinline__ void run_ops(float2* sh, int m, int n_ops, GetOp get,
   }
 }
 
+// Runs a program from global memory on the LDS state.  Descriptors and
+// coefficients travel kChunk ops at a time: while a chunk runs, its threads
+// hold the next chunk's coefficients (thread 16 j + e the e-th of op j) and
+// the descriptors of the one after in flight, and put them into LDS before the
+// barrier that ends the chunk, so an op waits for no global memory.
+constexpr int kChunk = 16;
+static_assert(kChunk * kStaged == 256, "one coefficient per thread of the smallest workgroup");
+__device__ __forceinline__ void run_program(float2* sh, int m, int n_ops, const qsim_op* __restrict__ ops,
+                                            const float2* __restrict__ cf) {
+  __shared__ float2 cs[2][kChunk][kStaged];
+  __shared__ int4 ds[2][kChunk];
+  if (n_ops <= 0) return;
+  const int t = threadIdx.x, j = t / kStaged, e = t % kStaged;
+  auto desc = [&](int c) -> int4 {
+    const int k = c * kChunk + j;
+    return t < kChunk * kStaged && k < n_ops ? reinterpret_cast<const int4*>(ops)[k] : make_int4(0, 0, 0, 0);
+  };
+  auto coef = [&](int4 d) -> float2 {
+    const qsim_op op = __builtin_bit_cast(qsim_op, d);
+    return e < op_ncoef(op) ? cf[op.coef + e] : make_float2(0.f, 0.f);
+  };
+  auto put = [&](int c, int4 d, float2 v) {
+    if (t < kChunk * kStaged) {
+      cs[c & 1][j][e] = v;
+      if (e == 0) ds[c & 1][j] = d;
+    }
+  };
+  int4 d0 = desc(0), d1 = desc(1);
+  put(0, d0, coef(d0));
+  __syncthreads();
+  for (int c = 0; c * kChunk < n_ops; ++c) {
+    const float2 v = coef(d1);
+    const int4 d2 = desc(c + 2);
+    const int n = n_ops - c * kChunk < kChunk ? n_ops - c * kChunk : kChunk;
+    for (int k = 0; k < n; ++k) {
+      int4 d = ds[c & 1][k];
+      d.x = __builtin_amdgcn_readfirstlane(d.x);
+      d.y = __builtin_amdgcn_readfirstlane(d.y);
+      d.z = __builtin_amdgcn_readfirstlane(d.z);
+      d.w = __builtin_amdgcn_readfirstlane(d.w);
+      qsim_op op = __builtin_bit_cast(qsim_op, d);
+      const bool staged = op_ncoef(op) >= 0;
+      if (staged) op.coef = 0;
+      if (staged) apply_op(sh, m, op, cs[c & 1][k]);
+      else apply_op(sh, m, op, cf);
+      if (k + 1 == n) put(c + 1, d1, v);
+      __syncthreads();
+    }
+    d1 = d2;
+  }
+}
+
 // ------------------------------------------------------------ tile geometry
 struct TileGeom {
   int n, m, L;          // state qubits, tile bits, contiguous low bits
@@ -282,7 +367,7 @@ __device__ void tile_store(const float2* sh, float4* __restrict__ st, uint64_t b
   for (uint32_t s = threadIdx.x; s < ns; s += blockDim.x) st[tile_slot(s, base, g)] = sh4[s];
 }
 
-__global__ __launch_bounds__(kTileThreads) void k_tile_program(float4* __restrict__ st, TileGeom g,
+__global__ __launch_bounds__(kTileThreadsMax) void k_tile_program(float4* __restrict__ st, TileGeom g,
                                                               const qsim_op* __restrict__ ops,
                                                               int n_ops,
                                                               const float2* __restrict__ cf) {
@@ -291,7 +376,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_program(float4* __restric
   const uint64_t base = tile_base(gblock<uint64_t>(), g);
   tile_load(sh, st, base, g);
   __syncthreads();
-  run_ops(sh, g.m, n_ops, [&](int k) { return ops[k]; }, cf);
+  run_program(sh, g.m, n_ops, ops, cf);
   tile_store(sh, st, base, g);
 }
 
@@ -301,7 +386,7 @@ struct Fused1Q {
   uint8_t q[kFusedMax];   // tile-local target of gate k
   int first, count;       // gates [first, first+count) of the caller's list
 };
-__global__ __launch_bounds__(kTileThreads) void k_tile_fused1q(float4* __restrict__ st, TileGeom g,
+__global__ __launch_bounds__(kTileThreadsMax) void k_tile_fused1q(float4* __restrict__ st, TileGeom g,
                                                               Fused1Q f,
                                                               const float2* __restrict__ gates) {
   extern __shared__ float2 sh[];
@@ -480,7 +565,7 @@ __device__ void lds_sample(const float2* sh, int n, uint64_t seed, uint32_t shot
   }
 }
 
-__global__ __launch_bounds__(kTileThreads) void k_instances(float2* __restrict__ states,
+__global__ __launch_bounds__(kTileThreadsMax) void k_instances(float2* __restrict__ states,
                                                            const qsim_instance* __restrict__ inst,
                                                            const qsim_op* __restrict__ ops,
                                                            const float2* __restrict__ cf,
@@ -499,7 +584,7 @@ __global__ __launch_bounds__(kTileThreads) void k_instances(float2* __restrict__
   }
   __syncthreads();
   const qsim_op* iops = ops + in.op_off;
-  run_ops(sh, n, (int)in.n_ops, [&](int k) { return iops[k]; }, cf);
+  run_program(sh, n, (int)in.n_ops, iops, cf);
   if (in.want & 1)
     for (uint32_t i = threadIdx.x; i < N; i += blockDim.x) gst[i] = sh[i];
   if (in.shots) lds_sample(sh, n, in.seed, in.shots, shots_out + in.shot_off, pre);
@@ -641,7 +726,7 @@ int qsim_tile_program(void* stream, void* state, int n_qubits, uint64_t tile_mas
   if (int rc = make_geom(g, n_qubits, tile_mask)) return rc;
   const uint64_t tiles = 1ull << g.nc;
   const size_t lds = sizeof(float2) << g.m;
-  hipLaunchKernelGGL(k_tile_program, grid1d(tiles), dim3(kTileThreads), lds, as_stream(stream),
+  hipLaunchKernelGGL(k_tile_program, grid1d(tiles), dim3(tile_threads(g.m)), lds, as_stream(stream),
                      (float4*)state, g, (const qsim_op*)ops_dev, n_ops, (const float2*)coefs_dev);
   return launch_status("tile_program");
 }
@@ -683,7 +768,7 @@ int qsim_apply_gates_fused(void* stream, void* state, int n_qubits, const void* 
       f.q[j] = (uint8_t)__builtin_popcountll(mask & ((1ull << t) - 1));  // local position
     }
     const size_t lds = sizeof(float2) << g.m;
-    hipLaunchKernelGGL(k_tile_fused1q, grid1d(1ull << g.nc), dim3(kTileThreads), lds, s,
+    hipLaunchKernelGGL(k_tile_fused1q, grid1d(1ull << g.nc), dim3(tile_threads(g.m)), lds, s,
                        (float4*)state, g, f, (const float2*)gates_dev);
     if (int rc = launch_status("apply_gates_fused")) return rc;
     k += cnt;
@@ -736,7 +821,7 @@ int qsim_run_instances(void* stream, void* states_base, uint64_t n_state_slots,
     if (int rc = check_ops(ops_host + in.op_off, in.n_ops, in.n_qubits, n_coefs, i)) return rc;
   }
   const size_t lds = sizeof(float2) << max_qubits;
-  hipLaunchKernelGGL(k_instances, dim3(n_inst), dim3(kTileThreads), lds, as_stream(stream),
+  hipLaunchKernelGGL(k_instances, dim3(n_inst), dim3(tile_threads(max_qubits)), lds, as_stream(stream),
                      (float2*)states_base, (const qsim_instance*)inst_dev, (const qsim_op*)ops_dev,
                      (const float2*)coefs_dev, (int64_t*)shots_dev);
   return launch_status("run_instances");
