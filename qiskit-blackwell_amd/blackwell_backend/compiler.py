@@ -293,46 +293,26 @@ def _mask(qs):
     return m
 
 
-def plan_blocks(ops, n, k=5, effort=1, arrays=None):
+def plan_blocks(ops, n, k=5, effort=1):
     """Pack unitary ops into dense blocks of min(k, n) qubits with the
     library's host planner (qsim_plan_blocks_search, FP64): an op joins a
     block if its qubits lie in the block's qubit set and none of them was
     touched by an earlier op left out; effort 1 (the default) also searches
     the block qubit sets around each seed op, effort 0 is the greedy scan
     alone.  measure/reset split the
-    list into independently planned segments.  arrays: a list that keeps the
-    segments' flat arrays for a later plan of the same ops (plan_passes);
-    they are half of its time.  Returns a list of Block | Op (ops wider than k
-    pass through)."""
+    list into independently planned segments.  Returns a list of Block | Op
+    (ops wider than k pass through)."""
     out = []
     seg = []
-    arrays = _segment_arrays(arrays)
     for op in ops:
         if op.kind in ("measure", "reset"):
-            out.extend(_plan_segment(seg, n, k, effort, arrays))
+            out.extend(_plan_segment(seg, n, k, effort))
             seg = []
             out.append(op)
         else:
             seg.append(op)
-    out.extend(_plan_segment(seg, n, k, effort, arrays))
+    out.extend(_plan_segment(seg, n, k, effort))
     return out
-
-
-def _segment_arrays(kept):
-    """Function of a segment's ops that gives its _op_arrays; called once per
-    non-empty segment in order, it takes them from the list `kept` or puts
-    them there (None: nothing is kept)."""
-    if kept is None:
-        return _op_arrays
-    done = iter(tuple(kept))
-
-    def arrays(ops):
-        a = next(done, None)
-        if a is None:
-            a = _op_arrays(ops)
-            kept.append(a)
-        return a
-    return arrays
 
 
 def plan_blocks_arrays(n, op_nq, op_qubits, op_mats, k=5, effort=1):
@@ -380,10 +360,10 @@ def _op_arrays(ops):
     return nq, qb, np.concatenate(mats)
 
 
-def _plan_segment(ops, n, k, effort, arrays):
+def _plan_segment(ops, n, k, effort=1):
     if not ops:
         return []
-    refs, bqs, bm = plan_blocks_arrays(n, *arrays(ops), k, effort)
+    refs, bqs, bm = plan_blocks_arrays(n, *_op_arrays(ops), k, effort)
     res = []
     for e in refs:
         if e >= 0:
@@ -432,17 +412,15 @@ def plan_passes_arrays(n, op_nq, op_qubits, op_mats, tile_bits, low_bits):
     return refs, passes[:int((refs >= 0).sum())], blocks[:n_blk.value], frags[:n_blk.value]
 
 
-def plan_passes(ops, n, tile_bits, low_bits, arrays=None):
-    """Pack unitary ops into block passes (n >= PASS_MIN_QUBITS); arrays as
-    plan_blocks.  Returns a list of PassRun | Op (measure/reset, and ops of
-    more than 4 qubits)."""
+def plan_passes(ops, n, tile_bits, low_bits):
+    """Pack unitary ops into block passes (n >= PASS_MIN_QUBITS).  Returns a
+    list of PassRun | Op (measure/reset, and ops of more than 4 qubits)."""
     out, seg = [], []
-    arrays = _segment_arrays(arrays)
 
     def flush():
         if not seg:
             return
-        refs, passes, blocks, frags = plan_passes_arrays(n, *arrays(seg), tile_bits, low_bits)
+        refs, passes, blocks, frags = plan_passes_arrays(n, *_op_arrays(seg), tile_bits, low_bits)
         e = 0
         while e < len(refs):
             if refs[e] < 0:

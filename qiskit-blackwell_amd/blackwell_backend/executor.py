@@ -33,31 +33,17 @@ from . import compiler as C
 
 WHOLE_TILE_MAX = 13     # n <= 13: the whole state is one LDS tile (64 KiB)
 BLOCK_MIN_QUBITS = 10   # the MFMA block kernel needs 2^10 amplitudes
-# auto-mode cost model for 10 <= n <= 13 (MI355X measurements): one op of the
-# one-workgroup LDS program costs ~2 us at 12 qubits and scales with the
-# amplitudes per thread; one fused block costs ~5 us (launch-bound at this size)
-WHOLE_OP_US_12Q = 2.0
-BLOCK_US = 5.0
+# auto between 10 and 13 qubits, us: an op of the one-workgroup LDS program
+# against a block pass and each op that no pass holds (_auto_mode)
+WHOLE_OP_US = lambda n: 0.55 + 0.65 * 2.0 ** (n - 12)
+PASS_US = 5.0
+WIDE_OP_US = 6.0
 # plan steps a HIP graph can hold: library launches on the current stream with
 # device-resident arguments only (no host uploads, no host-side decisions)
 GRAPH_SAFE_STEPS = ("passes", "blocks", "mfma", "tile", "mcgate")
 # fusion widths of the MFMA block kernels and the smallest state each runs on
 BLOCK_WIDTHS = {4: 11, 5: BLOCK_MIN_QUBITS, 6: 13}
 TUNE_REPS = 3
-# Tile programs above 13 qubits: a tile of m qubits is one workgroup, so m
-# trades ops fused per HBM pass against workgroups per pass (2^(n-m)).
-# Measured on MI355X (A/B circuit families, 16 and 20 qubits): 10-qubit
-# tiles beat 13-qubit ones by 2-3x there (13-qubit tiles give 8-128
-# workgroups); larger states can afford larger tiles.
-AUTO_TILES_MAX_QUBITS = 20   # auto considers tile programs up to this size
-# auto-mode cost model for 14 <= n <= 20 (same measurements): a tile pass
-# ~5 us plus ~0.85 us per op at 16 qubits (x1.13 per qubit; a dense 4x4 op
-# counts 1.4, a wider dense op 2); a fused block ~8.2 us at 16 qubits (x1.07
-# per qubit)
-TILE_PASS_US = 5.0
-TILE_OP_US_16Q = 0.85
-TILE_OP_WEIGHT = {"m2": 1.4, "mk": 2.0}
-BLOCK_US_16Q = 8.2
 
 
 def block_width(mode):
@@ -70,6 +56,11 @@ def block_modes(n):
     return [f"blocks/{k}" if k != 5 else "blocks" for k, nmin in sorted(BLOCK_WIDTHS.items()) if n >= nmin]
 
 
+# Tile programs above 13 qubits: a tile of m qubits is one workgroup, so m
+# trades ops fused per HBM pass against workgroups per pass (2^(n-m)).
+# Measured on MI355X (A/B circuit families, 16 and 20 qubits): 10-qubit
+# tiles beat 13-qubit ones by 2-3x there (13-qubit tiles give 8-128
+# workgroups); larger states can afford larger tiles.
 def default_tile_shape(n):
     """(tile qubits, always-included low qubits) of "tiles" for n qubits."""
     if n <= WHOLE_TILE_MAX:
@@ -187,7 +178,6 @@ class CompiledCircuit:
         self._blocks = None
         self._tiles = None
         self._auto = None
-        self._arrays = None
         self._graphs = {}
         self._tuned = {}
         self.has_stochastic = any(o.kind in ("measure", "reset") for o in ops)
@@ -273,13 +263,13 @@ class CompiledCircuit:
                 best, best_ms = mode, ms
         return best
 
-    def block_entries(self, k=5, arrays=None):
+    def block_entries(self, k=5):
         """plan_blocks of the ops with k-qubit blocks (computed once per
         compiled circuit and width)."""
         if self._blocks is None:
             self._blocks = {}
         if k not in self._blocks:
-            self._blocks[k] = C.plan_blocks(self.ops, self.n_qubits, k=k, arrays=arrays)
+            self._blocks[k] = C.plan_blocks(self.ops, self.n_qubits, k=k)
         return self._blocks[k]
 
     # ---------------------------------------------------------------- plans
@@ -299,13 +289,8 @@ class CompiledCircuit:
         return self._tiles
 
     def resolve_mode(self, mode, device=None):
-        """auto: the whole state as one LDS program below 10 qubits; between
-        10 and 13 qubits that or MFMA block passes, and between 14 and 20
-        qubits tile programs or block passes, where the cost model prices the
-        MFMA side as one launch per 5-qubit block (deep circuits favour it:
-        one block absorbs many ops); block passes above.  The tile programs'
-        compensated arithmetic is the more exact, so the line between the two
-        stays where one launch per block puts it although a pass is cheaper.
+        """auto: the whole state as one LDS program below 10 qubits, block
+        passes above, but for the circuits _auto_mode names.
         tune: the mode tuned_mode measured fastest on `device`."""
         if mode == "tune":
             if device is None:
@@ -314,29 +299,30 @@ class CompiledCircuit:
         if mode != "auto":
             return mode
         if self._auto is None:
-            arrays = []
-            self._auto = self._auto_mode(arrays)
-            # the plan that follows takes the decision's arrays over
-            self._arrays = arrays if self._auto == "passes" else None
+            self._auto = self._auto_mode()
         return self._auto
 
-    def _auto_mode(self, arrays):
+    def _auto_mode(self):
+        """Block passes from 10 qubits on: over ladders, QFT, SU(4) volume and
+        multi-controlled circuits of 10 to 20 qubits and depths 1 to 8 they
+        measured faster than LDS programs (10 qubits 17-52 us against 22-134,
+        13 qubits 18-97 against 33-374, 16 qubits 20-130 against 26-330, 20
+        qubits 27-267 against 53-667) and closer to FP64 (QFT of 16 qubits
+        1.5e-7 against 5.7e-7, SU(4) volume 1.7e-7 against 2.7e-7).  An op on
+        more than four qubits interrupts a pass and takes a launch of its own,
+        where an LDS program of at most 13 qubits goes on: 100 ops of 12 qubits,
+        10 / 20 / 50 of them with six controls, 79 / 130 / 194 us in passes
+        against 103 / 109 / 104, of 13 qubits 69 / 122 / 198 against 153 / 161 /
+        149.  Dense matrices of five qubits are slow in LDS programs (20 of
+        100: 183 against 778 us), and tile programs of 14 qubits and more lose
+        at every share (14 qubits 58 / 105 / 184 against 104 / 156 / 249)."""
         n = self.n_qubits
-        if n < BLOCK_MIN_QUBITS:
+        if n < C.PASS_MIN_QUBITS:
             return "whole"
-        if n > AUTO_TILES_MAX_QUBITS:
-            return "passes"
         if n > WHOLE_TILE_MAX:
-            passes = sum(1 for e in self.tile_entries() if isinstance(e, C.TilePass))
-            others = len(self.tile_entries()) - passes
-            w_ops = sum(TILE_OP_WEIGHT.get(o.kind, 1.0) for o in self.ops)
-            t_tiles = (passes * TILE_PASS_US + w_ops * TILE_OP_US_16Q * 1.13 ** (n - 16)
-                       + others * BLOCK_US_16Q)
-            t_blocks = len(self.block_entries(arrays=arrays)) * BLOCK_US_16Q * 1.07 ** (n - 16)
-            return "tiles" if t_tiles < t_blocks else "passes"
-        t_whole = len(self.ops) * WHOLE_OP_US_12Q * 2.0 ** (n - 12)
-        t_blocks = len(self.block_entries(arrays=arrays)) * BLOCK_US
-        return "passes" if t_blocks < t_whole else "whole"
+            return "passes"
+        wide = sum(1 for o in self.ops if len(o.all_qubits) > 4 and o.kind != "mk")
+        return "whole" if len(self.ops) * WHOLE_OP_US(n) < PASS_US + wide * WIDE_OP_US else "passes"
 
     def _build(self, mode, device):
         n = self.n_qubits
@@ -361,8 +347,7 @@ class CompiledCircuit:
         if mode == "passes":
             if n < C.PASS_MIN_QUBITS:
                 raise ValueError(f"block passes need n >= {C.PASS_MIN_QUBITS} (n = {n})")
-            arrays, self._arrays = self._arrays, None
-            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n), arrays=arrays), device)
+            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n)), device)
         if mode == "blocks":
             if n < 10:
                 return self._build_tiles(C.plan_tiles(self.ops, n, m=n), device)
