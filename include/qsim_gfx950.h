@@ -565,6 +565,14 @@ int qsim_cheb_pauli_batch_step(void* stream, int n_qubits, int n_groups, const v
                                const void* sm, const void* coef, int n_rhs, double scale,
                                const void* t_cur, void* t_prev_next, void* acc, void* comp,
                                double c_re, double c_im, int first);
+/* The whole series sum_k c_k T_k, k = 0..n_terms (n_terms >= 1), as the terms
+ * of qsim_cheb_pauli_batch_step give it: coeffs (host) holds n_terms + 1 complex
+ * pairs, t0 T_0 on entry, and the vectors are scratch otherwise.  The sum is
+ * left in t1 where n_terms is odd and in t0 where it is even.  t0 and t1:
+ * 16-byte aligned.  (new)                                                   */
+int qsim_cheb_pauli_evolve(void* stream, int n_qubits, int n_groups, const void* groups,
+                           const void* sm, const void* coef, int n_rhs, double scale, void* t0,
+                           void* t1, void* acc, void* comp, const double* coeffs, int n_terms);
 /* acc = c * t, comp = 0 (first Chebyshev term), n elements. (new)        */
 int qsim_cheb_init_acc(void* stream, void* acc, void* comp, const void* t, int64_t n,
                        double c_re, double c_im);

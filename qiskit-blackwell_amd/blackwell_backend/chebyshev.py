@@ -28,12 +28,13 @@ the default.
 A Hamiltonian built from a Pauli sum keeps its grouped Pauli tables, and a
 single state with FP64 row sums runs each term matrix-free by default
 (qsim_cheb_pauli_step): every entry is recomputed from the tables as the
-CSR builder computes it, so no index or value stream is read.  Batches of
-16 qubits and more do the same when all entries are real
-(qsim_cheb_pauli_batch_step, state-major, so without the two transposes):
-the states share the entry evaluation and a tile of T_k in LDS, and the
-sums are those of the CSR term bit for bit.  The CSR stays for small
-batches, complex entries, fp32c row sums and the split term.
+CSR builder computes it, so no index or value stream is read.  When all
+entries are real, one state of 9 qubits or more and batches of 16 qubits and
+more run the whole series in one call (qsim_cheb_pauli_evolve): a tile of
+T_k in LDS serves the near entries, the states of a batch share the entry
+evaluation, the accumulator is updated by two terms at a time, and the sums
+are those of the CSR terms bit for bit.  The CSR stays for small batches,
+complex entries, fp32c row sums and the split term.
 
 Row sums of the SpMM (accumulate=):
   "fp64"   every FP32 x FP32 product is exact in FP64 and is summed with
@@ -42,6 +43,7 @@ Row sums of the SpMM (accumulate=):
   "fp32c"  TwoProduct + Neumaier compensated FP32, the reference's
            TwoProduct/Kahan row sum (bwk/csrc/spmv_sm120.cu:26-54).
 """
+import ctypes
 import math
 import time
 
@@ -84,18 +86,16 @@ ACCUMULATE = {"fp64": 0, "fp32c": 1}
 
 
 def tiled_term(pauli, n, R):
-    """Whether the tiled matrix-free term (qsim_cheb_pauli_batch_step) runs R
-    states of n qubits: real entries, and a size where it measured faster
-    than what it replaces.  Batches against the CSR term, us per term of a
-    Heisenberg chain: 17 qubits with 2 / 32 states 23 -> 16 and 81 -> 67,
+    """Whether the tiled matrix-free terms (qsim_cheb_pauli_evolve) run R states
+    of n qubits: real entries, and a size where they measured faster than
+    what they replace.  One state always: a term of a Heisenberg chain takes
+    6.8 / 8.1 / 17.5 us on 12 / 16 / 19 qubits, 9.5 / 14 / 25 untiled.  Batches
+    against the CSR term: 17 qubits with 2 / 32 states 23 -> 16 and 81 -> 64 us,
     16 qubits with 16 states 33 -> 30 but with 8 states 20 -> 24, 14 qubits
-    with 32 states 12 -> 16 (the CSR and T_k fit the L2s there).  One state
-    against the untiled term: 18 qubits 17.1 -> 14.3, 19 qubits 25 -> 26."""
+    with 32 states 12 -> 16 (the CSR and T_k fit the L2s there)."""
     if pauli.groups is None or n < _lib.PAULI_BATCH_MIN_QUBITS:
         return False
-    if R == 1:
-        return n <= 18
-    return R > 1 and (n >= 17 or (n == 16 and R >= 16))
+    return R == 1 or (R > 1 and (n >= 17 or (n == 16 and R >= 16)))
 
 
 def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumulate="fp64", split=False,
@@ -107,7 +107,7 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     built from (qsim_cheb_pauli_step) instead of the CSR; None (default)
     does so for one state with accumulate="fp64" when the Hamiltonian
     carries its Pauli tables, and, when its entries are real, for batches of
-    the sizes tiled_term names (qsim_cheb_pauli_batch_step)."""
+    the sizes tiled_term names (qsim_cheb_pauli_evolve)."""
     if accumulate not in ACCUMULATE:
         raise ValueError(f"accumulate must be one of {sorted(ACCUMULATE)}, got {accumulate!r}")
     mode = ACCUMULATE[accumulate]
@@ -143,14 +143,11 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     comp = torch.empty_like(A)
     s = stream_handle(dev)
     n_el = N * R
-    c0 = complex(coeffs[0])
-    call("qsim_cheb_init_acc", s, ptr(acc), ptr(comp), ptr(A), n_el, c0.real, c0.imag)
     if use_tiled:
-        targs = (h.n_qubits,) + pauli.batch_args() + (R, scale)
-
-        def term(cur_, prv_, ck, first):
-            call("qsim_cheb_pauli_batch_step", s, *targs, ptr(cur_), ptr(prv_), ptr(acc), ptr(comp),
-                 ck.real, ck.imag, first)
+        cf = np.ascontiguousarray(coeffs, dtype=np.complex128)
+        call("qsim_cheb_pauli_evolve", s, h.n_qubits, *pauli.batch_args(), R, scale, ptr(A), ptr(B), ptr(acc),
+             ptr(comp), ctypes.c_void_p(cf.ctypes.data), K)
+        out = B if K % 2 else A
     elif use_mf:
         pargs = (h.n_qubits,) + pauli.step_args() + (scale,)
 
@@ -171,13 +168,16 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
         def term(cur_, prv_, ck, first):
             call("qsim_cheb_spmm_step", s, *args, ptr(cur_), ptr(prv_), ptr(acc), ptr(comp),
                  ck.real, ck.imag, first, mode)
-    term(A, B, complex(coeffs[1]), 1)
-    cur, prv = B, A
-    for k in range(2, K + 1):
-        term(cur, prv, complex(coeffs[k]), 0)
-        cur, prv = prv, cur
-    call("qsim_cheb_finish", s, ptr(prv), ptr(acc), ptr(comp), n_el)
-    out = prv if use_tiled else prv.transpose(0, 1).contiguous()
+    if not use_tiled:
+        c0 = complex(coeffs[0])
+        call("qsim_cheb_init_acc", s, ptr(acc), ptr(comp), ptr(A), n_el, c0.real, c0.imag)
+        term(A, B, complex(coeffs[1]), 1)
+        cur, prv = B, A
+        for k in range(2, K + 1):
+            term(cur, prv, complex(coeffs[k]), 0)
+            cur, prv = prv, cur
+        call("qsim_cheb_finish", s, ptr(prv), ptr(acc), ptr(comp), n_el)
+        out = prv.transpose(0, 1).contiguous()
     torch.cuda.synchronize(dev)
     elapsed = time.perf_counter() - t_start
     info = {

@@ -161,7 +161,8 @@ class PauliTables:
         return self.args() + (_lib.ptr(self.gconst),)
 
     def batch_args(self):
-        """(n_groups, groups, sm, coef) pointers for qsim_cheb_pauli_batch_step."""
+        """(n_groups, groups, sm, coef) pointers for qsim_cheb_pauli_batch_step and
+        qsim_cheb_pauli_evolve."""
         from blackwell_kernels import _lib
         return (self.n_groups, _lib.ptr(self.groups), _lib.ptr(self.sm), _lib.ptr(self.coef))
 

@@ -96,6 +96,7 @@ PROTOTYPES = {
                                        _vp, _vp, _d, _d, _i]),
     "qsim_cheb_pauli_step": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _d, _vp, _vp, _vp, _vp, _d, _d, _i]),
     "qsim_cheb_pauli_batch_step": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _d, _vp, _vp, _vp, _vp, _d, _d, _i]),
+    "qsim_cheb_pauli_evolve": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _d, _vp, _vp, _vp, _vp, _vp, _i]),
     "qsim_cheb_init_acc": (_i, [_vp, _vp, _vp, _vp, _i64, _d, _d]),
     "qsim_cheb_finish": (_i, [_vp, _vp, _vp, _vp, _i64]),
 }

@@ -10,6 +10,7 @@
 // epilogue, so one launch per Chebyshev term touches A, T_k, T_{k-1}, the
 // accumulator and its compensation exactly once.
 #include "qsim_internal.hpp"
+#include <utility>
 
 namespace qsim {
 
@@ -721,33 +722,63 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli1(int n_groups, const ui
   }
 }
 
-// Matrix-free term over a Pauli sum with real entries, C right-hand sides per
-// workgroup (RHS-major: vector j at j * 2^n).  A workgroup owns a tile of 256
-// consecutive rows, lane = row: it copies the tile's T_k (C vectors) into LDS,
-// serves the groups whose X mask stays inside the tile from there, and loads
-// the others as the contiguous partner tile (lanes permuted by the mask's low
-// bits).  Entries, their rounding and the FP64 sum in group order are those of
+// What a matrix-free term does with T_{k+1} once its row sums are there.  The
+// accumulator pair is read and written by every second term only, which adds
+// c_k T_k (T_k's own rows are in LDS) and then c_{k+1} T_{k+1}: the additions
+// and their order are those of one accumulation per term, and a term moves 40
+// instead of 56 bytes per row on average.  The first term starts the pair from
+// c_0 T_0, the last one writes acc + comp in the place of T_{k+1}.
+enum : int { kChebFirst = 1, kChebInit = 2, kChebPair = 4, kChebSkip = 8, kChebLast = 16 };
+struct ChebAcc {
+  float2 c, c_cur;                              // c_{k+1}, c_k
+  int mode;
+};
+template <bool NT>
+__device__ __forceinline__ void cheb_store(const RowSum<kAccF64>& sum, double scale, const ChebAcc& e, float2 own,
+                                           float2* __restrict__ tpn, float2* __restrict__ acc,
+                                           float2* __restrict__ comp, uint64_t at) {
+  const bool first = e.mode & kChebFirst;
+  const float2 tp = first ? make_float2(0.f, 0.f) : ld2<NT>(tpn + at);
+  const float2 tn = sum.next(scale, tp, first);
+  if (!(e.mode & kChebLast)) st2<NT>(tpn + at, tn);
+  if (e.mode & kChebSkip) return;
+  float2 a, k2;
+  if (e.mode & kChebInit) {
+    a = cmulc(e.c_cur, own);
+    k2 = make_float2(0.f, 0.f);
+  } else {
+    a = ld2<NT>(acc + at);
+    k2 = ld2<NT>(comp + at);
+    if (e.mode & kChebPair) {
+      const float2 v = cmulc(e.c_cur, own);
+      neu_add(a.x, k2.x, v.x);
+      neu_add(a.y, k2.y, v.y);
+    }
+  }
+  const float2 v = cmulc(e.c, tn);
+  neu_add(a.x, k2.x, v.x);
+  neu_add(a.y, k2.y, v.y);
+  if (e.mode & kChebLast) {
+    st2<NT>(tpn + at, make_float2(a.x + k2.x, a.y + k2.y));
+  } else {
+    st2<NT>(acc + at, a);
+    st2<NT>(comp + at, k2);
+  }
+}
+
+// Matrix-free terms over a Pauli sum with real entries.  A workgroup owns a
+// tile of consecutive rows: it copies the tile's T_k into LDS, serves the
+// groups whose X mask stays inside the tile from there, and loads the others
+// as the contiguous partner tile (lanes permuted by the mask's low bits).
+// Entries, their rounding and the FP64 sum in group order are those of
 // k_cheb_pauli1, so the results have its bits; a row whose entry is zero adds
 // nothing, and a group whose entry is zero in the whole wave loads nothing.
 //  * Tables: one 64-byte record per group (qsim_pauli_group) holds everything
 //    of a group of one or two terms, so a group costs one scalar load instead
 //    of a chain of four.
-//  * C = 4: the entry of one or two terms is picked, not summed: the wave's
-//    part of the parities on the scalar unit, the lane's part by popcounts
-//    only where a mask reaches the lane bits.  C = 1 sums the signed terms
-//    (the scalar work would not be shared).
-//  * A branch merges before the FMAs: every kind of group yields one value per
-//    row, and one sequence of FMAs adds it (FMAs in each branch made the
-//    compiler copy the FP64 sums at every merge: 48 VALU instructions per
-//    group at C = 4 against 36; 12.5 against 11.2 us at C = 1, 17 qubits).
-// What bounds it: at C = 4 the T_k loads that miss L2 (3.2 GB per 20-qubit term
-// of 32 right-hand sides, about 5.5 TB/s), then the entry evaluation; at C = 1
-// the evaluation.  Times per term of a Heisenberg chain against the kernels
-// before, us: 20 qubits with 2 / 4 / 8 / 32 right-hand sides 273 / 278 / 385 /
-// 838 (CSR) -> 72 / 88 / 153 / 617, 22 qubits with 32 3660 -> 2672; one
-// right-hand side of 10 / 15 / 18 qubits 9.5 / 14.1 / 17.1 (k_cheb_pauli1) ->
-// 7.5 / 10.0 / 14.3.  C = 2 and 8 and tiles of 512 and 1024 rows measured the
-// same to 15 % slower.
+//  * The entry of one or two terms is picked, not summed: the wave's part of
+//    the parities on the scalar unit, the lane's part by popcounts only where a
+//    mask reaches the lane bits.
 struct PauliGroup {       // qsim_pauli_group
   uint64_t xm;
   uint32_t t0;
@@ -760,15 +791,35 @@ __device__ __forceinline__ bool nonzero(double v) { return (__double_as_longlong
 __device__ __forceinline__ double flip_sign(double v, uint32_t bit31) {
   return __hiloint2double((int)((uint32_t)__double2hiint(v) ^ bit31), __double2loint(v));
 }
+__device__ __forceinline__ uint32_t par64(uint64_t m) { return (uint32_t)__builtin_popcountll(m) & 1u; }
+// Entry of a one- or two-term group from the parities of its terms: +-(c0 + c1)
+// where they agree, +-(c0 - c1) where they differ, the sign that of c0.
+__device__ __forceinline__ double pair_entry(const PauliGroup& d, uint32_t p0, uint32_t p1) {
+  return flip_sign(((p0 ^ p1) & 1u) == 0 ? d.same : d.diff, p0 << 31);
+}
 
-template <typename R, int C, int U, bool NT>
+// Four vectors per workgroup (vector j at j * 2^n), tiles of 256 rows, lane =
+// row: an entry is evaluated once for the four.  A branch merges before the
+// FMAs: every kind of group yields one value per row, and one sequence of FMAs
+// adds it (FMAs in each branch made the compiler copy the FP64 sums at every
+// merge: 48 VALU instructions per group against 36).
+// What bounds it: the T_k loads that miss L2 (3.2 GB per 20-qubit term of 32
+// vectors with the accumulator in every term, about 5.5 TB/s), then the entry
+// evaluation.  Times per term of a Heisenberg chain against the CSR term, us:
+// 20 qubits with 2 / 4 / 8 / 32 vectors 273 / 278 / 385 / 838 -> 72 / 88 / 153
+// / 617, 22 qubits with 32 3660 -> 2672, all with one accumulation per term;
+// with one per two terms 32 states of 20 qubits evolve in 35.8 ms instead of
+// 43.4 (58.7 on the CSR).  Two and eight vectors and tiles of 512 and 1024 rows measured the same to 15 % slower.
+constexpr int kPauliVecs = 4;
+template <typename R, bool NT>
 __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const PauliGroup* __restrict__ tab,
                                                          const uint64_t* __restrict__ sm,
                                                          const double2* __restrict__ coef, int n_bits,
                                                          int n_rhs, int by_rhs, double scale,
                                                          const float2* __restrict__ tc,
                                                          float2* __restrict__ tpn, float2* __restrict__ acc,
-                                                         float2* __restrict__ comp, float2 c, int first) {
+                                                         float2* __restrict__ comp, ChebAcc e) {
+  constexpr int C = kPauliVecs;
   constexpr uint32_t rows = kThreads;
   constexpr int b = __builtin_ctz(rows);
   __shared__ float4 X4[C * rows / 2];
@@ -807,28 +858,16 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const Pau
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t wbase = base | (uint64_t)(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6);
   // parity of the wave's part of the row under mask m
-  auto wpar = [&](uint64_t m) -> uint32_t { return (uint32_t)__builtin_popcountll(wbase & m) & 1u; };
-  // entry of a one- or two-term group from its parities: +-(c0 + c1) where
-  // they agree, +-(c0 - c1) where they differ, the sign that of c0
-  auto uniform_entry = [&](const PauliGroup d) -> double {
-    const uint32_t p0 = wpar(d.m0), p1 = wpar(d.m1);
-    return flip_sign(p0 == p1 ? d.same : d.diff, p0 << 31);
+  auto wpar = [&](uint64_t m) -> uint32_t { return par64(wbase & m); };
+  auto needed = [&](const PauliGroup& d) -> bool {
+    if (d.kind != QSIM_PAULI_GROUP_PAIR || ((d.m0 | d.m1) & 63u)) return true;
+    return nonzero(pair_entry(d, wpar(d.m0), wpar(d.m1)));
   };
-  auto needed = [&](const PauliGroup d) -> bool {
-    if (C == 1 || d.kind != QSIM_PAULI_GROUP_PAIR || ((d.m0 | d.m1) & 63u)) return true;
-    return nonzero(uniform_entry(d));
-  };
-  auto row_parity = [&](uint64_t m) -> uint32_t {
-    return (sizeof(R) == 4 ? (uint32_t)__popc((uint32_t)r & (uint32_t)m) : (uint32_t)__popcll((uint64_t)r & m)) << 31;
-  };
-  auto add_group = [&](const PauliGroup d, const float2 (&x)[C]) {
+  auto add_group = [&](const PauliGroup& d, const float2 (&x)[C]) {
     double v;
-    if (d.kind == QSIM_PAULI_GROUP_PAIR && C == 1) {
-      v = (double)(float)(flip_sign(d.c0, row_parity(d.m0)) + flip_sign(d.c1, row_parity(d.m1)));
-    } else if (d.kind == QSIM_PAULI_GROUP_PAIR && ((d.m0 | d.m1) & 63u)) {
-      const uint32_t p0 = (uint32_t)__popc(lane & (uint32_t)d.m0) + wpar(d.m0);
-      const uint32_t p1 = (uint32_t)__popc(lane & (uint32_t)d.m1) + wpar(d.m1);
-      v = flip_sign(((p0 ^ p1) & 1u) == 0 ? d.same : d.diff, p0 << 31);
+    if (d.kind == QSIM_PAULI_GROUP_PAIR && ((d.m0 | d.m1) & 63u)) {
+      v = pair_entry(d, (uint32_t)__popc(lane & (uint32_t)d.m0) + wpar(d.m0),
+                     (uint32_t)__popc(lane & (uint32_t)d.m1) + wpar(d.m1));
     } else if (d.kind == QSIM_PAULI_GROUP_TERMS) {
       v = 0.0;
 #pragma unroll 4
@@ -838,7 +877,7 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const Pau
       }
       v = (double)(float)v;
     } else {
-      v = d.kind == QSIM_PAULI_GROUP_PAIR ? uniform_entry(d) : d.same;
+      v = d.kind == QSIM_PAULI_GROUP_PAIR ? pair_entry(d, wpar(d.m0), wpar(d.m1)) : d.same;
     }
     asm volatile("" : "+v"(v));                 // one vector value from here on, whatever the kind
     if (v != 0.0) {
@@ -857,59 +896,224 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const Pau
     for (int j = 0; j < C; ++j) x[j] = X[j * rows + (l ^ m)];
     add_group(d, x);
   }
-  for (; g < n_groups; g += U) {
-    float2 x[U][C];
-    PauliGroup d[U];
-    bool need[U];
+  for (; g < n_groups; ++g) {
+    const PauliGroup d = tab[g];
+    if (!needed(d)) continue;
+    const R m = (R)d.xm & (R)(n_rows - 1);
+    float2 x[C];
 #pragma unroll
-    for (int u = 0; u < U; ++u) d[u] = tab[g + u < n_groups ? g + u : n_groups - 1];
-#pragma unroll
-    for (int u = 0; u < U; ++u) need[u] = g + u < n_groups && needed(d[u]);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (!need[u]) continue;
-      const R m = (R)d[u].xm & (R)(n_rows - 1);
-#pragma unroll
-      for (int j = 0; j < C; ++j) x[u][j] = (tc + voff[j])[r ^ m];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (need[u]) add_group(d[u], x[u]);
+    for (int j = 0; j < C; ++j) x[j] = (tc + voff[j])[r ^ m];
+    add_group(d, x);
   }
 #pragma unroll
-  for (int j = 0; j < C; ++j) {
-    if (grp * C + j >= (uint32_t)n_rhs) continue;
-    const uint64_t at = voff[j] + r;
-    const float2 tp = first ? make_float2(0.f, 0.f) : ld2<NT>(tpn + at);
-    const float2 tn = sum[j].next(scale, tp, first != 0);
-    st2<NT>(tpn + at, tn);
-    const float2 v = cmulc(c, tn);
-    float2 a = ld2<NT>(acc + at), k2 = ld2<NT>(comp + at);
-    neu_add(a.x, k2.x, v.x);
-    neu_add(a.y, k2.y, v.y);
-    st2<NT>(acc + at, a);
-    st2<NT>(comp + at, k2);
-  }
+  for (int j = 0; j < C; ++j)
+    if (grp * C + j < (uint32_t)n_rhs)
+      cheb_store<NT>(sum[j], scale, e, X[j * rows + l], tpn, acc, comp, voff[j] + r);
 }
 
-template <typename R, int C, int U>
-static void launch_pauli(hipStream_t s, int n_groups, const void* groups, const void* sm, const void* coef, int n,
-                         int n_rhs, double scale, const void* tc, void* tpn, void* acc, void* comp, float2 c,
-                         int first) {
-  const uint64_t ng = ceil_div((uint64_t)n_rhs, C);
-  const uint64_t blocks = ng * ((1ull << n) / kThreads);
+// One vector: 2^LR rows per thread, 256 apart, in tiles of 256 << LR rows.
+// With one vector to serve, the chain of table loads and scalar parities of a
+// group is what a term waits for, so the groups are looked at side by side:
+// lane i holds group i's record and works out, once per wave and for 64 groups
+// at a time, the wave's part of the parities, the entry where it is the same
+// in the whole wave, and whether the group is needed at all.  The walk over the
+// needed groups then takes scalars from lanes (v_readlane) and waits for T_k
+// only, which it loads for U groups together.  What bounds it: on small states
+// the latency of the walk (a workgroup or less per CU), from 19 qubits on the
+// far loads, most of which another XCD wrote.  us per term of a Heisenberg
+// chain of 12 / 16 / 19 qubits: 6.8 / 8.1 / 17.5 (k_cheb_pauli1 9.5 / 14 / 25;
+// the walk with scalar table loads, as in k_cheb_pauli, 13 / 16 / 29).  A
+// 19-qubit evolution 1820 -> 1300 us with the launches in one call.
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ float flip_signf(float v, uint32_t bit31) {
+  return __uint_as_float(__float_as_uint(v) ^ bit31);
+}
+template <typename R, int LR, int U, bool NT>
+__global__ __launch_bounds__(kThreads) void k_cheb_pauli_one(int n_groups, const PauliGroup* __restrict__ tab,
+                                                             const uint64_t* __restrict__ sm,
+                                                             const double2* __restrict__ coef, int n_bits,
+                                                             double scale, const float2* __restrict__ tc,
+                                                             float2* __restrict__ tpn, float2* __restrict__ acc,
+                                                             float2* __restrict__ comp, ChebAcc e) {
+  constexpr int RR = 1 << LR, b = __builtin_ctz(kThreads) + LR;
+  constexpr uint32_t rows = 1u << b;
+  constexpr uint32_t qm = rows - kThreads;      // the row-of-thread bits
+  __shared__ float4 X4[rows / 2];
+  const float2* X = reinterpret_cast<const float2*>(X4);
+  const uint64_t n_tiles = (1ull << n_bits) >> b;
+  uint64_t tile = gblock<uint64_t>();
+  if (tile >= n_tiles) return;                  // whole workgroup: past the last tile
+  if (n_tiles >= 8) tile = (tile & 7u) * (n_tiles >> 3) + (tile >> 3);   // an eighth of the tiles per XCD
+  const R base = (R)(tile << b);
+  for (uint32_t i = threadIdx.x; i < rows / 2; i += kThreads) X4[i] = reinterpret_cast<const float4*>(tc + base)[i];
+  const uint32_t l = threadIdx.x, lane = l & 63u;
+  const R wbase = base | (R)(l & ~63u);
+  auto wpar = [&](uint64_t m) -> uint32_t {
+    return (uint32_t)(sizeof(R) == 4 ? __popc((uint32_t)wbase & (uint32_t)m) : __popcll((uint64_t)wbase & m)) & 1u;
+  };
+  auto qpar = [&](uint32_t m, int q) -> uint32_t { return (uint32_t)__popc(m & (uint32_t)(q * kThreads)); };
+  RowSum<kAccF64> sum[RR];
+  bool loaded = false;
+  for (int g0 = 0; g0 < n_groups; g0 += 64) {
+    // lane i: group g0 + i
+    const bool valid = (int)lane < n_groups - g0;
+    const PauliGroup d = tab[valid ? g0 + (int)lane : n_groups - 1];
+    const uint32_t reach = (uint32_t)(d.m0 | d.m1);
+    const uint32_t p0 = wpar(d.m0), p1 = wpar(d.m1);
+    const bool pair = d.kind == QSIM_PAULI_GROUP_PAIR, terms = d.kind == QSIM_PAULI_GROUP_TERMS;
+    const float same = (float)d.same, diff = (float)d.diff;      // FP32 values
+    const float vu = pair ? flip_signf(p0 == p1 ? same : diff, p0 << 31) : same;
+    const bool uni = !terms && !(pair && (reach & (63u | qm)));
+    const uint64_t is_uni = __ballot(uni), is_terms = __ballot(terms), is_q = __ballot(pair && (reach & qm));
+    const uint64_t odd0 = __ballot(p0 != 0), odd1 = __ballot(p1 != 0);
+    uint64_t todo = __ballot(valid && !(uni && vu == 0.f));
+    const uint32_t xlo = (uint32_t)d.xm, xhi = (uint32_t)(d.xm >> 32), m0 = (uint32_t)d.m0, m1 = (uint32_t)d.m1;
+    const uint32_t same_b = __float_as_uint(same), diff_b = __float_as_uint(diff), vu_b = __float_as_uint(vu);
+    if (!loaded) __syncthreads();
+    loaded = true;
+    while (todo) {
+      int gi[U];
+      float2 x[U][RR];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        gi[u] = todo ? __builtin_ctzll(todo) : -1;
+        todo &= todo - 1;
+        if (gi[u] < 0) continue;
+        R xm = (R)from_lane(xlo, gi[u]);
+        if constexpr (sizeof(R) == 8) xm |= (R)from_lane(xhi, gi[u]) << 32;
+        if (xm < rows) {
+#pragma unroll
+          for (int q = 0; q < RR; ++q) x[u][q] = X[(l + q * kThreads) ^ (uint32_t)xm];
+        } else {
+#pragma unroll
+          for (int q = 0; q < RR; ++q) x[u][q] = tc[(base | (R)(l + q * kThreads)) ^ xm];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (gi[u] < 0) continue;
+        const int g = gi[u];
+        float v[RR];
+        if (is_uni >> g & 1) {
+          const float w = __uint_as_float(from_lane(vu_b, g));
+#pragma unroll
+          for (int q = 0; q < RR; ++q) v[q] = w;
+        } else {
+          if (is_terms >> g & 1) {
+            const uint32_t t0 = from_lane(d.t0, g), nt = from_lane(d.nt, g);
+            double w[RR];
+#pragma unroll
+            for (int q = 0; q < RR; ++q) w[q] = 0.0;
+            for (uint32_t c0 = 0; c0 < nt; c0 += 64) {
+              const uint32_t left = nt - c0 < 64u ? nt - c0 : 64u;
+              const uint32_t t = t0 + c0 + (lane < left ? lane : left - 1);
+              const uint64_t m = sm[t];
+              const double cs = flip_sign(coef[t].x, wpar(m) << 31);
+              const uint32_t mlo = (uint32_t)m, chi = (uint32_t)__double2hiint(cs), clo = (uint32_t)__double2loint(cs);
+#pragma unroll 4
+              for (uint32_t j = 0; j < left; ++j) {
+                const uint32_t mj = from_lane(mlo, j);
+                const uint32_t s = from_lane(chi, j) ^ ((uint32_t)__popc(lane & mj) << 31);
+                const uint32_t lo = from_lane(clo, j);
+#pragma unroll
+                for (int q = 0; q < RR; ++q) w[q] += __hiloint2double((int)(s ^ (qpar(mj, q) << 31)), (int)lo);
+              }
+            }
+#pragma unroll
+            for (int q = 0; q < RR; ++q) v[q] = (float)w[q];
+          } else {
+            const uint32_t a0 = from_lane(m0, g), a1 = from_lane(m1, g);
+            const float vs = __uint_as_float(from_lane(same_b, g)), vd = __uint_as_float(from_lane(diff_b, g));
+            const uint32_t q0 = (uint32_t)__popc(lane & a0) + (uint32_t)(odd0 >> g & 1);
+            const uint32_t q1 = (uint32_t)__popc(lane & a1) + (uint32_t)(odd1 >> g & 1);
+            if (LR && (is_q >> g & 1)) {
+#pragma unroll
+              for (int q = 0; q < RR; ++q) {
+                const uint32_t r0 = q0 + qpar(a0, q), r1 = q1 + qpar(a1, q);
+                v[q] = flip_signf(((r0 ^ r1) & 1u) ? vd : vs, r0 << 31);
+              }
+            } else {
+              const float w = flip_signf(((q0 ^ q1) & 1u) ? vd : vs, q0 << 31);
+#pragma unroll
+              for (int q = 0; q < RR; ++q) v[q] = w;
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < RR; ++q)            // a row whose entry is zero takes nothing from T_k
+            if (v[q] == 0.f) x[u][q] = make_float2(0.f, 0.f);
+        }
+#pragma unroll
+        for (int q = 0; q < RR; ++q) {
+          asm volatile("" : "+v"(v[q]));          // one vector value from here on, whatever the kind
+          sum[q].add_r((double)v[q], x[u][q]);
+        }
+      }
+    }
+  }
+  if (!loaded) __syncthreads();
+#pragma unroll
+  for (int q = 0; q < RR; ++q)
+    cheb_store<NT>(sum[q], scale, e, X[l + q * kThreads], tpn, acc, comp, (uint64_t)base + l + q * kThreads);
+}
+
+struct PauliTerm {        // a matrix-free Hamiltonian with real entries, and the vectors
+  int n_groups;
+  const PauliGroup* groups;
+  const uint64_t* sm;
+  const double2* coef;
+  int n, n_rhs;
+  double scale;
+};
+
+template <typename R, int LR, int U>
+static void launch_pauli_one(hipStream_t s, const PauliTerm& h, const float2* tc, float2* tpn, float2* acc,
+                             float2* comp, const ChebAcc& e) {
+  auto* kern = nt_for_bytes(32ull << h.n) ? k_cheb_pauli_one<R, LR, U, true> : k_cheb_pauli_one<R, LR, U, false>;
+  hipLaunchKernelGGL(kern, grid1d((1ull << h.n) / (kThreads << LR)), dim3(kThreads), 0, s, h.n_groups, h.groups,
+                     h.sm, h.coef, h.n, h.scale, tc, tpn, acc, comp, e);
+}
+
+template <typename R>
+static void launch_pauli(hipStream_t s, const PauliTerm& h, const float2* tc, float2* tpn, float2* acc, float2* comp,
+                         const ChebAcc& e) {
+  if (h.n_rhs == 1) {
+    // us per evolution of a Heisenberg chain (t = 1, 43 to 70 terms) at 1 / 2 / 4
+    // rows per thread: 12 qubits 420 / 478 / 564, 16 qubits 580 / 670 / 796,
+    // 18 qubits 921 / 929 / 1015, 19 qubits 1313 / 1234 / 1270, 20 qubits 2204 /
+    // 1916 / 1906, 21 qubits 4054 / 3292 / 3183, 22 qubits 7900 / 6143 / 5732
+    // (8 rows: 6258 there); more rows share the work on a group but leave fewer
+    // waves.  Four groups' loads together, two where four rows already are.
+    if (h.n <= 18) launch_pauli_one<R, 0, 4>(s, h, tc, tpn, acc, comp, e);
+    else if (h.n <= 20) launch_pauli_one<R, 1, 4>(s, h, tc, tpn, acc, comp, e);
+    else launch_pauli_one<R, 2, 2>(s, h, tc, tpn, acc, comp, e);
+    return;
+  }
+  const uint64_t ng = ceil_div((uint64_t)h.n_rhs, kPauliVecs);
+  const uint64_t blocks = ng * ((1ull << h.n) / kThreads);
   // T_k, T_{k-1} and the accumulator pair stream together: nontemporal once
   // the four exceed the MALL (20 qubits, 32 right-hand sides: 622 against
   // 659 us; 8, which fit: 171 against 155 us)
-  const bool nt = nt_for_bytes((32ull * n_rhs) << n);
+  const bool nt = nt_for_bytes((32ull * h.n_rhs) << h.n);
   // a group of vectors per XCD while its T_k (32 B a row) is a few L2s large:
   // 16 qubits, 32 right-hand sides 38 against 44 us, 20 qubits 609 against
   // 622; 22 qubits 2890 against 2733 us
-  const int by_rhs = ng % 8 == 0 && n <= 20;
-  auto* kern = nt ? k_cheb_pauli<R, C, U, true> : k_cheb_pauli<R, C, U, false>;
-  hipLaunchKernelGGL(kern, grid1d(blocks), dim3(kThreads), 0, s, n_groups, (const PauliGroup*)groups,
-                     (const uint64_t*)sm, (const double2*)coef, n, n_rhs, by_rhs, scale, (const float2*)tc,
-                     (float2*)tpn, (float2*)acc, (float2*)comp, c, first);
+  const int by_rhs = ng % 8 == 0 && h.n <= 20;
+  auto* kern = nt ? k_cheb_pauli<R, true> : k_cheb_pauli<R, false>;
+  hipLaunchKernelGGL(kern, grid1d(blocks), dim3(kThreads), 0, s, h.n_groups, h.groups, h.sm, h.coef, h.n, h.n_rhs,
+                     by_rhs, h.scale, tc, tpn, acc, comp, e);
+}
+
+static int check_pauli(const PauliTerm& h, const void* t_cur, const void* t_prev_next, const void* acc,
+                       const void* comp) {
+  if (h.n < QSIM_PAULI_BATCH_MIN_QUBITS || h.n > QSIM_MAX_QUBITS)
+    return fail(QSIM_ERANGE, "n_qubits=%d outside %d..%d", h.n, QSIM_PAULI_BATCH_MIN_QUBITS, QSIM_MAX_QUBITS);
+  if (h.n_groups < 0 || h.n_rhs < 1 || h.n_rhs > (1 << 20))
+    return fail(QSIM_EINVAL, "bad sizes (n_groups=%d, n_rhs=%d)", h.n_groups, h.n_rhs);
+  if ((h.n_groups > 0 && (!h.groups || !h.sm || !h.coef)) || !t_cur || !t_prev_next || !acc || !comp)
+    return fail(QSIM_EINVAL, "NULL pointer argument");
+  return QSIM_OK;
 }
 
 __global__ __launch_bounds__(kThreads) void k_cheb_init(float2* __restrict__ acc,
@@ -1068,20 +1272,39 @@ int qsim_cheb_pauli_step(void* stream, int n_qubits, int n_groups, const void* x
 int qsim_cheb_pauli_batch_step(void* stream, int n_qubits, int n_groups, const void* groups, const void* sm,
                                const void* coef, int n_rhs, double scale, const void* t_cur, void* t_prev_next,
                                void* acc, void* comp, double c_re, double c_im, int first) {
-  if (n_qubits < QSIM_PAULI_BATCH_MIN_QUBITS || n_qubits > QSIM_MAX_QUBITS)
-    return fail(QSIM_ERANGE, "n_qubits=%d outside %d..%d", n_qubits, QSIM_PAULI_BATCH_MIN_QUBITS, QSIM_MAX_QUBITS);
-  if (n_groups < 0 || n_rhs < 1 || n_rhs > (1 << 20))
-    return fail(QSIM_EINVAL, "bad sizes (n_groups=%d, n_rhs=%d)", n_groups, n_rhs);
-  if ((n_groups > 0 && (!groups || !sm || !coef)) || !t_cur || !t_prev_next || !acc || !comp)
-    return fail(QSIM_EINVAL, "NULL pointer argument");
+  const PauliTerm h = {n_groups, (const PauliGroup*)groups, (const uint64_t*)sm, (const double2*)coef, n_qubits,
+                       n_rhs, scale};
+  if (int rc = check_pauli(h, t_cur, t_prev_next, acc, comp)) return rc;
   if (((uintptr_t)t_cur & 15u) != 0) return fail(QSIM_EINVAL, "t_cur must be 16-byte aligned");
-  hipStream_t s = as_stream(stream);
-  const float2 c = f2(c_re, c_im);
-  const bool wide = n_qubits > 32, one = n_rhs == 1;
-  auto* launch = one ? (wide ? launch_pauli<uint64_t, 1, 2> : launch_pauli<uint32_t, 1, 2>)
-                     : (wide ? launch_pauli<uint64_t, 4, 1> : launch_pauli<uint32_t, 4, 1>);
-  launch(s, n_groups, groups, sm, coef, n_qubits, n_rhs, scale, t_cur, t_prev_next, acc, comp, c, first);
+  const ChebAcc e = {f2(c_re, c_im), make_float2(0.f, 0.f), first ? kChebFirst : 0};
+  (n_qubits > 32 ? launch_pauli<uint64_t> : launch_pauli<uint32_t>)(as_stream(stream), h, (const float2*)t_cur,
+                                                                    (float2*)t_prev_next, (float2*)acc,
+                                                                    (float2*)comp, e);
   return launch_status("cheb_pauli_batch_step");
+}
+
+int qsim_cheb_pauli_evolve(void* stream, int n_qubits, int n_groups, const void* groups, const void* sm,
+                           const void* coef, int n_rhs, double scale, void* t0, void* t1, void* acc, void* comp,
+                           const double* coeffs, int n_terms) {
+  const PauliTerm h = {n_groups, (const PauliGroup*)groups, (const uint64_t*)sm, (const double2*)coef, n_qubits,
+                       n_rhs, scale};
+  if (int rc = check_pauli(h, t0, t1, acc, comp)) return rc;
+  if (!coeffs) return fail(QSIM_EINVAL, "NULL pointer argument");
+  if (n_terms < 1) return fail(QSIM_EINVAL, "n_terms < 1");
+  if ((((uintptr_t)t0 | (uintptr_t)t1) & 15u) != 0) return fail(QSIM_EINVAL, "t0 and t1 must be 16-byte aligned");
+  auto* launch = n_qubits > 32 ? launch_pauli<uint64_t> : launch_pauli<uint32_t>;
+  float2 *cur = (float2*)t0, *prv = (float2*)t1;
+  for (int k = 1; k <= n_terms; ++k) {
+    ChebAcc e = {f2(coeffs[2 * k], coeffs[2 * k + 1]), f2(coeffs[2 * k - 2], coeffs[2 * k - 1]), 0};
+    if (k == 1) e.mode = kChebFirst | kChebInit;
+    else if (k % 2) e.mode = kChebPair;
+    else if (k < n_terms) e.mode = kChebSkip;
+    if (k == n_terms) e.mode |= kChebLast;
+    launch(as_stream(stream), h, cur, prv, (float2*)acc, (float2*)comp, e);
+    if (int rc = launch_status("cheb_pauli_evolve")) return rc;
+    std::swap(cur, prv);
+  }
+  return QSIM_OK;
 }
 
 int qsim_cheb_init_acc(void* stream, void* acc, void* comp, const void* t, int64_t n, double c_re,

@@ -1,5 +1,6 @@
 """The tiled matrix-free Chebyshev term (qsim_cheb_pauli_batch_step) and its
 group records."""
+import ctypes
 import os
 import sys
 
@@ -137,3 +138,60 @@ def test_tiled_term_checks_its_arguments():
     assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, None, 16, 16, 1, *z) == 1
     assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, 16, 16, 16, 0, *z) == 1
     assert lib.qsim_cheb_pauli_batch_step(None, 10, 1, 16, 16, 16, 1, 1.0, 24, 16, 16, 16, 0.0, 0.0, 0) == 1
+
+
+def dense_terms(n, seed):
+    """More groups than lanes of a wave (X pairs), one of them with more terms
+    than lanes (Z strings)."""
+    rng = np.random.default_rng(seed)
+    pairs = [(i, j) for i in range(n) for j in range(i)]
+
+    def lab(ch, qs):
+        return "".join(ch if n - 1 - p in qs else "I" for p in range(n))
+
+    out = [(lab("Z", q), rng.uniform(-1, 1)) for q in pairs + [(i,) for i in range(n)]]
+    for q in pairs:
+        out += [(lab("X", q), rng.uniform(-1, 1)), (lab("Y", q), rng.uniform(-1, 1))]
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,R,K,make", [(9, 1, 1, mixed_terms), (10, 1, 5, mixed_terms), (12, 1, 4, dense_terms),
+                                        (19, 1, 3, mixed_terms), (21, 1, 2, mixed_terms), (10, 3, 2, mixed_terms),
+                                        (12, 4, 5, dense_terms)])
+def test_whole_series_has_the_bits_of_its_terms(n, R, K, make):
+    """Odd and even term counts, every number of rows per thread: the series in
+    one call equals start, terms and finish by the untiled kernels."""
+    dev = torch.device("cuda", 0)
+    terms = make(n, n)
+    pt = PauliTables([t[0] for t in terms], [t[1] for t in terms], dev)
+    assert pt.groups is not None
+    g = torch.Generator(device=dev).manual_seed(n + R + K)
+    T0 = torch.view_as_complex(torch.randn(R, 1 << n, 2, device=dev, generator=g))
+    if K == 1:
+        T0[0, 5] = complex(float("inf"), 1.0)               # a zero entry takes nothing from it
+    c = np.random.default_rng(K).standard_normal((K + 1, 2)).view(np.complex128).reshape(-1)
+    s = _lib.stream_handle(dev)
+    a, b, acc, comp = T0.clone(), *[torch.full_like(T0, float("nan")) for _ in range(3)]
+    _lib.call("qsim_cheb_pauli_evolve", s, n, *pt.batch_args(), R, 0.1, ptr(a), ptr(b), ptr(acc), ptr(comp),
+              ctypes.c_void_p(c.ctypes.data), K)
+    got = (b if K % 2 else a).cpu().numpy()
+    for j in range(R):
+        cur, prv, acc, comp = T0[j].clone(), *[torch.empty_like(T0[j]) for _ in range(3)]
+        _lib.call("qsim_cheb_init_acc", s, ptr(acc), ptr(comp), ptr(cur), 1 << n, c[0].real, c[0].imag)
+        for k in range(1, K + 1):
+            _lib.call("qsim_cheb_pauli_step", s, n, *pt.step_args(), 0.1, ptr(cur), ptr(prv), ptr(acc), ptr(comp),
+                      c[k].real, c[k].imag, int(k == 1))
+            cur, prv = prv, cur
+        _lib.call("qsim_cheb_finish", s, ptr(prv), ptr(acc), ptr(comp), 1 << n)
+        assert np.array_equal(prv.cpu().numpy(), got[j], equal_nan=True)
+        assert np.isfinite(got[j]).any()
+
+
+def test_series_checks_its_arguments():
+    lib = _lib.load()
+    c = np.zeros(4)
+    call = lambda n=10, g=16, R=1, t0=16, t1=16, cf=c.ctypes.data, K=1: lib.qsim_cheb_pauli_evolve(
+        None, n, 1, g, 16, 16, R, 1.0, t0, t1, 16, 16, cf, K)
+    assert call(n=8) == 2 and call(g=None) == 1 and call(R=0) == 1 and call(cf=None) == 1 and call(K=0) == 1
+    assert call(t0=24) == 1 and call(t1=24) == 1 and call(t1=None) == 1
