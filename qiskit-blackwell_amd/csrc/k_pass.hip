@@ -37,19 +37,25 @@
 // banks whatever the block's qubits are.  The block record holds the swizzled
 // index of each single bit, so an address is an XOR of record entries.
 //
-// What bounds it: the CU's issue of the phases of a block.  At 28 qubits a
-// block takes 190 us on top of the others; copies without one phase show
-// 74 us for the products, 57-74 for the splits (11 VALU instructions per
-// amplitude), 36-68 for the LDS writes and 29 for addresses and LDS reads,
-// nearly additive whatever the waves per SIMD, and a pass 0.42 ms (0.68 for
-// its bytes alone, partly hidden).  Two workgroups of 8 waves per CU (13-qubit
-// tiles) are the best of 4, 8 and 16 waves for states that fill the chip; a
-// 12-qubit tile takes 8 waves for the sake of states of at most 21 qubits, which
-// leave a CU one or two tiles (20 qubits: 175 us against 192 with 4 waves).
-// Loading a set's amplitudes beside the products of the set before it costs
-// registers and measured 208 against 190 us.  The depth-28 SU(4) circuit: 92
-// launches of 5-qubit blocks 76.7 ms, 32 passes of 147 blocks 40.4 ms; depth 24
-// at 24 qubits 3.85 -> 1.75 ms.
+// What bounds it: the vector pipe.  At 28 qubits a set takes 148 VALU
+// instructions (88 of them split its amplitudes, 16 join the accumulators) at 4
+// cycles and 12 products at 32, and the counters show these adding up to all
+// SIMD cycles, at 1.76 GHz: a wave's products do not run beside another's VALU
+// work here, and the tile's bytes (0.68 ms a pass alone) hide behind the two.
+// So only fewer instructions help: LDS addresses without the array's base,
+// slots stored as two amplitudes instead of four selects, scalar bases in
+// global addresses (163 -> 148 a set) took the depth-24 SU(4) circuit at 24
+// qubits from 1752 to 1707 us, depth 28 at 28 qubits from 40.3 to 39.7 ms.
+// Measured and not taken: residues by v_dot2c_f32_bf16 (32 instructions fewer
+// at twice the cycles, no gain), the next tile loaded into registers beside the
+// blocks by workgroups that stay (42.4 ms), consecutive blocks on the same wave
+// bits without the barrier between them (40.5 ms), the next set's amplitudes
+// loaded beside the products (208 us a block against 190).
+// Two workgroups of 8 waves per CU (13-qubit tiles) are the best of 4, 8 and 16
+// waves for states that fill the chip; a 12-qubit tile takes 8 waves for the
+// sake of states of at most 21 qubits, which leave a CU one or two tiles (20
+// qubits: 175 us against 192 with 4 waves).  92 launches of 5-qubit blocks took
+// 76.7 ms for the depth-28 circuit, 32 passes of 143 blocks take 39.7.
 #include "qsim_internal.hpp"
 #include <string.h>
 #include <algorithm>
@@ -105,8 +111,23 @@ __device__ __forceinline__ f32x16 mul_parts(const bf16x8 a[kFrags], const bf16x8
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2 * KA + 1], b[2 * KB + 1], acc, 0, 0, 0);
 }
 
-// One tile of one pass, by a workgroup of W waves.
-template <int M, int W, bool NT>
+// An amplitude at a byte offset of LDS.  The tile is the only thing there and
+// starts at 0, so an offset is an address: through the array's symbol the
+// compiler adds that 0 at every access, after the XORs.
+typedef __attribute__((address_space(3))) f32x2v lds_amp;
+__device__ __forceinline__ float2 lds_get(uint32_t at) {
+  const f32x2v v = *(const lds_amp*)at;
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void lds_put(uint32_t at, float x, float y) {
+  const f32x2v v = {x, y};
+  *(lds_amp*)at = v;
+}
+
+// One tile of one pass, by a workgroup of W waves.  OFF holds the byte offset
+// of a thread's place in a tile: 32 bits up to 29 qubits, so that an address is
+// a scalar base and one register.
+template <int M, int W, bool NT, typename OFF>
 __device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile, const PassGeom& g,
                                           const uint4* __restrict__ blocks, const float4* __restrict__ frags,
                                           int n_blocks) {
@@ -115,42 +136,42 @@ __device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile
   constexpr int TB = __builtin_ctz(T);                // slot bits that run over the threads
   constexpr int SETS = 1 << (M - 9);
   constexpr int SPW = SETS >= W ? SETS / W : 1;       // sets per wave
-  extern __shared__ float4 X4[];
-  char* Xb = reinterpret_cast<char*>(X4);
   const int tid = threadIdx.x;
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint64_t base = tile;
 #pragma unroll
   for (int j = 0; j < M; ++j) base = ins0(base, g.tq(j));
-  base >>= 1;                                         // in slots; the first tile qubit is 0
-  uint64_t toff = 0;
+  OFF toff = 0;
 #pragma unroll
-  for (int j = 0; j < TB; ++j) toff |= (uint64_t)((tid >> j) & 1) << (g.tq(j + 1) - 1);
-  const uint32_t tsw = pass_sw(2u * tid);
-  uint64_t koff[SLOTS];
+  for (int j = 0; j < TB; ++j) toff |= (OFF)((tid >> j) & 1) << (g.tq(j + 1) + 3);
+  const uint32_t tsw = pass_sw(2u * tid) * 8u;
+  auto place = [&](int k) -> float4* {                // slot k of the thread; the first tile qubit is 0
+    uint64_t at = base;
 #pragma unroll
-  for (int k = 0; k < SLOTS; ++k) {
-    koff[k] = base;
-#pragma unroll
-    for (int j = TB; j < M - 1; ++j) koff[k] |= (uint64_t)((k >> (j - TB)) & 1) << (g.tq(j + 1) - 1);
-  }
+    for (int j = TB; j < M - 1; ++j) at |= (uint64_t)((k >> (j - TB)) & 1) << g.tq(j + 1);
+    return reinterpret_cast<float4*>(reinterpret_cast<char*>(st) + at * 8u + toff);
+  };
   {
     float4 v[SLOTS];
 #pragma unroll
-    for (int k = 0; k < SLOTS; ++k) v[k] = ld4<NT>(st + (koff[k] + toff));
+    for (int k = 0; k < SLOTS; ++k) v[k] = ld4<NT>(place(k));
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) {
-      // an odd swizzled index swaps the two amplitudes of a slot
-      const uint32_t p = tsw ^ pass_sw(2u * k * T);
-      const bool odd = p & 1;
-      X4[p >> 1] = make_float4(odd ? v[k].z : v[k].x, odd ? v[k].w : v[k].y, odd ? v[k].x : v[k].z,
-                               odd ? v[k].y : v[k].w);
+      // the slot's two amplitudes are neighbours in LDS, in either order
+      const uint32_t p = tsw ^ pass_sw(2u * k * T) * 8u;
+      lds_put(p, v[k].x, v[k].y);
+      lds_put(p ^ 8u, v[k].z, v[k].w);
     }
   }
   bf16x8 a[kFrags];
+  auto load_frags = [&](int b) {
+    // a base in the middle: every fragment within an instruction's offset of it
+    const float4* fb = frags + (size_t)b * (64 * kFrags) + 64 * (kFrags / 2);
 #pragma unroll
-  for (int q = 0; q < kFrags; ++q) a[q] = as_frag(frags[q * 64 + lane]);
+    for (int q = 0; q < kFrags; ++q) a[q] = as_frag((fb + 64 * (q - kFrags / 2))[lane]);
+  };
+  load_frags(0);
   uint4 d0 = blocks[0], d1 = blocks[1];
   __syncthreads();
   for (int b = 0; b < n_blocks; ++b) {
@@ -182,7 +203,7 @@ __device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile
       for (int i = 0; i < SPW; ++i) {
         float2 x[8];
 #pragma unroll
-        for (int s = 0; s < 8; ++s) x[s] = *reinterpret_cast<const float2*>(Xb + (sbase[i] ^ ro[s]));
+        for (int s = 0; s < 8; ++s) x[s] = lds_get(sbase[i] ^ ro[s]);
         bf16x8 bp[kFrags];
         split_set(x, bp);
         f32x16 big = {0.f}, small = {0.f};
@@ -194,13 +215,11 @@ __device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile
         small = mul_parts<1, 0>(a, bp, small);
         if (i + 1 == SPW) {
           // the next block's fragments travel while the results are written
-#pragma unroll
-          for (int q = 0; q < kFrags; ++q) a[q] = as_frag(frags[(size_t)nb * (64 * kFrags) + q * 64 + lane]);
+          load_frags(nb);
         }
 #pragma unroll
         for (int s = 0; s < 8; ++s)
-          *reinterpret_cast<float2*>(Xb + (sbase[i] ^ ro[s])) =
-              make_float2(big[2 * s] + small[2 * s], big[2 * s + 1] + small[2 * s + 1]);
+          lds_put(sbase[i] ^ ro[s], big[2 * s] + small[2 * s], big[2 * s + 1] + small[2 * s + 1]);
       }
     }
     __syncthreads();
@@ -209,20 +228,19 @@ __device__ __forceinline__ void pass_tile(float4* __restrict__ st, uint64_t tile
   }
 #pragma unroll
   for (int k = 0; k < SLOTS; ++k) {
-    const uint32_t p = tsw ^ pass_sw(2u * k * T);
-    const bool odd = p & 1;
-    const float4 v = X4[p >> 1];
-    st4<NT>(st + (koff[k] + toff), make_float4(odd ? v.z : v.x, odd ? v.w : v.y, odd ? v.x : v.z, odd ? v.y : v.w));
+    const uint32_t p = tsw ^ pass_sw(2u * k * T) * 8u;
+    const float2 u = lds_get(p), w = lds_get(p ^ 8u);
+    st4<NT>(place(k), make_float4(u.x, u.y, w.x, w.y));
   }
 }
 
-template <int M, int W, bool NT>
+template <int M, int W, bool NT, typename OFF>
 __global__ __launch_bounds__(64 * W, 4) void k_pass(float4* __restrict__ st, uint64_t n_tiles, PassGeom g,
                                                     const uint4* __restrict__ blocks,
                                                     const float4* __restrict__ frags, int n_blocks) {
   const uint64_t tile = gblock<uint64_t>();
   if (tile >= n_tiles) return;                        // whole workgroup: past the last tile
-  pass_tile<M, W, NT>(st, tile, g, blocks, frags, n_blocks);
+  pass_tile<M, W, NT, OFF>(st, tile, g, blocks, frags, n_blocks);
 }
 
 // One pass of each of n_recs states in one launch: workgroup b takes the tile
@@ -254,10 +272,10 @@ __global__ __launch_bounds__(64 * kBatchWaves, 4) void k_pass_batch(const qsim_p
   const float4* fr = frags + (size_t)rec.first_block * (64 * kFrags);
   const uint64_t tile = b - rec.tile_begin;
   switch (rec.tile_bits) {
-    case 10: pass_tile<10, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
-    case 11: pass_tile<11, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
-    case 12: pass_tile<12, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
-    default: pass_tile<13, kBatchWaves, false>(st, tile, g, bl, fr, rec.n_blocks); break;
+    case 10: pass_tile<10, kBatchWaves, false, uint64_t>(st, tile, g, bl, fr, rec.n_blocks); break;
+    case 11: pass_tile<11, kBatchWaves, false, uint64_t>(st, tile, g, bl, fr, rec.n_blocks); break;
+    case 12: pass_tile<12, kBatchWaves, false, uint64_t>(st, tile, g, bl, fr, rec.n_blocks); break;
+    default: pass_tile<13, kBatchWaves, false, uint64_t>(st, tile, g, bl, fr, rec.n_blocks); break;
   }
 }
 
@@ -266,12 +284,11 @@ static void launch_pass(hipStream_t s, void* state, int n, const PassGeom& g, co
                         const void* frags, int n_blocks) {
   const uint64_t tiles = 1ull << (n - M);
   const size_t lds = sizeof(float2) << M;
-  if (nt_for_qubits(n))
-    hipLaunchKernelGGL((k_pass<M, W, true>), grid1d(tiles), dim3(64 * W), lds, s, (float4*)state, tiles, g,
-                       (const uint4*)blocks, (const float4*)frags, n_blocks);
-  else
-    hipLaunchKernelGGL((k_pass<M, W, false>), grid1d(tiles), dim3(64 * W), lds, s, (float4*)state, tiles, g,
-                       (const uint4*)blocks, (const float4*)frags, n_blocks);
+  auto* kern = n > 29             ? k_pass<M, W, true, uint64_t>
+               : nt_for_qubits(n) ? k_pass<M, W, true, uint32_t>
+                                  : k_pass<M, W, false, uint32_t>;
+  hipLaunchKernelGGL(kern, grid1d(tiles), dim3(64 * W), lds, s, (float4*)state, tiles, g, (const uint4*)blocks,
+                     (const float4*)frags, n_blocks);
 }
 
 // Host check of one record: the swizzled indices of m distinct tile bits.
