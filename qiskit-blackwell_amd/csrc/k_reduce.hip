@@ -217,36 +217,36 @@ __device__ __forceinline__ double wave_incl_scan(double v, int lane) {
   return v;
 }
 
-__device__ __forceinline__ void leaf_scan(const float4* __restrict__ leaf, int lane, int nl,
-                                          LeafScan& L) {
-  L.q[0] = L.q[1] = L.q[2] = L.q[3] = 0.0;
-  if (2 * lane < nl) {
-    const float4 v0 = leaf[lane];
-    L.q[0] = p2(lo2(v0)); L.q[1] = p2(hi2(v0));
-  }
-  if (128 + 2 * lane < nl) {
-    const float4 v1 = leaf[64 + lane];
-    L.q[2] = p2(lo2(v1)); L.q[3] = p2(hi2(v1));
-  }
-  const double pa = L.q[0] + L.q[1];
-  const double ia = wave_incl_scan(pa, lane);
-  double prev = __shfl_up(ia, 1, 64);
-  double base = lane == 0 ? 0.0 : prev;
-  L.c[0] = base + L.q[0];
+// The amplitudes of a leaf, one slot of either half per lane.
+struct LeafSlots {
+  float4 v0, v1;
+};
+__device__ __forceinline__ LeafSlots leaf_load(const float4* __restrict__ leaf, int lane, int nl) {
+  LeafSlots s = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+  if (2 * lane < nl) s.v0 = leaf[lane];
+  if (128 + 2 * lane < nl) s.v1 = leaf[64 + lane];
+  return s;
+}
+__device__ __forceinline__ void leaf_scan_lo(const LeafSlots& s, int lane, LeafScan& L) {
+  L.q[0] = p2(lo2(s.v0)); L.q[1] = p2(hi2(s.v0));
+  const double ia = wave_incl_scan(L.q[0] + L.q[1], lane);
+  const double prev = __shfl_up(ia, 1, 64);
+  L.c[0] = (lane == 0 ? 0.0 : prev) + L.q[0];
   L.c[1] = L.c[0] + L.q[1];
+}
+__device__ __forceinline__ void leaf_scan_hi(const LeafSlots& s, int lane, LeafScan& L) {
+  L.q[2] = p2(lo2(s.v1)); L.q[3] = p2(hi2(s.v1));
   const double half = __shfl(L.c[1], 63, 64);
-  const double pb = L.q[2] + L.q[3];
-  const double ib = wave_incl_scan(pb, lane);
-  prev = __shfl_up(ib, 1, 64);
-  base = half + (lane == 0 ? 0.0 : prev);
-  L.c[2] = base + L.q[2];
+  const double ib = wave_incl_scan(L.q[2] + L.q[3], lane);
+  const double prev = __shfl_up(ib, 1, 64);
+  L.c[2] = half + (lane == 0 ? 0.0 : prev) + L.q[2];
   L.c[3] = L.c[2] + L.q[3];
 }
 
 // Leaf totals: one wave per leaf, the four |a|^2 of each lane (the
-// leaf_scan layout, 1 KiB per load) summed across the wave by the fixed
+// scan's layout, 1 KiB per load) summed across the wave by the fixed
 // butterfly of wave_sum.  The in-leaf search recomputes the cumulative sums
-// with leaf_scan; where rounding makes the two disagree, an x past the scan's
+// with leaf_scan_lo and _hi; where rounding makes the two disagree, an x past the scan's
 // total takes the leaf's last nonzero amplitude.
 template <bool NT>
 __global__ __launch_bounds__(kThreads) void k_leaf_totals(const float4* __restrict__ st,
@@ -386,44 +386,59 @@ __device__ __forceinline__ int64_t leaf_last_nonzero(const LeafScan& L, int lane
 }
 
 // Index sampled for x = u * total by one wave.  Leaf j = largest j with
-// pre[j] <= x; a leaf with zero total reached by rounding steps back to the
+// pre[j] <= x, found by 64 probes a round, one per lane: a binary search waits
+// for 16 loads in a row at 24 qubits, this for three.  A leaf with zero total reached by rounding steps back to the
 // previous nonzero leaf, and an x past the leaf's own total (rounding again)
 // takes the leaf's last nonzero amplitude, so a zero-probability index is
 // never returned.
 __device__ __forceinline__ int64_t sample_one(const float4* __restrict__ st, uint64_t n_amps,
                                               uint64_t nl, const double* __restrict__ pre,
                                               const double* __restrict__ tot, double x, int lane) {
-  uint64_t lo = 0, hi = nl - 1;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi + 1) >> 1;
-    if (pre[mid] <= x) lo = mid; else hi = mid - 1;
+  uint64_t leaf = 0, n = nl;              // among leaf .. leaf + n - 1
+  while (n > 1) {
+    const uint64_t step = (n + 63) >> 6, off = (uint64_t)lane * step;
+    const uint64_t below = __ballot(off < n && pre[off < n ? leaf + off : leaf] <= x) | 1u;
+    const uint64_t at = (uint64_t)(63 - __clzll((unsigned long long)below)) * step;
+    leaf += at;
+    n = n - at < step ? n - at : step;
   }
-  uint64_t leaf = lo;
-  while (leaf > 0 && !(tot[leaf] > 0.0)) --leaf;
-  const double y = x - pre[leaf];
   const int nla = (int)(n_amps < (uint64_t)kLeaf ? n_amps : kLeaf);
+  LeafSlots S = leaf_load(st + leaf * (kLeaf / 2), lane, nla);   // beside its total, which is rarely 0
+  if (leaf > 0 && !(tot[leaf] > 0.0)) {
+    do --leaf;
+    while (leaf > 0 && !(tot[leaf] > 0.0));
+    S = leaf_load(st + leaf * (kLeaf / 2), lane, nla);
+  }
+  const double y = x - pre[leaf];
+  // smallest index with nonzero probability whose cumulative exceeds y: first
+  // half (amplitudes 2l, 2l+1), then, if it is not there, second half (128 + 2l,
+  // 129 + 2l)
   LeafScan L;
-  leaf_scan(st + leaf * (kLeaf / 2), lane, nla, L);
-  // smallest index with nonzero probability whose cumulative exceeds y:
-  // first half (amplitudes 2l, 2l+1), then second half (128 + 2l, 129 + 2l)
+  leaf_scan_lo(S, lane, L);
   const bool h0 = L.q[0] > 0.0 && L.c[0] > y, h1 = L.q[1] > 0.0 && L.c[1] > y;
-  const bool h2 = L.q[2] > 0.0 && L.c[2] > y, h3 = L.q[3] > 0.0 && L.c[3] > y;
-  const uint64_t hit_lo = __ballot(h0 || h1), hit_hi = __ballot(h2 || h3);
+  const uint64_t hit_lo = __ballot(h0 || h1);
   int64_t local;
   if (hit_lo) {
     const int fl = __ffsll((unsigned long long)hit_lo) - 1;
     local = 2 * fl + __shfl(h0 ? 0 : 1, fl, 64);
-  } else if (hit_hi) {
-    const int fl = __ffsll((unsigned long long)hit_hi) - 1;
-    local = 128 + 2 * fl + __shfl(h2 ? 0 : 1, fl, 64);
   } else {
-    local = leaf_last_nonzero(L, lane);
-    if (local < 0) local = 0;  // all-zero state: index 0 (as the reference)
+    leaf_scan_hi(S, lane, L);
+    const bool h2 = L.q[2] > 0.0 && L.c[2] > y, h3 = L.q[3] > 0.0 && L.c[3] > y;
+    const uint64_t hit_hi = __ballot(h2 || h3);
+    if (hit_hi) {
+      const int fl = __ffsll((unsigned long long)hit_hi) - 1;
+      local = 128 + 2 * fl + __shfl(h2 ? 0 : 1, fl, 64);
+    } else {
+      local = leaf_last_nonzero(L, lane);
+      if (local < 0) local = 0;  // all-zero state: index 0 (as the reference)
+    }
   }
   return (int64_t)(leaf * kLeaf) + local;
 }
 
-// One wave per shot.
+// One wave per shot.  What bounds it: the latency of the probes and of the leaf,
+// then the lane exchanges of the scans, of which the second half's runs only
+// where the first has no hit.  65536 shots of 24 qubits 72 -> 40 us.
 __global__ __launch_bounds__(kThreads) void k_sample(const float4* __restrict__ st, uint64_t n_amps,
                                                      uint64_t nl, const double* __restrict__ pre,
                                                      const double* __restrict__ tot,
