@@ -205,19 +205,22 @@ static void launch_expect_kind(hipStream_t s, const void* state, int n, uint64_t
 // tile after tile; slots are added in order at the end, so sums are
 // deterministic as before.
 //
-// What bounds it: FP64 issue (14 of the 20 vector instructions per 64 slots of
-// a group of one term are FP64, at about 4.4 cycles each), then the tile loads,
-// which do not overlap it.  The 93 terms of a Heisenberg chain, plain passes
-// (two launches and a read of the state per group) -> tiled passes: 12 / 16 /
-// 20 / 24 / 28 qubits 151 / 245 / 302 / 1208 / 18600 -> 27 / 44 / 43 / 256 /
-// 4000 us.  Measured and not taken: the next tile loaded into registers during
-// the evaluation 4290 us, tiles of 2^12 at 256 threads 4556, 1024 threads 4675
-// (two parts a group; 512 threads there 4713).
+// What bounds it: vector issue (busy 59 % of the time before groups shared
+// units, 29 % of it conversions to FP64), then the tile loads, which do not
+// overlap it.  The 4 n - 3 terms of a Heisenberg chain, plain passes (two
+// launches and a read of the state per group) -> tiled passes -> units of two
+// groups: 20 / 22 / 24 / 26 qubits 302 / - / 1208 / - -> 43 / 83 / 254 / 975 ->
+// 38.5 / 72 / 212 / 804 us; 12 and 16 qubits 151 and 245 -> 27 and 38.  Measured
+// and not taken, at 28 qubits and 4000 us: the next tile loaded into registers
+// during the evaluation 4290 us, tiles of 2^12 at 256 threads 4556, 1024 threads
+// 4675 (two parts a group; 512 threads there 4713).
 struct ExpGroup {
   uint16_t x;                     // tile-local x mask
   uint8_t h, im;                  // its highest bit; Im(zc) instead of Re(zc)
   uint16_t t0, nt;                // terms [t0, t0 + nt), nt <= kExpMaxTerms
   uint16_t zl[4];                 // tile-local z masks of the first four
+  uint16_t x2;                    // not 0: two groups, the second with this x mask (exp_unit2)
+  uint8_t lo, hi;                 // their pivot bits, lo < hi
 };
 struct ExpTerm {
   uint64_t z;                     // z mask outside the tile
@@ -231,13 +234,17 @@ constexpr int kPassWaves = kPassThreads / 64, kExpTileMax = 13, kExpTileMin = 10
 // 49 us, 28 qubits 340 against 635; a single group stays on the plain pass.
 constexpr int kPassMinGroups = 2;
 constexpr size_t kPassWindow = 2048;   // groups looked at per pass: planning stays linear in their number
+// Smallest state whose groups share units: energies of chains of 12 / 14 / 18
+// qubits 27.3 / 39.4 / 39.6 us apart against 29.4 / 40.5 / 40.8 joined, 20 / 22 /
+// 24 / 26 qubits 43 / 83 / 254 / 975 against 38.5 / 72 / 212 / 804.
+constexpr int kJoinMinQubits = 20;
 struct ExpPass {
   uint32_t tq[4];                 // tile qubits, ascending, one byte each; the first four are 0..3
   int n_groups, n_terms, seg;
   ExpGroup g[kPassGroups];
   ExpTerm t[kPassTerms];
 };
-static_assert(sizeof(ExpPass) <= 3584, "kernel arguments");
+static_assert(sizeof(ExpPass) <= 3712, "kernel arguments");
 __host__ __device__ inline int exp_tq(const ExpPass& a, int j) { return (int)((a.tq[j >> 2] >> (8 * (j & 3))) & 255u); }
 
 // Sums of a unit kept per term: the lanes are added over the lane bits whose
@@ -247,6 +254,19 @@ constexpr int kSlotLanes = 4;
 
 // Kinds of a group: x = 0; x = 1 (pairs inside a slot); x > 1 even; x > 1 odd.
 enum { kDiag, kInSlot, kPair, kPairSwap };
+
+// Adds a unit's lane sums of term j, with its lane and tile signs, to its slot.
+__device__ __forceinline__ void exp_unit_sum(const ExpPass& a, const ExpGroup& g, int j, double acc, uint32_t il,
+                                             uint64_t base, uint32_t lane, double* slot) {
+  const ExpTerm t = a.t[g.t0 + j];
+  const int minus = (__popc(il & (uint32_t)(t.zl >> 1)) + __popcll(base & t.z)) & 1;
+  double r = acc * (double)(minus ? -t.fac : t.fac);
+  r += lane_xor(r, 1);
+  r += lane_xor(r, 2);
+  r += lane_xor(r, 8);
+  r += lane_xor(r, 32);
+  if ((lane & 0x2b) == 0) slot[(j << a.seg) * kSlotLanes + (lane >> 4) * 2 + (lane >> 2 & 1)] += r;
+}
 
 // A unit's sums for its NT terms: steps of 64 slots from slot step p0 on.
 template <int NT, bool IM, int KIND>
@@ -298,15 +318,68 @@ __device__ __forceinline__ void exp_unit(const char* Xb, const ExpPass& a, const
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     if (j >= g.nt) continue;
-    const ExpTerm t = a.t[g.t0 + j];
-    const int minus = (__popc(il & (uint32_t)(t.zl >> 1)) + __popcll(base & t.z)) & 1;
-    double r = acc[j] * (double)(minus ? -t.fac : t.fac);
-    r += lane_xor(r, 1);
-    r += lane_xor(r, 2);
-    r += lane_xor(r, 8);
-    r += lane_xor(r, 32);
-    if ((lane & 0x2b) == 0) slot[(j << a.seg) * kSlotLanes + (lane >> 4) * 2 + (lane >> 2 & 1)] += r;
+    exp_unit_sum(a, g, j, acc[j], il, base, lane, slot);
   }
+}
+
+// A unit of two groups (even x masks, real parts, NA and NB terms): the four
+// slots i, i ^ x, i ^ x2 and i ^ x ^ x2 hold two pairs of either group, so
+// four slots are converted to FP64 for four pairs, where two units convert four
+// for two.  i runs over the slots with both pivot bits clear; the sign of the
+// second pair of a group is that of the first times the other mask's.
+template <int NA, int NB>
+__device__ __forceinline__ void exp_unit2(const char* Xb, const ExpPass& a, const ExpGroup g, uint32_t p0,
+                                          uint32_t steps, uint64_t base, uint32_t lane, double* slot) {
+  constexpr int U = 2, NT = NA + NB;
+  auto clear = [&](uint32_t p) -> uint32_t { return ins0(ins0(p, (int)g.lo - 1), (int)g.hi - 1); };
+  const uint32_t il = clear(lane), la = il * 16;
+  const uint32_t xa = (g.x >> 1) * 16u, xb = (g.x2 >> 1) * 16u;
+  double acc[NT], c1[NT], c2[NT];
+  uint64_t neg[NT];                       // bit k: the wave sign of step k is -1
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const uint32_t z = g.zl[j];
+    acc[j] = 0.0;
+    c1[j] = (z & 1) ? -1.0 : 1.0;
+    c2[j] = (__popc(z & (j < NA ? g.x2 : g.x)) & 1) ? -1.0 : 1.0;
+    neg[j] = __ballot(__popc(clear((p0 + lane) * 64) & (z >> 1)) & 1);
+  }
+  auto dot = [](const double (&x)[4], const double (&y)[4], int e) -> double {
+    return x[2 * e] * y[2 * e] + x[2 * e + 1] * y[2 * e + 1];
+  };
+  for (uint32_t k0 = 0; k0 < steps; k0 += U) {
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const uint32_t iw = clear((p0 + k0 + q) * 64) * 16;
+      auto slot_at = [&](uint32_t x, double (&d)[4]) {
+        const float4 v = *reinterpret_cast<const float4*>(Xb + (la ^ (iw ^ x)));
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+      };
+      double v0[4], va[4], vb[4], vc[4];
+      slot_at(0, v0);
+      slot_at(xa, va);
+      slot_at(xb, vb);
+      slot_at(xa ^ xb, vc);
+      double p[2][2], r[2][2];              // first and second pair of either group, per amplitude of a slot
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        p[0][e] = dot(v0, va, e);
+        r[0][e] = dot(vb, vc, e);
+        p[1][e] = dot(v0, vb, e);
+        r[1][e] = dot(va, vc, e);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int b = j < NA ? 0 : 1;
+        const uint32_t m = (uint32_t)(neg[j] >> k0);
+        const double t = __builtin_fma(c1[j], __builtin_fma(c2[j], r[b][1], p[b][1]),
+                                       __builtin_fma(c2[j], r[b][0], p[b][0]));
+        acc[j] = __builtin_fma(__hiloint2double((m >> q & 1u) ? (int)0xbff00000 : 0x3ff00000, 0), t, acc[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) exp_unit_sum(a, g, j, acc[j], il, base, lane, slot);
 }
 
 template <int M, bool NTL>
@@ -350,7 +423,7 @@ __global__ __launch_bounds__(kPassThreads) void k_expect_tile(ExpPass args, cons
       const ExpGroup g = next;
       next = group(u + kPassWaves);
       const uint32_t part_no = u & ((1u << a.seg) - 1u);
-      const uint32_t steps = (1u << (g.x > 1 ? M - 8 : M - 7)) >> a.seg;
+      const uint32_t steps = (1u << (g.x2 ? M - 9 : g.x > 1 ? M - 8 : M - 7)) >> a.seg;
       double* slot = slots + (((uint32_t)g.t0 << a.seg) + part_no) * kSlotLanes;
 #define QSIM_UNIT(NT, IM, KIND) exp_unit<NT, IM, KIND>(Xb, a, g, part_no * steps, steps, base, lane, slot)
 #define QSIM_UNIT_NT(IM, KIND)                 \
@@ -359,7 +432,12 @@ __global__ __launch_bounds__(kPassThreads) void k_expect_tile(ExpPass args, cons
     else if (g.nt == 2) QSIM_UNIT(2, IM, KIND); \
     else QSIM_UNIT(8, IM, KIND);               \
   } while (0)
-      if (g.x == 0) {
+      if (g.x2) {
+        const uint32_t s0 = part_no * steps;
+        if (g.nt == 2) exp_unit2<1, 1>(Xb, a, g, s0, steps, base, lane, slot);
+        else if (g.nt == 3) exp_unit2<1, 2>(Xb, a, g, s0, steps, base, lane, slot);
+        else exp_unit2<2, 2>(Xb, a, g, s0, steps, base, lane, slot);
+      } else if (g.x == 0) {
         if (g.nt <= 4) QSIM_UNIT(4, false, kDiag);
         else QSIM_UNIT(8, false, kDiag);
       } else if (g.x == 1) {
@@ -475,24 +553,48 @@ static int expectation_impl(hipStream_t s, const void* state, int n, int64_t n_t
     ExpPass a = {};
     uint64_t rest = tile;
     for (int j = 0; j < m; ++j, rest &= rest - 1) a.tq[j >> 2] |= (uint32_t)__builtin_ctzll(rest) << (8 * (j & 3));
-    a.n_groups = (int)in.size();
     a.n_terms = terms;
-    // the fewest parts that give each wave a unit (28 qubits, 93 terms: 3.99 ms
-    // with one part, 4.59 with two, 4.90 with four; 2 groups: 355 us with two
-    // parts, 340 with four), and at least 4 steps a unit
-    a.seg = std::min(a.n_groups >= kPassWaves ? 0 : a.n_groups >= kPassWaves / 2 ? 1 : 2, m - 10);
     int t = 0;
-    for (size_t i = 0; i < in.size(); ++i) {
-      TermGroup& g = groups[in[i]];
-      const uint32_t x = pack_bits(g.x, tile);
-      a.g[i] = {(uint16_t)x, (uint8_t)(x ? 31 - __builtin_clz(x) : 0), (uint8_t)g.im, (uint16_t)t, (uint16_t)g.cnt, {}};
-      for (int j = 0; j < g.cnt; ++j, ++t) {
+    auto add_terms = [&](ExpGroup& e, TermGroup& g) {
+      for (int j = 0; j < g.cnt; ++j, ++t, ++e.nt) {
         const int64_t k = order[g.beg + j];
         a.t[t] = {zm[k] & ~tile, (uint16_t)pack_bits(zm[k] & tile, tile), (int16_t)pair_factor(g.x, zm[k]), (int32_t)k};
-        if (j < 4) a.g[i].zl[j] = a.t[t].zl;
+        if (e.nt < 4) e.zl[e.nt] = a.t[t].zl;
       }
       g.done = true;
+    };
+    // groups of one or two terms that share a unit, in pairs as they come, where
+    // there are tiles enough to keep the chip busy
+    auto joins = [&](const TermGroup& g) {
+      return n >= kJoinMinQubits && g.x && !(g.x & 1) && !g.im && g.cnt <= 2;
+    };
+    for (size_t i = 0; i < in.size(); ++i) {
+      TermGroup* g = &groups[in[i]];
+      if (g->done) continue;
+      TermGroup* other = nullptr;
+      for (size_t k = i + 1; k < in.size() && joins(*g) && !other; ++k)
+        if (!groups[in[k]].done && joins(groups[in[k]])) other = &groups[in[k]];
+      if (other && other->cnt < g->cnt) std::swap(g, other);
+      ExpGroup& e = a.g[a.n_groups++];
+      const uint32_t x = pack_bits(g->x, tile);
+      e.x = (uint16_t)x;
+      e.h = (uint8_t)(x ? 31 - __builtin_clz(x) : 0);
+      e.im = (uint8_t)g->im;
+      e.t0 = (uint16_t)t;
+      add_terms(e, *g);
+      if (other) {
+        const uint32_t x2 = pack_bits(other->x, tile), y = x2 >> e.h & 1 ? x2 ^ x : x2;
+        const int h2 = 31 - __builtin_clz(y);
+        e.x2 = (uint16_t)x2;
+        e.lo = (uint8_t)std::min<int>(e.h, h2);
+        e.hi = (uint8_t)std::max<int>(e.h, h2);
+        add_terms(e, *other);
+      }
     }
+    // the fewest parts that give each wave a unit (28 qubits, 93 terms: 3.99 ms
+    // with one part, 4.59 with two, 4.90 with four; 2 groups: 355 us with two
+    // parts, 340 with four), and at least 4 steps a unit of one group
+    a.seg = std::min(a.n_groups >= kPassWaves ? 0 : a.n_groups >= kPassWaves / 2 ? 1 : 2, m - 10);
     switch (m) {
       case 10: launch_expect_tile<10>(s, state, n, a, ws, out); break;
       case 11: launch_expect_tile<11>(s, state, n, a, ws, out); break;

@@ -50,3 +50,34 @@ def test_tiled_expectations_match_numpy(n):
     tol = 2.0 * 2.0 ** (n - 53) * float(np.vdot(p64, p64).real)
     assert np.max(np.abs(got - np.array(want))) <= tol
     assert np.array_equal(bk.expectation_paulis(st, xs, zs).cpu().numpy(), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,odd", [(20, 0), (20, 1), (22, 0)])
+def test_groups_that_share_a_unit_match_numpy(n, odd):
+    """Even masks of one and two terms in every combination: masks that hold
+    each other's highest bit, neighbours and far ones, z with bit 0, on the
+    other mask's qubits and outside the tile, two Y; an even and an odd number
+    of groups, beside some that share none.  Tolerance as above."""
+    import blackwell_kernels as bk
+    rng = np.random.default_rng(n + odd)
+    hi = 1 << (n - 1)
+    masks = [(2, 1), (4, 2), (6, 2), (10, 1), (12, 2), (8, 2), (hi, 1), (hi | 2, 1), (3 << 9, 2), (1 << 10, 1)]
+    terms = [(0, 5), (0, hi | 1), (3, 0), (2, 2), (1, 8)]
+    for x, cnt in masks + [(hi | 4, 1)] * odd:
+        for _ in range(cnt):
+            z = int(rng.integers(0, 1 << n))
+            while bin(z & x).count("1") & 1 or (x, z) in terms:
+                z = int(rng.integers(0, 1 << n))
+            terms.append((x, z))
+    psi = (rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)).astype(np.complex64)
+    xs, zs = [t[0] for t in terms], [t[1] for t in terms]
+    got = bk.expectation_paulis(torch.from_numpy(psi).to("cuda:0"), xs, zs).cpu().numpy()
+    p64 = psi.astype(np.complex128)
+    i = np.arange(1 << n)
+    for (x, z), v in zip(terms, got):
+        par = (i ^ x) & z
+        for sh in (16, 8, 4, 2, 1):
+            par ^= par >> sh
+        want = (1j ** (bin(x & z).count("1") % 4) * np.vdot(p64, np.where(par & 1, -1, 1) * p64[i ^ x])).real
+        assert abs(v - want) <= 2.0 * 2.0 ** (n - 53) * float(np.vdot(p64, p64).real), (x, z)
