@@ -206,11 +206,12 @@ class CompiledCircuit:
 
     # ---------------------------------------------------------------- tuning
     def tuned_mode(self, device):
-        """The fastest execution mode for this circuit on `device`, measured
-        once: every applicable mode runs once to warm up and TUNE_REPS times
-        timed with HIP events on the launch stream, from |0...0>.  Above 13
-        qubits the candidates include LDS tile programs of several tile
-        shapes ("tiles/<tile qubits>/<low qubits>")."""
+        """The fastest of the plain, LDS and one-launch-per-block modes for this
+        circuit on `device`, measured once: each runs once to warm up and
+        TUNE_REPS times timed with HIP events on the launch stream, from
+        |0...0>.  Above 13 qubits the candidates include LDS tile programs of
+        several tile shapes ("tiles/<tile qubits>/<low qubits>").  Block passes
+        are not among them: "auto" picks those by rule."""
         key = str(device)
         if key in self._tuned:
             return self._tuned[key]
