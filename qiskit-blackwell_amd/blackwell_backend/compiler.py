@@ -299,20 +299,35 @@ def plan_blocks(ops, n, k=5, effort=1):
     block if its qubits lie in the block's qubit set and none of them was
     touched by an earlier op left out; effort 1 (the default) also searches
     the block qubit sets around each seed op, effort 0 is the greedy scan
-    alone.  measure/reset split the
-    list into independently planned segments.  Returns a list of Block | Op
-    (ops wider than k pass through)."""
+    alone.  measure/reset and ops on more than MAX_PLAN_QUBITS qubits split
+    the list into independently planned segments.  Returns a list of Block |
+    Op (ops wider than k pass through)."""
     out = []
+    for seg in _segments(ops):
+        if isinstance(seg, Op):
+            out.append(seg)
+        else:
+            out.extend(_plan_segment(seg, n, k, effort))
+    return out
+
+
+MAX_PLAN_QUBITS = 8      # widest op the native planners take
+
+
+def _segments(ops):
+    """ops in order as lists the native planners take and, between them, the
+    ops they do not: measure, reset and ops on more than MAX_PLAN_QUBITS qubits."""
     seg = []
     for op in ops:
-        if op.kind in ("measure", "reset"):
-            out.extend(_plan_segment(seg, n, k, effort))
+        if op.kind in ("measure", "reset") or len(op.all_qubits) > MAX_PLAN_QUBITS:
+            if seg:
+                yield seg
+            yield op
             seg = []
-            out.append(op)
         else:
             seg.append(op)
-    out.extend(_plan_segment(seg, n, k, effort))
-    return out
+    if seg:
+        yield seg
 
 
 def plan_blocks_arrays(n, op_nq, op_qubits, op_mats, k=5, effort=1):
@@ -346,24 +361,25 @@ def plan_blocks_arrays(n, op_nq, op_qubits, op_mats, k=5, effort=1):
     return refs, bqs[:nb], bm[:nb]
 
 
-def _op_arrays(ops):
-    """The planners' flat arrays of an op list: (op_nq, op_qubits, op_mats)."""
+def _op_arrays(ops, k):
+    """The planners' flat arrays of an op list: (op_nq, op_qubits, op_mats).
+    Ops on more than k qubits pass through and go by their qubits alone: their
+    matrices (8 MiB of eight 8-qubit ones) are left zero."""
     m = len(ops)
     nq = np.zeros(m, dtype=np.int32)
-    qb = np.full((m, 8), -1, dtype=np.int32)
+    qb = np.full((m, MAX_PLAN_QUBITS), -1, dtype=np.int32)
     mats = []
     for i, op in enumerate(ops):
         qs = op.all_qubits
         nq[i] = len(qs)
         qb[i, :len(qs)] = qs
-        mats.append(np.asarray(op.full_matrix(), dtype=np.complex128).reshape(-1))
+        mats.append(np.asarray(op.full_matrix(), dtype=np.complex128).reshape(-1) if len(qs) <= k
+                    else np.zeros(1 << (2 * len(qs)), dtype=np.complex128))
     return nq, qb, np.concatenate(mats)
 
 
 def _plan_segment(ops, n, k, effort=1):
-    if not ops:
-        return []
-    refs, bqs, bm = plan_blocks_arrays(n, *_op_arrays(ops), k, effort)
+    refs, bqs, bm = plan_blocks_arrays(n, *_op_arrays(ops, k), k, effort)
     res = []
     for e in refs:
         if e >= 0:
@@ -375,6 +391,7 @@ def _plan_segment(ops, n, k, effort=1):
 
 
 PASS_MIN_QUBITS = 10     # smallest state (and tile) of the block passes
+PASS_BLOCK_QUBITS = 4    # qubits of their blocks
 
 
 class PassRun:
@@ -415,12 +432,12 @@ def plan_passes_arrays(n, op_nq, op_qubits, op_mats, tile_bits, low_bits):
 def plan_passes(ops, n, tile_bits, low_bits):
     """Pack unitary ops into block passes (n >= PASS_MIN_QUBITS).  Returns a
     list of PassRun | Op (measure/reset, and ops of more than 4 qubits)."""
-    out, seg = [], []
-
-    def flush():
-        if not seg:
-            return
-        refs, passes, blocks, frags = plan_passes_arrays(n, *_op_arrays(seg), tile_bits, low_bits)
+    out = []
+    for seg in _segments(ops):
+        if isinstance(seg, Op):
+            out.append(seg)
+            continue
+        refs, passes, blocks, frags = plan_passes_arrays(n, *_op_arrays(seg, PASS_BLOCK_QUBITS), tile_bits, low_bits)
         e = 0
         while e < len(refs):
             if refs[e] < 0:
@@ -436,15 +453,6 @@ def plan_passes(ops, n, tile_bits, low_bits):
             last = int(p["first_block"][-1] + p["n_blocks"][-1])
             p["first_block"] -= first
             out.append(PassRun(p, blocks[first:last], frags[first:last]))
-        seg.clear()
-
-    for op in ops:
-        if op.kind in ("measure", "reset"):
-            flush()
-            out.append(op)
-        else:
-            seg.append(op)
-    flush()
     return out
 
 

@@ -1,0 +1,63 @@
+"""Ops on more qubits than a block or a pass holds: the planners let them
+through in order, and circuits with them run in every mode."""
+import numpy as np
+import pytest
+
+from oracle import statevector as O
+from test_compiler import _sim_ops
+from test_passes import _replay
+
+
+def _circuit(n, widths, seed):
+    """Layers of ry and CX with an X of w controls after each, w in widths."""
+    from blackwell_backend.circuit import QuantumCircuit
+    rng = np.random.default_rng(seed)
+    qc = QuantumCircuit(n)
+    for w in widths:
+        for q in range(n):
+            qc.ry(float(rng.uniform(0, 6)), q)
+        for q in range(0, n - 1, 2):
+            qc.cx(q, q + 1)
+        s = [int(x) for x in rng.choice(n, w + 1, replace=False)]
+        qc.mcx(s[:w], s[w])
+    return qc
+
+
+@pytest.mark.parametrize("n,widths", [(14, (8,)), (14, (10, 7, 4, 8)), (13, (9, 3, 10))])
+def test_planners_let_wide_ops_through(n, widths):
+    from blackwell_backend import compiler as C
+    from blackwell_backend.circuit import instructions
+    ops = C.compile_ops(instructions(_circuit(n, widths, n)))
+    ref = _sim_ops(n, ops)
+    psi = O.zero_state(n)
+    passed = []
+    for e in C.plan_passes(ops, n, 11, 4):
+        if isinstance(e, C.PassRun):
+            psi = _replay(psi, n, e)
+        else:
+            passed.append(len(e.all_qubits))
+            psi = O.apply_matrix(psi, e.full_matrix(), list(e.all_qubits))
+    assert passed == [w + 1 for w in widths if w > 3]
+    # coefficients are within 2^-26, 32 products to a row, over at most one block per op
+    assert np.max(np.abs(psi - ref)) < len(ops) * 32 * 2.0 ** -26
+    for k in (4, 5, 6):
+        psi = O.zero_state(n)
+        for e in C.plan_blocks(ops, n, k=k):
+            block = isinstance(e, C.Block)
+            assert block or len(e.all_qubits) > k
+            psi = O.apply_matrix(psi, e.mat if block else e.full_matrix(), list(e.qubits if block else e.all_qubits))
+        # FP64 products of at most 32 x 32 matrices
+        assert np.max(np.abs(psi - ref)) < len(ops) * 64 * 2.0 ** -52
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,widths", [(12, (8, 11)), (14, (8, 12, 4)), (15, (9, 6))])
+def test_wide_ops_run_in_every_mode(dev, n, widths):
+    from blackwell_backend import BlackwellSimulator
+    sim = BlackwellSimulator(dev)
+    qc = _circuit(n, widths, n)
+    exp, _ = sim.run_statevector(qc, mode="plain")
+    for mode in ("auto", "passes", "blocks", "tiles"):
+        got, _ = sim.run_statevector(qc, mode=mode)
+        # FP32 rounding of at most a few ulp per gate, over fewer than 100 gates
+        assert np.linalg.norm(got - exp) <= 100 * 4 * 2.0 ** -24, mode
