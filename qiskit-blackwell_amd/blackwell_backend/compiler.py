@@ -479,23 +479,32 @@ class TilePass:
         self.ops = ops
 
 
+TILE_DENSE_QUBITS = 5    # widest dense op of an LDS tile program
+
+
+def fits_tile(op):
+    """Whether an LDS tile program of enough qubits can run `op`."""
+    return op.kind not in ("measure", "reset") and (op.kind != "mk" or len(op.qubits) <= TILE_DENSE_QUBITS)
+
+
 def plan_tiles(ops, n, m=13, low=4):
     """Pack ops into tile passes of at most m qubits that always include
-    qubits 0..low-1 (contiguous 2^low-amplitude runs in HBM)."""
+    qubits 0..low-1 (contiguous 2^low-amplitude runs in HBM).  Ops that no
+    tile holds stay between them."""
     m = min(m, n)
     low = min(low, m)
     base = (1 << low) - 1
     remaining = list(ops)
     out = []
     while remaining:
-        if remaining[0].kind in ("measure", "reset"):
+        if not fits_tile(remaining[0]):
             out.append(remaining.pop(0))
             continue
         mask = base
         chosen, keep, blocked = [], [], set()
         for op in remaining:
             qs = set(op.all_qubits)
-            if op.kind in ("measure", "reset") or (qs & blocked):
+            if not fits_tile(op) or (qs & blocked):
                 blocked |= qs
                 keep.append(op)
                 continue

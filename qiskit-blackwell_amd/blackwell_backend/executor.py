@@ -135,6 +135,9 @@ def tile_ops(ops, mask):
             arr[i]["kind"] = _lib.OP_M2
             c = op.mat.reshape(-1)
         elif k == "mk":
+            if not C.fits_tile(op):
+                raise ValueError(f"dense op of {len(op.qubits)} qubits in a tile program (at most "
+                                 f"{C.TILE_DENSE_QUBITS})")
             arr[i]["kind"] = _lib.OP_MK
             c = op.mat.reshape(-1)
         elif k == "x":
@@ -331,8 +334,7 @@ class CompiledCircuit:
             return self._build_plain(self.ops, device)
         if mode == "whole":
             mask = (1 << n) - 1
-            unitary = [o for o in self.ops if o.kind not in ("measure", "reset")]
-            if len(unitary) == len(self.ops):
+            if all(C.fits_tile(o) for o in self.ops):
                 return self._build_tiles([C.TilePass(mask, self.ops)] if self.ops else [], device)
             mode = "tiles"
         if mode == "tiles":

@@ -3,6 +3,7 @@ through in order, and circuits with them run in every mode."""
 import numpy as np
 import pytest
 
+from helpers import rand_unitary
 from oracle import statevector as O
 from test_compiler import _sim_ops
 from test_passes import _replay
@@ -61,3 +62,41 @@ def test_wide_ops_run_in_every_mode(dev, n, widths):
         got, _ = sim.run_statevector(qc, mode=mode)
         # FP32 rounding of at most a few ulp per gate, over fewer than 100 gates
         assert np.linalg.norm(got - exp) <= 100 * 4 * 2.0 ** -24, mode
+
+
+def test_tile_plans_let_dense_ops_of_six_qubits_through():
+    """An LDS program runs dense ops of at most five qubits; it used to leave
+    larger ones out without an error."""
+    from blackwell_backend import compiler as C
+    from blackwell_backend.executor import tile_ops
+    ops = [C.Op("m1", [3], rand_unitary(2, 0)), C.Op("mk", [0, 2, 3, 5, 6, 8], rand_unitary(64, 1)),
+           C.Op("mk", [0, 2, 4, 5, 7], rand_unitary(32, 2))]
+    plan = C.plan_tiles(ops, 9, m=9)
+    assert [isinstance(e, C.TilePass) for e in plan] == [True, False, True] and plan[1] is ops[1]
+    assert [o for e in plan if isinstance(e, C.TilePass) for o in e.ops] == [ops[0], ops[2]]
+    with pytest.raises(ValueError, match="dense op of 6 qubits"):
+        tile_ops(ops, 0x1ff)
+
+
+@pytest.mark.gpu
+def test_dense_ops_of_six_qubits_run_or_are_refused(dev):
+    from blackwell_backend import BlackwellSimulator, compiler as C
+    from blackwell_backend.circuit import QuantumCircuit, instructions
+    sim = BlackwellSimulator(dev)
+    u = rand_unitary(64, 5)
+
+    def circuit(n):
+        qc = QuantumCircuit(n)
+        for q in range(n):
+            qc.ry(0.3 + q, q)
+        return qc.unitary(u, [0, 3, 4, 6, 7, n - 1]).cx(0, n - 1)
+    qc = circuit(14)
+    ref = _sim_ops(14, C.compile_ops(instructions(qc)))
+    for mode in ("auto", "passes", "blocks", "tiles", "plain"):
+        got, _ = sim.run_statevector(qc, mode=mode)
+        # 64-term FP32 sums in one block, a few ulp per gate elsewhere
+        assert np.linalg.norm(got - ref) <= (64 + 4 * 16) * 2.0 ** -24, mode
+    for n in (9, 12):
+        for mode in ("auto", "whole", "tiles", "plain"):
+            with pytest.raises(RuntimeError, match="wider blocks are not supported"):
+                sim.run_statevector(circuit(n), mode=mode)
