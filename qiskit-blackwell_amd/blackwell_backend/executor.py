@@ -44,6 +44,7 @@ GRAPH_SAFE_STEPS = ("passes", "blocks", "mfma", "tile", "mcgate")
 # fusion widths of the MFMA block kernels and the smallest state each runs on
 BLOCK_WIDTHS = {4: 11, 5: BLOCK_MIN_QUBITS, 6: 13}
 TUNE_REPS = 3
+MAX_CONTROLS = 7        # of the plain multi-controlled kernels
 
 
 def block_width(mode):
@@ -433,9 +434,18 @@ class CompiledCircuit:
                 mats.append(e.mat.astype(np.complex64).reshape(-1))
                 steps.append(("block", (len(mats) - 1, list(e.qubits))))
             else:
-                steps.append(("sub", self._build_plain([e], device)))
+                steps.append(("sub", self._build_single(e, device)))
         flush()
         return _Plan(self, steps, mats, None, None, device)
+
+    def _build_single(self, op, device):
+        """An op between blocks or passes, in a launch of its own: the plain kernel
+        or, above the controls that takes, an LDS program of tiles that hold it."""
+        if len(op.controls) > MAX_CONTROLS and len(op.all_qubits) <= WHOLE_TILE_MAX:
+            low = 4 if len(op.all_qubits) + 4 <= WHOLE_TILE_MAX else 1
+            m = max(len(op.all_qubits) + low, 10)
+            return self._build_tiles(C.plan_tiles([op], self.n_qubits, m=m, low=low), device)
+        return self._build_plain([op], device)
 
     def _build_passes(self, entries, device):
         steps, parts, off = [], [], 0
@@ -448,7 +458,7 @@ class CompiledCircuit:
             elif e.kind not in ("measure", "reset") and len(e.all_qubits) == 5:
                 steps.append(("sub", self._build_blocks(C.plan_blocks([e], self.n_qubits), device)))
             else:
-                steps.append(("sub", self._build_plain([e], device)))
+                steps.append(("sub", self._build_single(e, device)))
         return _Plan(self, steps, [], None, None, device, np.concatenate(parts) if parts else None)
 
     def _build_tiles(self, entries, device):

@@ -51,17 +51,34 @@ def test_planners_let_wide_ops_through(n, widths):
         assert np.max(np.abs(psi - ref)) < len(ops) * 64 * 2.0 ** -52
 
 
+def _apply(psi, n, op):
+    """O.apply_matrix, but X with many controls as the permutation it is."""
+    if op.kind != "x" or len(op.controls) < 6:
+        return O.apply_matrix(psi, op.full_matrix(), list(op.all_qubits))
+    i = np.arange(1 << n)
+    on = np.all([(i >> c) & 1 for c in op.controls], axis=0)
+    return psi[np.where(on, i ^ (1 << op.qubits[0]), i)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,widths", [(12, (8, 11)), (14, (8, 12, 4)), (15, (9, 6))])
-def test_wide_ops_run_in_every_mode(dev, n, widths):
-    from blackwell_backend import BlackwellSimulator
+@pytest.mark.parametrize("n,widths", [(12, (8, 11)), (14, (8, 12, 4)), (18, (9, 12, 6))])
+def test_wide_ops_run_between_blocks_and_passes(dev, n, widths):
+    """Up to 12 controls, past the seven that the plain kernel takes, on qubits
+    with and without the low ones."""
+    from blackwell_backend import BlackwellSimulator, compiler as C
+    from blackwell_backend.circuit import instructions
+    from blackwell_kernels._lib import QsimError
     sim = BlackwellSimulator(dev)
     qc = _circuit(n, widths, n)
-    exp, _ = sim.run_statevector(qc, mode="plain")
-    for mode in ("auto", "passes", "blocks", "tiles"):
+    ref = O.zero_state(n)
+    for op in C.compile_ops(instructions(qc)):
+        ref = _apply(ref, n, op)
+    for mode in ("auto", "passes", "blocks"):
         got, _ = sim.run_statevector(qc, mode=mode)
         # FP32 rounding of at most a few ulp per gate, over fewer than 100 gates
-        assert np.linalg.norm(got - exp) <= 100 * 4 * 2.0 ** -24, mode
+        assert np.linalg.norm(got - ref) <= 100 * 4 * 2.0 ** -24, mode
+    with pytest.raises(QsimError, match="controls must have 0-7 elements"):
+        sim.run_statevector(qc, mode="plain")
 
 
 def test_tile_plans_let_dense_ops_of_six_qubits_through():
