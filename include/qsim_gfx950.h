@@ -196,6 +196,12 @@ int qsim_plan_blocks_search(int n_qubits, int k, int effort, int n_ops, const in
 int qsim_apply_blocks(void* stream, void* state, int n_qubits, const void* blocks_dev,
                       const int32_t* block_qubits, int n_blocks);
 
+/* About how many blocks of at most k qubits qsim_plan_blocks needs for ops on
+ * the qubit sets op_masks, in circuit order: one scan per block that grows it
+ * from the first op left.  Ops on more than k qubits pass through uncounted.
+ * Host only.  (new)                                                       */
+int qsim_count_blocks(int n_qubits, int k, int n_ops, const uint64_t* op_masks, int* n_blocks);
+
 /* ---- block passes (new) -------------------------------------------------- */
 /* A pass: one trip of the state through memory that applies n_blocks dense
  * 4-qubit blocks to tiles of 2^m amplitudes held in LDS (tile_mask: the m

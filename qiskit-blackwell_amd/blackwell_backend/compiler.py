@@ -390,6 +390,22 @@ def _plan_segment(ops, n, k, effort=1):
     return res
 
 
+def count_blocks(ops, n, k=5):
+    """About how many k-qubit blocks plan_blocks makes of the unitary ops of at
+    most k qubits (qsim_count_blocks), without building matrices: the counts
+    of 100 to 600 ops take 0.1 to 0.4 ms, a plan 1 to 40."""
+    import ctypes
+    from blackwell_kernels import _lib
+    total, out = 0, ctypes.c_int(0)
+    for seg in _segments(ops):
+        if isinstance(seg, Op):
+            continue
+        masks = np.array([_mask(op.all_qubits) for op in seg], dtype=np.uint64)
+        _lib.call("qsim_count_blocks", n, k, len(seg), ctypes.c_void_p(masks.ctypes.data), ctypes.byref(out))
+        total += out.value
+    return total
+
+
 PASS_MIN_QUBITS = 10     # smallest state (and tile) of the block passes
 PASS_BLOCK_QUBITS = 4    # qubits of their blocks
 

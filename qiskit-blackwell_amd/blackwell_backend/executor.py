@@ -16,8 +16,8 @@ Modes:
            bf16 MFMA, many per trip through HBM (n >= 10): tiles of 10..13
            qubits stay in LDS for all the blocks of a pass;
   tiles  - LDS tile programs, many ops per HBM pass;
-  auto   - tiles (the whole state in one tile when n <= 13) for circuits with
-           few ops per qubit on at most 20 qubits, else passes;
+  auto   - one LDS program below 10 qubits, passes above, but for circuits that
+           blocks or LDS programs run faster (CompiledCircuit._auto_mode);
   tune   - every applicable mode timed once on the device, fastest kept
            (the fusion width is one of the choices).
 """
@@ -33,11 +33,32 @@ from . import compiler as C
 
 WHOLE_TILE_MAX = 13     # n <= 13: the whole state is one LDS tile (64 KiB)
 BLOCK_MIN_QUBITS = 10   # the MFMA block kernel needs 2^10 amplitudes
-# auto between 10 and 13 qubits, us: an op of the one-workgroup LDS program
-# against a block pass and each op that no pass holds (_auto_mode)
-WHOLE_OP_US = lambda n: 0.55 + 0.65 * 2.0 ** (n - 12)
-PASS_US = 5.0
-WIDE_OP_US = 6.0
+# What auto weighs, us by qubit count: a block pass, a 4-qubit block in it, a
+# launch of a 5-qubit block.  Least squares over the circuits of _auto_mode,
+# graph replays up to 20 qubits and plan runs above; from 22 on four times the
+# size takes four times as long.
+TRIP_US = {10: (2.2, 0.24, 3.6), 12: (3.4, 0.31, 6.5), 14: (3.3, 0.3, 7.3), 16: (3.3, 0.46, 7.6), 18: (4.2, 0.51, 8.1),
+           20: (8.3, 0.6, 10.6), 22: (11.0, 2.9, 20.0), 24: (32.0, 9.8, 58.0), 26: (140.0, 35.0, 210.0)}
+WIDE_OP_US = 1.5         # an op of six qubits and more, alone
+# LDS programs: an op of the whole state (10..13 qubits), a pass and an op of
+# tile programs (14..20), and a dense 5-qubit op of either
+WHOLE_OP_US = lambda n: 0.45 + 0.57 * 2.0 ** (n - 12)
+TILE_PASS_US = {14: 4.5, 16: 4.7, 18: 5.4, 20: 10.0}
+TILE_OP_US = {14: 0.59, 16: 0.58, 18: 0.6, 20: 0.85}
+DENSE5_OP_US = 42.0
+AUTO_TILES_MAX_QUBITS = 20
+PASS_US = 4.2            # the shortest plan of passes, below which a program of few ops is faster
+
+
+def _at_size(table, n):
+    """A table by even qubit counts at n: geometric means between its entries,
+    its last entry scaled with the state's size above them."""
+    top = max(table)
+    if n > top:
+        return np.asarray(table[top]) * 2.0 ** (n - top)
+    return np.sqrt(np.asarray(table[n & ~1]) * np.asarray(table[(n + 1) & ~1]))
+
+
 # plan steps a HIP graph can hold: library launches on the current stream with
 # device-resident arguments only (no host uploads, no host-side decisions)
 GRAPH_SAFE_STEPS = ("passes", "blocks", "mfma", "tile", "mcgate")
@@ -156,6 +177,21 @@ def tile_ops(ops, mask):
     return arr, cf
 
 
+def _pass_groups(entries):
+    """Entries of plan_passes with the ops between two runs of passes as one list."""
+    held = []
+    for e in entries:
+        if not isinstance(e, C.PassRun):
+            held.append(e)
+            continue
+        if held:
+            yield held
+            held = []
+        yield e
+    if held:
+        yield held
+
+
 class _Dev:
     """Device copies of a plan's matrices/op tables (one upload per plan)."""
 
@@ -180,6 +216,7 @@ class CompiledCircuit:
         self.phase0 = None if phi == 0.0 else complex(np.cos(phi), np.sin(phi))
         self._plans = {}
         self._blocks = None
+        self._passes = None
         self._tiles = None
         self._auto = None
         self._graphs = {}
@@ -277,6 +314,12 @@ class CompiledCircuit:
             self._blocks[k] = C.plan_blocks(self.ops, self.n_qubits, k=k)
         return self._blocks[k]
 
+    def pass_entries(self):
+        """plan_passes of the ops at the shape for their size (computed once)."""
+        if self._passes is None:
+            self._passes = C.plan_passes(self.ops, self.n_qubits, *pass_shape(self.n_qubits))
+        return self._passes
+
     # ---------------------------------------------------------------- plans
     def plan(self, mode, device):
         key = (mode, str(device))
@@ -294,8 +337,7 @@ class CompiledCircuit:
         return self._tiles
 
     def resolve_mode(self, mode, device=None):
-        """auto: the whole state as one LDS program below 10 qubits, block
-        passes above, but for the circuits _auto_mode names.
+        """auto: the plan _auto_mode expects to be the fastest.
         tune: the mode tuned_mode measured fastest on `device`."""
         if mode == "tune":
             if device is None:
@@ -308,26 +350,51 @@ class CompiledCircuit:
         return self._auto
 
     def _auto_mode(self):
-        """Block passes from 10 qubits on: over ladders, QFT, SU(4) volume and
-        multi-controlled circuits of 10 to 20 qubits and depths 1 to 8 they
-        measured faster than LDS programs (10 qubits 17-52 us against 22-134,
-        13 qubits 18-97 against 33-374, 16 qubits 20-130 against 26-330, 20
-        qubits 27-267 against 53-667) and closer to FP64 (QFT of 16 qubits
-        1.5e-7 against 5.7e-7, SU(4) volume 1.7e-7 against 2.7e-7).  An op on
-        more than four qubits interrupts a pass and takes a launch of its own,
-        where an LDS program of at most 13 qubits goes on: 100 ops of 12 qubits,
-        10 / 20 / 50 of them with six controls, 79 / 130 / 194 us in passes
-        against 103 / 109 / 104, of 13 qubits 69 / 122 / 198 against 153 / 161 /
-        149.  Dense matrices of five qubits are slow in LDS programs (20 of
-        100: 183 against 778 us), and tile programs of 14 qubits and more lose
-        at every share (14 qubits 58 / 105 / 184 against 104 / 156 / 249)."""
+        """Block passes from 10 qubits on, but where ops they cannot hold, or
+        many gates on the same five qubits, make another plan shorter.  Over
+        ladders, QFT, SU(4) volume and three-control circuits of 10 to 20 qubits
+        and depths 1 to 8 passes measured faster than LDS programs (10 qubits
+        17-52 us against 22-134, 16 qubits 20-130 against 26-330, 20 qubits 27-267
+        against 53-667) and closer to FP64, and half the time of 5-qubit blocks
+        above.  An op of five qubits interrupts a pass and is a block of its own
+        there, where block plans put its neighbours into it: 28 qubits, ten layers
+        of ry and four four-control X, 60.6 ms in passes against 31.9 in blocks,
+        the same four-control X and ry a hundred times 155 against 0.86, 60
+        SU(4) on the same five qubits 2.1 against 0.76; with H, X and CX layers
+        between the X 76.8 against 105.9.  So both are counted at TRIP_US, and LDS
+        programs too where ops of five qubits and more are: they hold controlled
+        ones of any width (16 qubits, ten layers of ry and four six-control X 312
+        us against 448)."""
         n = self.n_qubits
         if n < C.PASS_MIN_QUBITS:
             return "whole"
-        if n > WHOLE_TILE_MAX:
-            return "passes"
-        wide = sum(1 for o in self.ops if len(o.all_qubits) > 4 and o.kind != "mk")
-        return "whole" if len(self.ops) * WHOLE_OP_US(n) < PASS_US + wide * WIDE_OP_US else "passes"
+        wide = any(len(o.all_qubits) > C.PASS_BLOCK_QUBITS for o in self.ops)
+        if n <= WHOLE_TILE_MAX and not wide and len(self.ops) * WHOLE_OP_US(n) < PASS_US:
+            return "whole"
+        us = {"passes": self._passes_us(), "blocks": self._launches_us(self.ops)}
+        if wide and n <= AUTO_TILES_MAX_QUBITS and all(C.fits_tile(o) for o in self.ops if o.kind not in
+                                                       ("measure", "reset")):
+            dense = [len(o.qubits) for o in self.ops if o.kind == "mk"]
+            us_dense = sum(DENSE5_OP_US * 4.0 ** (k - C.TILE_DENSE_QUBITS) for k in dense)
+            if n <= WHOLE_TILE_MAX:
+                us["whole"] = (len(self.ops) - len(dense)) * WHOLE_OP_US(n) + us_dense
+            else:
+                tiles = self.tile_entries()
+                passes = sum(isinstance(e, C.TilePass) for e in tiles)
+                us["tiles"] = (passes * _at_size(TILE_PASS_US, n) + (len(tiles) - passes) * WIDE_OP_US
+                               + (len(self.ops) - len(dense)) * _at_size(TILE_OP_US, n) + us_dense)
+        return min(us, key=us.get)
+
+    def _launches_us(self, ops):
+        """About how long `ops` take as 5-qubit blocks and single wider ops."""
+        wide = sum(len(o.all_qubits) > 5 for o in ops)
+        return C.count_blocks(ops, self.n_qubits) * _at_size(TRIP_US, self.n_qubits)[2] + wide * WIDE_OP_US
+
+    def _passes_us(self):
+        """About how long plan_passes' plan takes."""
+        t_pass, t_block, _ = _at_size(TRIP_US, self.n_qubits)
+        return sum(len(e.passes) * t_pass + len(e.blocks) * t_block if isinstance(e, C.PassRun)
+                   else self._launches_us(e) for e in _pass_groups(self.pass_entries()))
 
     def _build(self, mode, device):
         n = self.n_qubits
@@ -351,7 +418,7 @@ class CompiledCircuit:
         if mode == "passes":
             if n < C.PASS_MIN_QUBITS:
                 raise ValueError(f"block passes need n >= {C.PASS_MIN_QUBITS} (n = {n})")
-            return self._build_passes(C.plan_passes(self.ops, n, *pass_shape(n)), device)
+            return self._build_passes(self.pass_entries(), device)
         if mode == "blocks":
             if n < 10:
                 return self._build_tiles(C.plan_tiles(self.ops, n, m=n), device)
@@ -368,9 +435,12 @@ class CompiledCircuit:
         raise ValueError(f"unknown execution mode {mode!r}")
 
     def _build_plain(self, ops, device):
+        steps, mats = [], []
+        self._plain_steps(ops, steps, mats)
+        return _Plan(self, steps, mats, None, None, device)
+
+    def _plain_steps(self, ops, steps, mats):
         n = self.n_qubits
-        mats = []
-        steps = []
         for op in ops:
             k, q = op.kind, op.qubits
             if k in ("measure", "reset"):
@@ -403,12 +473,14 @@ class CompiledCircuit:
                 steps.append(("block", (len(mats) - 1, list(q))))
             else:
                 raise ValueError(f"cannot execute op {op}")
-        return _Plan(self, steps, mats, None, None, device)
 
     def _build_blocks(self, entries, device):
+        steps, mats = [], []
+        self._block_steps(entries, steps, mats, device)
+        return _Plan(self, steps, mats, None, None, device)
+
+    def _block_steps(self, entries, steps, mats, device):
         n = self.n_qubits
-        mats = []
-        steps = []
         run = []                  # consecutive 5-qubit blocks -> one qsim_apply_blocks call
 
         def flush():
@@ -434,35 +506,34 @@ class CompiledCircuit:
                 mats.append(e.mat.astype(np.complex64).reshape(-1))
                 steps.append(("block", (len(mats) - 1, list(e.qubits))))
             else:
-                steps.append(("sub", self._build_single(e, device)))
+                self._single_step(e, steps, mats, device)
         flush()
-        return _Plan(self, steps, mats, None, None, device)
 
-    def _build_single(self, op, device):
-        """An op between blocks or passes, in a launch of its own: the plain kernel
-        or, above the controls that takes, an LDS program of tiles that hold it."""
+    def _single_step(self, op, steps, mats, device):
+        """An op between blocks, passes or tiles, in a launch of its own: the plain
+        kernel or, above the controls that takes, an LDS program of tiles that hold it."""
         if len(op.controls) > MAX_CONTROLS and len(op.all_qubits) <= WHOLE_TILE_MAX:
             low = 4 if len(op.all_qubits) + 4 <= WHOLE_TILE_MAX else 1
             m = max(len(op.all_qubits) + low, 10)
-            return self._build_tiles(C.plan_tiles([op], self.n_qubits, m=m, low=low), device)
-        return self._build_plain([op], device)
+            steps.append(("sub", self._build_tiles(C.plan_tiles([op], self.n_qubits, m=m, low=low), device)))
+        else:
+            self._plain_steps([op], steps, mats)
 
     def _build_passes(self, entries, device):
-        steps, parts, off = [], [], 0
-        for e in entries:
+        steps, mats, parts, off = [], [], [], 0
+        for e in _pass_groups(entries):
             if isinstance(e, C.PassRun):
                 # one device blob per plan: records then fragments of each run
                 steps.append(("passes", (e.passes, e.blocks, off, off + e.blocks.nbytes)))
                 parts += [e.blocks.view(np.uint8).reshape(-1), e.frags.view(np.uint8).reshape(-1)]
                 off += e.blocks.nbytes + e.frags.nbytes
-            elif e.kind not in ("measure", "reset") and len(e.all_qubits) == 5:
-                steps.append(("sub", self._build_blocks(C.plan_blocks([e], self.n_qubits), device)))
             else:
-                steps.append(("sub", self._build_single(e, device)))
-        return _Plan(self, steps, [], None, None, device, np.concatenate(parts) if parts else None)
+                # ops that no pass holds, those of five qubits fused where they share them
+                self._block_steps(C.plan_blocks(e, self.n_qubits), steps, mats, device)
+        return _Plan(self, steps, mats, None, None, device, np.concatenate(parts) if parts else None)
 
     def _build_tiles(self, entries, device):
-        all_ops, all_cf, steps = [], [], []
+        all_ops, all_cf, steps, mats = [], [], [], []
         op_off, cf_off = 0, 0
         for e in entries:
             if isinstance(e, C.TilePass):
@@ -474,12 +545,12 @@ class CompiledCircuit:
                 op_off += len(arr)
                 cf_off += cf.size
             else:
-                steps.append(("sub", self._build_plain([e], device)))
+                self._single_step(e, steps, mats, device)
         ops = np.concatenate(all_ops) if all_ops else np.zeros(0, dtype=OP_DTYPE)
         cf = np.concatenate(all_cf) if all_cf else np.zeros(0, dtype=np.complex128)
         if cf.size == 0:
             cf = np.zeros(1, dtype=np.complex128)
-        return _Plan(self, steps, [], ops, cf.astype(np.complex64), device)
+        return _Plan(self, steps, mats, ops, cf.astype(np.complex64), device)
 
 
 class _Plan:

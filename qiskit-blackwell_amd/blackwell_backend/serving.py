@@ -28,7 +28,7 @@ running batches and the HBM lane.
 Repeated circuits on the HBM lane replay as HIP graphs: a request that
 carries a circuit (no gate payload) and whose compiled circuit the server
 has already run once is executed by replaying a captured graph of state
-init + its pass plan (one host call instead of one launch per pass), into
+init + its "auto" plan (one host call instead of one per launch), into
 the graph's own buffer, which is sampled before the next replay on the
 same stream.  Gate-payload requests are unique by construction and run as
 batched pass steps instead.
@@ -360,7 +360,7 @@ class _HbmJob:
                 else:
                     self.state = torch.empty(1 << r.n_qubits, dtype=torch.complex64, device=dev)
                     cc.init_state(self.state)
-                    cc.plan(cc.resolve_mode("passes"), dev).run(self.state)
+                    cc.plan(cc.resolve_mode("auto"), dev).run(self.state)
             from blackwell_kernels import sample_with_uniforms, uniforms_splitmix
             u = uniforms_splitmix(r.seed, r.shots, dev)
             self.d_out = sample_with_uniforms(self.state, u)
@@ -522,7 +522,7 @@ class _GraphCache:
         if g is None:
             if self.seen[cc] < 2:
                 return None
-            mode = cc.resolve_mode("passes")
+            mode = cc.resolve_mode("auto")
             g = cc.graphed(mode, device)
             if g is None:
                 return None

@@ -9,9 +9,9 @@ before execution (simulator.py:555-604), the complex64 statevector
 Differences by design:
   * circuits are compiled by blackwell_backend.compiler (FP64 host fusion)
     into plans of prepared launches (blackwell_backend.executor);
-  * the default execution mode is "auto": LDS programs below 10 qubits (and
-    to 13 for circuits of mostly wide controlled gates), passes of 4-qubit
-    MFMA blocks above;
+  * the default execution mode is "auto": LDS programs below 10 qubits, passes
+    of 4-qubit MFMA blocks above, and 5-qubit blocks or LDS programs for
+    circuits those run faster (many gates on five qubits and more);
     mode="blocks" runs one launch per 5-qubit block,
     mode="plain" runs one kernel per gate, mode="blocks/<k>" fuses into
     k-qubit MFMA blocks (k = 4, 5, 6) and mode="tune" times the modes and

@@ -53,6 +53,7 @@ PROTOTYPES = {
     "qsim_plan_blocks": (_i, [_i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _pint]),
     "qsim_plan_blocks_search": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _pint]),
     "qsim_apply_blocks": (_i, [_vp, _vp, _i, _vp, _vp, _i]),
+    "qsim_count_blocks": (_i, [_i, _i, _i, _vp, _pint]),
     "qsim_plan_passes": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _pint, _pint]),
     "qsim_apply_passes": (_i, [_vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _i]),
     "qsim_apply_pass_batch": (_i, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64]),

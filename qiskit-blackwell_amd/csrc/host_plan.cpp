@@ -475,6 +475,44 @@ int qsim_plan_blocks(int n_qubits, int k, int n_ops, const int32_t* op_nq, const
                                  block_qubits, block_mats, n_out);
 }
 
+int qsim_count_blocks(int n_qubits, int k, int n_ops, const uint64_t* op_masks, int* n_blocks) {
+  if (n_qubits < 1 || n_qubits > QSIM_MAX_QUBITS) return fail(QSIM_ERANGE, "n_qubits=%d", n_qubits);
+  if (k < 1 || k > QSIM_MAX_BLOCK_QUBITS) return fail(QSIM_ERANGE, "block size k=%d outside 1..%d", k,
+                                                      QSIM_MAX_BLOCK_QUBITS);
+  if (n_ops < 0) return fail(QSIM_EINVAL, "n_ops < 0");
+  if (!n_blocks || (n_ops > 0 && !op_masks)) return fail(QSIM_EINVAL, "NULL pointer argument");
+  const uint64_t all = (1ull << n_qubits) - 1;
+  for (int i = 0; i < n_ops; ++i)
+    if (op_masks[i] == 0 || (op_masks[i] & ~all)) return fail(QSIM_EINVAL, "op %d: qubit set outside the state", i);
+  try {
+    std::vector<uint64_t> rem(op_masks, op_masks + n_ops);
+    size_t head = 0;                     // ops before it are done
+    int blocks = 0;
+    while (head < rem.size()) {
+      // ops left out are moved up behind the ones not looked at
+      uint64_t set = 0, blocked = 0;
+      size_t t = head, left = 0;
+      for (; t < rem.size() && (blocked & all) != all; ++t) {
+        const uint64_t m = rem[t];
+        if (!(m & blocked) && __builtin_popcountll(set | m) <= k) {
+          set |= m;
+        } else {
+          blocked |= m;
+          rem[head + left++] = m;
+        }
+      }
+      std::copy_backward(rem.begin() + head, rem.begin() + head + left, rem.begin() + t);
+      head = t - left;
+      if (set) ++blocks;
+      else ++head;                       // wider than a block, and so is all beside it: passes through
+    }
+    *n_blocks = blocks;
+    return QSIM_OK;
+  } catch (const std::bad_alloc&) {
+    return fail(QSIM_ENOMEM, "block count: out of host memory");
+  }
+}
+
 int qsim_plan_passes(int n_qubits, int tile_bits, int low_bits, int n_ops, const int32_t* op_nq,
                      const int32_t* op_qubits, const double* op_mats, int32_t* out_ref,
                      qsim_pass* passes, qsim_pass_block* blocks, uint16_t* frags, int* n_out,
