@@ -30,10 +30,11 @@ single state with FP64 row sums runs each term matrix-free by default
 (qsim_cheb_pauli_step): every entry is recomputed from the tables as the
 CSR builder computes it, so no index or value stream is read.  When all
 entries are real, one state of 9 qubits or more and batches of 16 qubits and
-more run the whole series in one call (qsim_cheb_pauli_evolve): a tile of
+more, of Hamiltonians without very many terms to an X mask (tiled_term), run
+the whole series in one call (qsim_cheb_pauli_evolve): a tile of
 T_k in LDS serves the near entries, the states of a batch share the entry
 evaluation, the accumulator is updated by two terms at a time, and the sums
-are those of the CSR terms bit for bit.  The CSR stays for small batches,
+are those of the CSR terms bit for bit.  The CSR stays for the other batches,
 complex entries, fp32c row sums and the split term.
 
 Row sums of the SpMM (accumulate=):
@@ -87,15 +88,48 @@ ACCUMULATE = {"fp64": 0, "fp32c": 1}
 
 def tiled_term(pauli, n, R):
     """Whether the tiled matrix-free terms (qsim_cheb_pauli_evolve) run R states
-    of n qubits: real entries, and a size where they measured faster than
-    what they replace.  One state always: a term of a Heisenberg chain takes
-    6.8 / 8.1 / 17.5 us on 12 / 16 / 19 qubits, 9.5 / 14 / 25 untiled.  Batches
-    against the CSR term: 17 qubits with 2 / 32 states 23 -> 16 and 81 -> 64 us,
-    16 qubits with 16 states 33 -> 30 but with 8 states 20 -> 24, 14 qubits
-    with 32 states 12 -> 16 (the CSR and T_k fit the L2s there)."""
+    of n qubits: real entries, and a size and Hamiltonian for which they measured
+    faster than what they replace.  Their work on a row is its groups (an entry
+    each, picked from at most two terms) and, for groups of more terms, each of
+    those; the CSR has one entry per group whatever its terms, for all states.
+
+    One state, against k_cheb_pauli1, which spreads the groups' bookkeeping less
+    but takes a term faster: a chain (half a term a group) of 12 / 16 / 19 / 22
+    qubits 6.8 / 8.1 / 17.5 / 96 us against 9.5 / 14 / 25 / 139, all-to-all Ising
+    (8 to 11 terms a group) of 17 / 20 / 24 qubits 17 / 62 / 935 against 21 / 53 /
+    790; 18 to 22 qubits cross at 2 to 3.5 terms a group.
+
+    Batches, against the CSR: see batch_term_us.  Smaller ones than 17 qubits, or
+    16 with 16 states, stay there (16 qubits with 8 states 20 against 24 us, 14
+    with 32 states 12 against 16: the CSR and T_k fit the L2s)."""
     if pauli.groups is None or n < _lib.PAULI_BATCH_MIN_QUBITS:
         return False
-    return R == 1 or (R > 1 and (n >= 17 or (n == 16 and R >= 16)))
+    if R == 1:
+        return n <= 17 or pauli.long_terms <= 2.5 * pauli.n_groups
+    if not (R > 1 and (n >= 17 or (n == 16 and R >= 16))):
+        return False
+    tiled, csr = batch_term_us(pauli.n_groups, pauli.long_terms, n, R)
+    return tiled <= csr
+
+
+def batch_term_us(groups, long_terms, n, R):
+    """(tiled, CSR): about how many us a Chebyshev term of R >= 2 states of n qubits
+    takes, `groups` X-mask groups of which those of three terms and more hold
+    `long_terms`.  Fitted on chains, all-to-all Ising and XYZ, sums of random
+    strings, fermion pair terms (8 strings a mask) and one mask with up to 1000
+    terms, 16 to 21 qubits and 2 to 32 states: of the two routes it names the
+    faster or one within 20 %.  us tiled against CSR at 17 qubits: chain of 4 /
+    32 states 27 / 72 against 34 / 97, Ising 26 / 69 against 20 / 70, 1017 terms
+    in 18 groups 84 / 289 against 20 / 70; at 20 qubits Ising 94 / 562 against
+    165 / 667, 1020 terms in 21 groups 303 / 1845 against 165 / 671."""
+    rows = float(1 << n)
+    vecs = -(-R // 4)                                  # a workgroup takes four states and 256 rows
+    per_row = (1.5 + 1300.0 / (vecs * rows / 256)) * (1.0 if R >= 4 else 0.7)     # ps a group; few workgroups wait more
+    tiled = 9.0 + 1e-6 * rows * vecs * per_row * (groups + 0.11 * long_terms)
+    per_entry = 4.8 + 0.65 * R                         # ps
+    if 12.0 * groups * rows > 1 << 28:                 # the matrix no longer stays in the MALL
+        per_entry *= 1.0 + R / 80.0
+    return tiled, 5.0 + 1e-6 * rows * groups * per_entry
 
 
 def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumulate="fp64", split=False,
@@ -106,8 +140,8 @@ def chebyshev_evolve_batch(states, hamiltonian_csr, t, precision=1e-10, accumula
     matrix_free: run each term from the Pauli tables the Hamiltonian was
     built from (qsim_cheb_pauli_step) instead of the CSR; None (default)
     does so for one state with accumulate="fp64" when the Hamiltonian
-    carries its Pauli tables, and, when its entries are real, for batches of
-    the sizes tiled_term names (qsim_cheb_pauli_evolve)."""
+    carries its Pauli tables, and, when its entries are real, for batches
+    that tiled_term names (qsim_cheb_pauli_evolve)."""
     if accumulate not in ACCUMULATE:
         raise ValueError(f"accumulate must be one of {sorted(ACCUMULATE)}, got {accumulate!r}")
     mode = ACCUMULATE[accumulate]

@@ -135,9 +135,11 @@ class PauliTables:
     int64), toff (int32), sm (uint64 as int64), coef (FP64 pairs), the
     layout qsim_pauli_csr_count and qsim_cheb_pauli_step take, plus gconst
     (constant_group_entries) for the matrix-free Chebyshev term and, when
-    every coefficient is real, groups (real_group_records, else None)."""
+    every coefficient is real, groups (real_group_records, else None) and
+    long_terms, the number of terms in groups that a record does not hold."""
 
     def __init__(self, labels, coeffs, device):
+        from blackwell_kernels._lib import PAULI_TERMS
         xm, toff, sm, coef = pauli_groups(labels, coeffs)
         dev = torch.device(device)
         self.n_groups = len(xm)
@@ -149,6 +151,7 @@ class PauliTables:
         self.gconst = torch.from_numpy(gc.reshape(-1) if gc.size else np.zeros(2)).to(dev)
         recs = real_group_records(xm, toff, sm, coef, gc)
         self.groups = None if recs is None or not recs.size else torch.from_numpy(recs.view(np.uint8)).to(dev)
+        self.long_terms = 0 if recs is None else int(recs["nt"][recs["kind"] == PAULI_TERMS].sum())
 
     def args(self):
         """(n_groups, xm, toff, sm, coef) pointers for qsim_pauli_csr_count / _fill."""

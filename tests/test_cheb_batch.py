@@ -195,3 +195,46 @@ def test_series_checks_its_arguments():
         None, n, 1, g, 16, 16, R, 1.0, t0, t1, 16, 16, cf, K)
     assert call(n=8) == 2 and call(g=None) == 1 and call(R=0) == 1 and call(cf=None) == 1 and call(K=0) == 1
     assert call(t0=24) == 1 and call(t1=24) == 1 and call(t1=None) == 1
+
+
+def _ising(n, extra=0):
+    """ZZ on every pair, or `extra` Z strings in their place, and X on every qubit."""
+    rng = np.random.default_rng(n + extra)
+    lab = lambda ch, qs: "".join(ch if n - 1 - p in qs else "I" for p in range(n))
+    qs = [rng.choice(n, 4, replace=False) for _ in range(extra)] or [(i, j) for i in range(n) for j in range(i)]
+    return [(lab("Z", q), rng.uniform(-1, 1)) for q in qs] + [(lab("X", (q,)), rng.uniform(-1, 1)) for q in range(n)]
+
+
+def test_tiled_terms_are_chosen_by_the_hamiltonian():
+    """Against the faster route of each as measured: (tables, qubits, states,
+    tiled).  All-to-all Ising and one X mask of a thousand terms are the CSR's
+    at 17 qubits, and the untiled kernel's for one state of 18 qubits and more."""
+    from blackwell_backend.chebyshev import tiled_term
+    tables = lambda terms: PauliTables([t[0] for t in terms], [t[1] for t in terms], "cpu")
+    chain = lambda n: tables([("".join(ch if n - 1 - p in (i, i + 1) else "I" for p in range(n)), 0.3 + i + j)
+                              for i in range(n - 1) for j, ch in enumerate("ZXY")] + _ising(n, 1)[1:])
+    for n in (17, 20):
+        t = chain(n)
+        assert t.long_terms == n - 1
+        assert [tiled_term(t, n, R) for R in (1, 2, 4, 8, 32)] == [True] * 5
+        t = tables(_ising(n))
+        assert (t.n_groups, t.long_terms) == (n + 1, n * (n - 1) // 2)
+        assert [tiled_term(t, n, R) for R in (1, 4, 8)] == ([True, False, False] if n == 17 else [False, True, True])
+        t = tables(_ising(n, 1000))
+        assert [tiled_term(t, n, R) for R in (1, 2, 4, 8, 32)] == [n == 17, False, False, False, False]
+    assert not tiled_term(chain(16), 16, 8) and tiled_term(chain(16), 16, 16) and not tiled_term(chain(16), 16, 0)
+    assert tiled_term(chain(12), 12, 1) and not tiled_term(chain(8), 8, 1) and not tiled_term(chain(12), 12, 32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,R,matrix_free", [(17, 4, False), (18, 1, True), (18, 3, True)])
+def test_evolution_of_many_terms_a_mask_has_the_same_bits_by_either_route(n, R, matrix_free):
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(n)
+    X = torch.view_as_complex(torch.randn(R, 1 << n, 2, device=dev, generator=g))
+    X = X / torch.linalg.vector_norm(X, dim=1, keepdim=True)
+    h = HamiltonianCSR.from_sparse_pauli_op(SparsePauliOp.from_list(_ising(n, 300)), device=dev)
+    a, ia = chebyshev_evolve_batch(X, h, 0.05, 1e-7)
+    b, ib = chebyshev_evolve_batch(X, h, 0.05, 1e-7, matrix_free=False)
+    assert ia["matrix_free"] == matrix_free and not ib["matrix_free"]
+    assert np.array_equal(a.cpu().numpy(), b.cpu().numpy())
