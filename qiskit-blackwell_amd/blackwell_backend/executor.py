@@ -251,8 +251,8 @@ class CompiledCircuit:
         circuit on `device`, measured once: each runs once to warm up and
         TUNE_REPS times timed with HIP events on the launch stream, from
         |0...0>.  Above 13 qubits the candidates include LDS tile programs of
-        several tile shapes ("tiles/<tile qubits>/<low qubits>").  Block passes
-        are not among them: "auto" picks those by rule."""
+        several tile shapes ("tiles/<tile qubits>/<low qubits>").  Mode "tune"
+        times the block passes against it (fastest_mode)."""
         key = str(device)
         if key in self._tuned:
             return self._tuned[key]
@@ -266,6 +266,17 @@ class CompiledCircuit:
         best = self._time_modes(cands, device)
         self._tuned[key] = best
         return best
+
+    def fastest_mode(self, device):
+        """Mode "tune": the faster of tuned_mode's choice and, from 10 qubits on,
+        the block passes, by the same timing rule."""
+        key = ("fastest", str(device))
+        if key not in self._tuned:
+            best = self.tuned_mode(device)
+            if self.n_qubits >= C.PASS_MIN_QUBITS:
+                best = self._time_modes([best, "passes"], device)
+            self._tuned[key] = best
+        return self._tuned[key]
 
     def tuned_block_width(self, device):
         """(mode, {width: ms}): the fusion width of the MFMA block plan
@@ -338,11 +349,11 @@ class CompiledCircuit:
 
     def resolve_mode(self, mode, device=None):
         """auto: the plan _auto_mode expects to be the fastest.
-        tune: the mode tuned_mode measured fastest on `device`."""
+        tune: the mode fastest_mode measured on `device`."""
         if mode == "tune":
             if device is None:
                 raise ValueError("mode 'tune' needs the device to measure on")
-            return self.tuned_mode(device)
+            return self.fastest_mode(device)
         if mode != "auto":
             return mode
         if self._auto is None:

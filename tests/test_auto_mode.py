@@ -128,3 +128,17 @@ def test_served_circuits_take_the_auto_plan(dev):
         server.serve(reqs, realtime=False)
         for r in reqs:
             assert np.linalg.norm(r.state - ref) <= 440 * 4 * 2.0 ** -24, name
+
+
+@pytest.mark.gpu
+def test_tune_times_the_passes_too(dev):
+    """An SU(4) volume circuit runs in passes in less than half the time of every
+    other mode; five-qubit ops on one set of qubits are one block."""
+    from blackwell_backend import BlackwellSimulator, workloads as W
+    sim = BlackwellSimulator(dev, mode="tune")
+    for qc, want in ((W.su4_volume(18, 12, 3), "passes"), (_circuits(18)["same"][0], "blocks")):
+        cc = sim.compile(qc)
+        got, _ = sim.run_statevector(qc)
+        mode = cc.resolve_mode("tune", sim.device)
+        assert mode.startswith(want)
+        assert np.linalg.norm(got - _sim_ops(18, cc.ops)) <= len(cc.ops) * 4 * 2.0 ** -24
