@@ -518,7 +518,10 @@ def plan_tiles(ops, n, m=13, low=4):
             continue
         mask = base
         chosen, keep, blocked = [], [], set()
-        for op in remaining:
+        for i, op in enumerate(remaining):
+            if len(blocked) == n:                # the rest waits for the ops left out
+                keep += remaining[i:]
+                break
             qs = set(op.all_qubits)
             if not fits_tile(op) or (qs & blocked):
                 blocked |= qs
