@@ -25,6 +25,7 @@ Stage 3, planning:
                   fit a 2^m-amplitude tile, one HBM round trip per pass.
 """
 import cmath
+import itertools
 import math
 
 import numpy as np
@@ -390,20 +391,24 @@ def _plan_segment(ops, n, k, effort=1):
     return res
 
 
-def count_blocks(ops, n, k=5):
-    """About how many k-qubit blocks plan_blocks makes of the unitary ops of at
-    most k qubits (qsim_count_blocks), without building matrices: the counts
-    of 100 to 600 ops take 0.1 to 0.4 ms, a plan 1 to 40."""
+def count_blocks(ops, n, k=5, qubits=None):
+    """About how many k-qubit blocks plan_blocks makes of the ops of at most k
+    qubits (k < n; qsim_count_blocks), without building matrices: counting 100 to
+    600 ops takes 0.1 to 0.2 ms, planning them 1 to 40.  qubits: every op's
+    all_qubits, where the caller has them."""
     import ctypes
     from blackwell_kernels import _lib
-    total, out = 0, ctypes.c_int(0)
-    for seg in _segments(ops):
-        if isinstance(seg, Op):
-            continue
-        masks = np.array([_mask(op.all_qubits) for op in seg], dtype=np.uint64)
-        _lib.call("qsim_count_blocks", n, k, len(seg), ctypes.c_void_p(masks.ctypes.data), ctypes.byref(out))
-        total += out.value
-    return total
+    if not ops:
+        return 0
+    everything = tuple(range(n))             # what splits a plan keeps all that follows behind it
+    sets = [everything if len(q) > MAX_PLAN_QUBITS or op.kind in ("measure", "reset") else q
+            for op, q in zip(ops, qubits or [op.all_qubits for op in ops])]
+    lens = np.fromiter(map(len, sets), np.int64, len(sets))
+    bits = np.uint64(1) << np.fromiter(itertools.chain.from_iterable(sets), np.uint64, int(lens.sum()))
+    masks = np.bitwise_or.reduceat(bits, np.cumsum(lens) - lens)
+    out = ctypes.c_int(0)
+    _lib.call("qsim_count_blocks", n, k, len(masks), ctypes.c_void_p(masks.ctypes.data), ctypes.byref(out))
+    return out.value
 
 
 PASS_MIN_QUBITS = 10     # smallest state (and tile) of the block passes

@@ -379,10 +379,15 @@ class CompiledCircuit:
         n = self.n_qubits
         if n < C.PASS_MIN_QUBITS:
             return "whole"
-        wide = any(len(o.all_qubits) > C.PASS_BLOCK_QUBITS for o in self.ops)
+        qubits = [o.all_qubits for o in self.ops]
+        wide = max(map(len, qubits), default=0) > C.PASS_BLOCK_QUBITS
         if n <= WHOLE_TILE_MAX and not wide and len(self.ops) * WHOLE_OP_US(n) < PASS_US:
             return "whole"
-        us = {"passes": self._passes_us(), "blocks": self._launches_us(self.ops)}
+        us = {"passes": self._passes_us()}
+        # each touched qubit is in a block: a plan of fewer launches needs no count
+        least = -(-len(set().union(*qubits)) // 5) * _at_size(TRIP_US, n)[2]
+        if wide or least < us["passes"]:
+            us["blocks"] = self._launches_us(self.ops, qubits)
         if wide and n <= AUTO_TILES_MAX_QUBITS and all(C.fits_tile(o) for o in self.ops if o.kind not in
                                                        ("measure", "reset")):
             dense = [len(o.qubits) for o in self.ops if o.kind == "mk"]
@@ -396,16 +401,18 @@ class CompiledCircuit:
                                + (len(self.ops) - len(dense)) * _at_size(TILE_OP_US, n) + us_dense)
         return min(us, key=us.get)
 
-    def _launches_us(self, ops):
-        """About how long `ops` take as 5-qubit blocks and single wider ops."""
-        wide = sum(len(o.all_qubits) > 5 for o in ops)
-        return C.count_blocks(ops, self.n_qubits) * _at_size(TRIP_US, self.n_qubits)[2] + wide * WIDE_OP_US
+    def _launches_us(self, ops, qubits):
+        """About how long `ops`, on the qubit tuples `qubits`, take as 5-qubit blocks
+        and single wider ops."""
+        wide = sum(len(q) > 5 for q in qubits)
+        return (C.count_blocks(ops, self.n_qubits, 5, qubits) * _at_size(TRIP_US, self.n_qubits)[2]
+                + wide * WIDE_OP_US)
 
     def _passes_us(self):
         """About how long plan_passes' plan takes."""
         t_pass, t_block, _ = _at_size(TRIP_US, self.n_qubits)
         return sum(len(e.passes) * t_pass + len(e.blocks) * t_block if isinstance(e, C.PassRun)
-                   else self._launches_us(e) for e in _pass_groups(self.pass_entries()))
+                   else self._launches_us(e, [o.all_qubits for o in e]) for e in _pass_groups(self.pass_entries()))
 
     def _build(self, mode, device):
         n = self.n_qubits
