@@ -210,7 +210,9 @@ int qsim_count_blocks(int n_qubits, int k, int n_ops, const uint64_t* op_masks, 
  * bits, then the rest; index j sits at j with bits 5..9 and 10..12 XORed onto
  * bits 0..4), and QSIM_PASS_BLOCK_BF16 bf16 values hold its matrix, each
  * coefficient as the sum of three bf16 parts, in MFMA fragment order.
- * qsim_plan_passes writes all three.                                      */
+ * qsim_plan_passes writes all three.  Amplitudes are split the same way,
+ * exactly where their parts are between 2^-100 and 2^127; smaller ones lose
+ * bits below 2^-126, and FP32 values that round to infinity in bf16 are lost. */
 #define QSIM_PASS_MIN_TILE 10
 #define QSIM_PASS_MAX_TILE 13
 #define QSIM_PASS_BLOCK_BF16 3072
@@ -549,8 +551,9 @@ int qsim_cheb_pauli_step(void* stream, int n_qubits, int n_groups, const void* x
  * coef, and by kind
  *   CONST  same = the entry, the same in every row;
  *   PAIR   one or two terms: masks m0, m1 and coefficients c0, c1 (a missing
- *          second term has mask and coefficient 0), same = c0 + c1 and
- *          diff = c0 - c1 rounded to FP32;
+ *          second term has mask and coefficient 0; the kernels read only
+ *          their sum and difference), same = c0 + c1 and diff = c0 - c1
+ *          rounded to FP32;
  *   TERMS  any number of terms, read from sm and coef (real parts).        */
 #define QSIM_PAULI_GROUP_CONST 0
 #define QSIM_PAULI_GROUP_PAIR  1

@@ -803,13 +803,13 @@ __device__ __forceinline__ double pair_entry(const PauliGroup& d, uint32_t p0, u
 // FMAs: every kind of group yields one value per row, and one sequence of FMAs
 // adds it (FMAs in each branch made the compiler copy the FP64 sums at every
 // merge: 48 VALU instructions per group against 36).
-// What bounds it: the T_k loads that miss L2 (3.2 GB per 20-qubit term of 32
-// vectors with the accumulator in every term, about 5.5 TB/s), then the entry
-// evaluation.  Times per term of a Heisenberg chain against the CSR term, us:
-// 20 qubits with 2 / 4 / 8 / 32 vectors 273 / 278 / 385 / 838 -> 72 / 88 / 153
-// / 617, 22 qubits with 32 3660 -> 2672, all with one accumulation per term;
-// with one per two terms 32 states of 20 qubits evolve in 35.8 ms instead of
-// 43.4 (58.7 on the CSR).  Two and eight vectors and tiles of 512 and 1024 rows measured the same to 15 % slower.
+// What bounds it: the T_k loads that miss L2, then the entry evaluation (VALU busy
+// 49 %).  A term of 32 vectors of 20 qubits fetches 2.7 GB past L2 and writes
+// 0.5, 5.8 TB/s; of 22 qubits 14.8 and 2.1, 7.0 TB/s.  Times per term of a
+// Heisenberg chain against the CSR term, us: 20 qubits with 2 / 4 / 8 / 32
+// vectors 273 / 278 / 385 / 838 -> 72 / 88 / 153 / 617, 22 qubits with 32 3660
+// -> 2672, all with one accumulation per term; with one per two terms 565 and
+// 2440 for 32.  Two and eight vectors and tiles of 512 and 1024 rows measured the same to 15 % slower.
 constexpr int kPauliVecs = 4;
 template <typename R, bool NT>
 __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const PauliGroup* __restrict__ tab,
@@ -923,7 +923,10 @@ __global__ __launch_bounds__(kThreads) void k_cheb_pauli(int n_groups, const Pau
 // far loads, most of which another XCD wrote.  us per term of a Heisenberg
 // chain of 12 / 16 / 19 qubits: 6.8 / 8.1 / 17.5 (k_cheb_pauli1 9.5 / 14 / 25;
 // the walk with scalar table loads, as in k_cheb_pauli, 13 / 16 / 29).  A
-// 19-qubit evolution 1820 -> 1300 us with the launches in one call.
+// 19-qubit evolution 1790 -> 1270 us with the launches in one call.  Groups of
+// three terms and more cost a term and row more than in k_cheb_pauli1: past 2 to
+// 3.5 of them a group that kernel is the faster from 18 qubits on (the callers'
+// rule).
 __device__ __forceinline__ uint32_t from_lane(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
 }

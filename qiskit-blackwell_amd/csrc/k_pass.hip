@@ -14,21 +14,23 @@
 // as B operand and as D result (register 4 q + 2 e + part), so a set is read
 // and written as whole amplitudes at the same eight LDS addresses.
 //
-// Arithmetic: FP32 amplitudes as exact sums of three bf16 (hi + mid + lo, each
-// rounded to nearest, 3 x 8 bits), coefficients as three bf16 within 2^-26 of
-// their FP64 value (closer than FP32), multiplied on v_mfma_f32_32x32x16_bf16
-// with FP32 accumulation.  Products of two bf16 are exact.  The hi*hi sums have
-// an accumulator of their own, where they are all but exact; the five smaller
-// products (lo with hi, mid with mid, mid with hi; the three left out are below
-// 2^-26 of a term) are summed from the smallest up in a second one, and one
-// FP32 addition joins the two.  Error of the norm against FP64: 1.9e-7 after
-// 24 random blocks on 13 qubits, 5.0e-7 on the FP32 matrix instructions; SU(4)
-// volume 28 qubits 5.4e-7 against 1.2e-6.  Accumulating everything in one chain
-// doubles the error of structured blocks (27-qubit QFT 5.7e-7 against 3.5e-7).
-// A permutation block moves its amplitudes bit for bit (hi + (mid + lo) has no
-// rounding).  The FP32 instructions run at 1/16 of the bf16 rate and, measured
-// here, not beside VALU work: 277 us per block at 28 qubits (218 at their peak)
-// against 190 us.
+// Arithmetic: FP32 amplitudes as sums of three bf16 (hi + mid + lo, each
+// rounded to nearest, 3 x 8 bits), exact for magnitudes from 2^-100 to 2^127:
+// below, the last bits of lo fall under the smallest bf16, and the top 2^-8 of
+// FP32's range rounds hi up to infinity.  Coefficients are three bf16 within
+// 2^-26 of their FP64 value (closer than FP32), multiplied on
+// v_mfma_f32_32x32x16_bf16 with FP32 accumulation.  Products of two bf16 are
+// exact.  The hi*hi sums have an accumulator of their own, where they are all
+// but exact; the five smaller products (lo with hi, mid with mid, mid with hi;
+// the three left out are below 2^-26 of a term) are summed from the smallest up
+// in a second one, and one FP32 addition joins the two.  Error of the norm
+// against FP64: 1.9e-7 after 24 random blocks on 13 qubits, 5.0e-7 on the FP32
+// matrix instructions; SU(4) volume 28 qubits 5.4e-7 against 1.2e-6.
+// Accumulating everything in one chain doubles the error of structured blocks
+// (27-qubit QFT 5.7e-7 against 3.5e-7).  A permutation block moves amplitudes of
+// that range bit for bit (hi + (mid + lo) has no rounding).  The FP32
+// instructions run at 1/16 of the bf16 rate and, measured here, not beside VALU
+// work: 277 us per block at 28 qubits (218 at their peak) against 190 us.
 //
 // LDS addresses are linear over GF(2): amplitude j of the tile sits at
 // sw(j) = j with bits 5..9 and 10..13 folded onto bits 0..4.  The planner
@@ -37,12 +39,16 @@
 // banks whatever the block's qubits are.  The block record holds the swizzled
 // index of each single bit, so an address is an XOR of record entries.
 //
-// What bounds it: the vector pipe.  At 28 qubits a set takes 148 VALU
-// instructions (88 of them split its amplitudes, 16 join the accumulators) at 4
-// cycles and 12 products at 32, and the counters show these adding up to all
-// SIMD cycles, at 1.76 GHz: a wave's products do not run beside another's VALU
-// work here, and the tile's bytes (0.68 ms a pass alone) hide behind the two.
-// So only fewer instructions help: LDS addresses without the array's base,
+// What bounds it: issue, of vector instructions before products, with waits that
+// the waves at hand do not all cover.  At 28 qubits and 3.5 blocks a pass the
+// counters give a set 144 vector instructions, 12 of them products; 88 split its
+// amplitudes, 16 join the accumulators.  Of all SIMD cycles 34 % run a product
+// and 47 % a vector instruction (at 4 cycles each), half of the products'
+// cycles beside a vector instruction, so 36 % issue neither; a wave spends 29 %
+// of its time at a wait or barrier and 47 % ready but not picked.  The tile's
+// bytes cross memory once each way (2.15 GB) and hide in part: 1.08 ms a pass
+// with 3.5 blocks, 0.68 for the bytes alone.
+// Fewer vector instructions did help: LDS addresses without the array's base,
 // slots stored as two amplitudes instead of four selects, scalar bases in
 // global addresses (163 -> 148 a set) took the depth-24 SU(4) circuit at 24
 // qubits from 1752 to 1707 us, depth 28 at 28 qubits from 40.3 to 39.7 ms.
@@ -83,7 +89,7 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
   const f32x2v v = {a, b};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
-// x = hi + mid + lo exactly, each a pair of bf16 rounded to nearest.
+// x = hi + mid + lo (exactly in the range above), each a pair of bf16 rounded to nearest.
 __device__ __forceinline__ void split3(float2 x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   hi = pk_bf16(x.x, x.y);
   const float rx = x.x - __uint_as_float(hi << 16), ry = x.y - __uint_as_float(hi & 0xffff0000u);

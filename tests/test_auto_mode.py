@@ -11,7 +11,7 @@ from test_compiler import _sim_ops
 
 
 def _circuits(n):
-    """name -> (circuit, plans that measured within 25 % of the fastest at 24 qubits)."""
+    """name -> (circuit, the plan that measured fastest on its family from 22 qubits on)."""
     from blackwell_backend import workloads as W
     from blackwell_backend.circuit import QuantumCircuit
     rng = np.random.default_rng(n)
