@@ -326,10 +326,12 @@ class CompiledCircuit:
         return self._blocks[k]
 
     def pass_entries(self):
-        """plan_passes of the ops at the shape for their size (computed once)."""
-        if self._passes is None:
-            self._passes = C.plan_passes(self.ops, self.n_qubits, *pass_shape(self.n_qubits))
-        return self._passes
+        """plan_passes of the ops at the shape for their size, kept from the choice
+        of a mode to the building of its plan."""
+        entries = self._passes
+        if entries is None:
+            entries = self._passes = C.plan_passes(self.ops, self.n_qubits, *pass_shape(self.n_qubits))
+        return entries
 
     # ---------------------------------------------------------------- plans
     def plan(self, mode, device):
@@ -374,8 +376,8 @@ class CompiledCircuit:
         SU(4) on the same five qubits 2.1 against 0.76; with H, X and CX layers
         between the X 76.8 against 105.9.  So both are counted at TRIP_US, and LDS
         programs too where ops of five qubits and more are: they hold controlled
-        ones of any width (16 qubits, ten layers of ry and four six-control X 312
-        us against 448)."""
+        ones of any width (16 qubits, the ten layers 531 us in passes, 342 in
+        blocks, 246 in tiles)."""
         n = self.n_qubits
         if n < C.PASS_MIN_QUBITS:
             return "whole"
@@ -399,7 +401,10 @@ class CompiledCircuit:
                 passes = sum(isinstance(e, C.TilePass) for e in tiles)
                 us["tiles"] = (passes * _at_size(TILE_PASS_US, n) + (len(tiles) - passes) * WIDE_OP_US
                                + (len(self.ops) - len(dense)) * _at_size(TILE_OP_US, n) + us_dense)
-        return min(us, key=us.get)
+        best = min(us, key=us.get)
+        if best != "passes":
+            self._passes = None              # 6 KiB a block
+        return best
 
     def _launches_us(self, ops, qubits):
         """About how long `ops`, on the qubit tuples `qubits`, take as 5-qubit blocks
@@ -436,7 +441,8 @@ class CompiledCircuit:
         if mode == "passes":
             if n < C.PASS_MIN_QUBITS:
                 raise ValueError(f"block passes need n >= {C.PASS_MIN_QUBITS} (n = {n})")
-            return self._build_passes(self.pass_entries(), device)
+            entries, self._passes = self.pass_entries(), None     # the plan has them on the device
+            return self._build_passes(entries, device)
         if mode == "blocks":
             if n < 10:
                 return self._build_tiles(C.plan_tiles(self.ops, n, m=n), device)
