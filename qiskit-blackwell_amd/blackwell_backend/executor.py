@@ -12,7 +12,7 @@ Modes:
   blocks - 5-qubit dense blocks on FP32 MFMA (n >= 10), other entries plain;
   blocks/<k> - the same with k-qubit blocks, k = 4, 5, 6 (k = 4 needs
            n >= 11 and k = 6 n >= 13 for their MFMA kernels);
-  passes - 4-qubit dense blocks, FP32 values as exact bf16 triples on the
+  passes - 4-qubit dense blocks, FP32 values as bf16 triples on the
            bf16 MFMA, many per trip through HBM (n >= 10): tiles of 10..13
            qubits stay in LDS for all the blocks of a pass;
   tiles  - LDS tile programs, many ops per HBM pass;
